@@ -74,34 +74,36 @@ __global__ __launch_bounds__(256) void k_split(const float *src, int ld_src, uin
 // columns of C may come from two weight matrices (B0 for n < N0, B1 for the N1 after it),
 // so the q and kv_a projections of the same tokens run as one launch.
 //
-// Block tile 256 x BN (BN = 256 or 128), eight math waves (2 per SIMD) in a WM x WN grid, each
-// owning a (256 / WM) x (BN / WN) quadrant of v_mfma_f32_16x16x32 tiles. Large tiles keep
-// the L2 traffic at 24-32 bytes per clock per CU at the MFMA rate. The lo operand, when it
-// is given and needed, is a second pass over k: the k loop runs over [Ah | Al] against
-// [B | B], so each stage is one A and one B tile with a k step of 64, and all stages have
-// the same shape. They stream into an LDS ring of 3 stages (2 where 3 do not fit) by
-// global_load_lds_dwordx4 DMA, issued by four more waves that do nothing else: a DMA
-// instruction holds its wave until the memory system accepts it (about a quarter of a math
-// wave's time when the math waves issued their own), so the math waves only compute and meet
-// the DMA waves at one barrier per stage (the DMA waves wait for stage kt's data before it).
-// 128-byte rows with slot s at s ^ (r & 7) spread the 8 rows one ds_read_b128 phase touches
-// over distinct banks. Each wave reads all its fragments of a 32-deep k-sub before its MFMAs.
-// The lo pass runs when Al is given and either no flag is given or *lo_flag != 0 (the flag
-// is raised by the producer of Al when some lo word is non-zero). Requires K % 64 == 0, lda
+// Block tile BM x BN, MW math waves in a WM x WN grid, each owning (BM / WM) x 64 columns of
+// v_mfma_f32_16x16x32 tiles. With LO a stage of the LDS ring holds a k step of Ah, of Al and of
+// B, so each B tile is taken in once for both parts (two passes over k took in 4/3 of the
+// bytes); the Al part is neither fetched nor multiplied when *lo_flag says that it is zero.
+// The stages stream in by global_load_lds_dwordx4 DMA, issued by four more waves that do nothing
+// else: a DMA instruction holds its wave until the memory system accepts it (about a quarter of
+// a math wave's time when the math waves issued their own), so the math waves only compute and
+// meet the DMA waves at one barrier per stage (the DMA waves wait for stage kt's data before it).
+// The 16-byte slots of a row are XOR-swizzled so that the 8 rows one ds_read_b128 phase touches
+// fall into distinct banks. Each wave reads all its fragments of a 32-deep k-sub before its
+// MFMAs. The lo part runs when Al is given and either no flag is given or *lo_flag != 0 (the
+// flag is raised by the producer of Al when some lo word is non-zero). Requires K % 64 == 0, lda
 // and ldb multiples of 8.
-constexpr int kGBm = 256;
-constexpr int kGemmMath = 8, kGemmDma = 4;  // waves of a GEMM block
+constexpr int kGemmDma = 4;  // DMA waves of a GEMM block
 
-template <int BN>
-struct GemmShape {
-    static constexpr int BK = 64, RowB = BK * 2, Spr = BK / 8;  // 16-byte slots per row
-    static constexpr int WM = BN == 256 ? 2 : 4, WN = 8 / WM;
-    static constexpr int TM = kGBm / WM / 16, TN = BN / WN / 16;  // 16x16 tiles per wave
-    static constexpr int ATile = kGBm * RowB, BTile = BN * RowB;
-    static constexpr int Stage = ATile + BTile;
-    static constexpr int Stages = (160 * 1024) / Stage >= 3 ? 3 : 2;  // ring depth that fits
+template <int BM_, int BN_, int BK_, int MW_, int BPC_, bool LO_>
+struct GemmCfg {
+    static constexpr int BM = BM_, BN = BN_, BK = BK_, MW = MW_, BPC = BPC_;  // BPC: blocks per CU
+    static constexpr bool LO = LO_;
+    static constexpr int RowB = BK * 2, Spr = BK / 8;  // 16-byte slots per row
+    static constexpr int WN = BN / 64, WM = MW / WN, TM = BM / WM / 16, TN = 4;
+    static constexpr int ATile = BM * RowB, BTile = BN * RowB;
+    static constexpr int Stage = (LO ? 2 : 1) * ATile + BTile;
+    static constexpr int Fit = (160 * 1024 / BPC) / Stage;
+    static constexpr int Stages = Fit > 8 ? 8 : Fit;  // ring depth that fits
     static constexpr int Smem = Stages * Stage;
-    __device__ static int swz(int row) { return row & 7; }
+    static constexpr int Threads = 64 * (MW + kGemmDma);
+    static_assert(Stages >= 2 && TM >= 1 && WM * WN == MW && WM * TM * 16 == BM, "tile shape");
+    static_assert(Smem >= MW * 16 * 68 * 4, "the epilogue's staging fits the ring");
+    __device__ static int swz(int row) { return BK == 64 ? row & 7 : (row >> 1) & 3; }
 };
 
 struct GemmArgs {
@@ -152,10 +154,9 @@ __device__ __forceinline__ void wait_stages(int later) {
     }
 }
 
-template <int BN, int EPI, bool F16>
-__global__ __launch_bounds__(64 * (kGemmMath + kGemmDma)) void k_gemm16(GemmArgs a, GemmEpi e) {
-    using Sh = GemmShape<BN>;
-    constexpr int BK = Sh::BK, RowB = Sh::RowB, Spr = Sh::Spr;
+template <class Sh, int EPI, bool F16>
+__global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) void k_gemm16(GemmArgs a, GemmEpi e) {
+    constexpr int BM = Sh::BM, BN = Sh::BN, BK = Sh::BK, RowB = Sh::RowB, Spr = Sh::Spr;
     constexpr int TM = Sh::TM, TN = Sh::TN;
     __shared__ __attribute__((aligned(16))) uint8_t smem[Sh::Smem];
     const uint32_t sbase = lds_addr(smem);
@@ -164,28 +165,29 @@ __global__ __launch_bounds__(64 * (kGemmMath + kGemmDma)) void k_gemm16(GemmArgs
     const int wm = w / Sh::WN, wn = w % Sh::WN;
     const int M = a.M, N0 = a.N0, N1 = a.N1, K = a.K, lda = a.lda, ldb = a.ldb;
     const int tn0 = (N0 + BN - 1) / BN, tn = tn0 + (N1 + BN - 1) / BN;
-    const int tm = (M + kGBm - 1) / kGBm, ntiles = tm * tn;
-    // Tiles in row-major order; with ntiles % 8 == 0, XCD b % 8 takes a contiguous eighth
-    // of them (blocks of one XCD share A rows in its L2).
-    int tile = blockIdx.x;
-    if (ntiles % 8 == 0) tile = (blockIdx.x & 7) * (ntiles / 8) + (blockIdx.x >> 3);
+    const int tm = (M + BM - 1) / BM, ntiles = tm * tn;
+    // Tiles in row-major order, XCD b % 8 taking a contiguous eighth of them (blocks of one XCD
+    // share A rows in its L2).
+    const int xcd = blockIdx.x & 7, per = ntiles >> 3, rem = ntiles & 7;
+    const int tile = xcd * per + min(xcd, rem) + (blockIdx.x >> 3);
     const int mt = tile / tn, nt = tile % tn;
     const bool seg1 = nt >= tn0;
     const uint16_t *B = seg1 ? a.B1 : a.B0;
     const int Nseg = seg1 ? N1 : N0;
     const int nb0 = seg1 ? (nt - tn0) * BN : nt * BN;  // first row of B in this tile
     const int c0 = seg1 ? N0 + nb0 : nb0;              // first column of C
-    const int m0 = mt * kGBm;
-    const bool use_lo = a.Al && (!a.lo_flag || *a.lo_flag);
+    const int m0 = mt * BM;
+    const bool use_lo = Sh::LO && a.Al && (!a.lo_flag || *a.lo_flag);
 
-    const int nk = K / BK, nkt = use_lo ? 2 * nk : nk;  // k steps of the hi pass, of all passes
+    const int nkt = K / BK;
     constexpr int NS = Sh::Stages;
-    if (w >= kGemmMath) {
+    if (w >= Sh::MW) {
         // DMA wave dw: instruction i fills slot (4i + dw) * 64 + l of a tile: row p / Spr,
         // physical slot p % Spr holding logical slot (p % Spr) ^ swz(row). Rows past the end of
         // A or B are clamped to the last row (their results are never stored).
-        const int dw = w - kGemmMath;
+        const int dw = w - Sh::MW;
         constexpr int NA = Sh::ATile / (kGemmDma * 1024), NB = Sh::BTile / (kGemmDma * 1024);
+        static_assert(NA >= 1 && NB >= 1, "whole DMA instructions per tile");
         uint32_t aoff[NA], boff[NB];
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
@@ -200,25 +202,35 @@ __global__ __launch_bounds__(64 * (kGemmMath + kGemmDma)) void k_gemm16(GemmArgs
         const uint8_t *gah = (const uint8_t *)(a.Ah + (size_t)m0 * lda);
         const uint8_t *gal = use_lo ? (const uint8_t *)(a.Al + (size_t)m0 * lda) : gah;
         const uint8_t *gb = (const uint8_t *)(B + (size_t)nb0 * ldb);
-        auto issue = [&](int kt, int stage) __attribute__((always_inline)) {
-            const uint32_t dst = sbase + stage * Sh::Stage + (uint32_t)dw * 1024;
-            const bool lo = kt >= nk;
-            const uint8_t *ga = lo ? gal : gah;
-            const size_t ko = (size_t)(lo ? kt - nk : kt) * BK * 2;
+        auto stream = [&](auto lo_tag) __attribute__((always_inline)) {
+            constexpr bool kLo = decltype(lo_tag)::value;
+            auto issue = [&](int kt, int stage) __attribute__((always_inline)) {
+                const uint32_t dst = sbase + stage * Sh::Stage + (uint32_t)dw * 1024;
+                const size_t ko = (size_t)kt * RowB;
 #pragma unroll
-            for (int i = 0; i < NA; ++i) dma_b128_s(ga + ko, aoff[i], dst + i * (kGemmDma * 1024));
+                for (int i = 0; i < NA; ++i) dma_b128_s(gah + ko, aoff[i], dst + i * (kGemmDma * 1024));
 #pragma unroll
-            for (int i = 0; i < NB; ++i) dma_b128_s(gb + ko, boff[i], dst + Sh::ATile + i * (kGemmDma * 1024));
+                for (int i = 0; i < NB; ++i) dma_b128_s(gb + ko, boff[i], dst + Sh::ATile + i * (kGemmDma * 1024));
+                if constexpr (kLo) {
+#pragma unroll
+                    for (int i = 0; i < NA; ++i)
+                        dma_b128_s(gal + ko, aoff[i], dst + Sh::ATile + Sh::BTile + i * (kGemmDma * 1024));
+                }
+            };
+#pragma unroll
+            for (int q = 0; q < NS - 1; ++q)
+                if (q < nkt) issue(q, q);
+            int fill = NS - 1;
+            for (int kt = 0; kt < nkt; ++kt) {
+                // stage kt has landed when at most min(NS - 2, nkt - 1 - kt) later stages are in flight
+                wait_stages<(kLo ? 2 : 1) * NA + NB, NS - 2>(min(NS - 2, nkt - 1 - kt));
+                lds_barrier();  // stage kt is in LDS; every math wave is done with stage kt - 1
+                if (kt + NS - 1 < nkt) issue(kt + NS - 1, fill);
+                fill = fill + 1 == NS ? 0 : fill + 1;
+            }
         };
-#pragma unroll
-        for (int q = 0; q < NS - 1; ++q)
-            if (q < nkt) issue(q, q);
-        for (int kt = 0; kt < nkt; ++kt) {
-            // stage kt has landed when at most min(NS - 2, nkt - 1 - kt) later stages are in flight
-            wait_stages<NA + NB, NS - 2>(min(NS - 2, nkt - 1 - kt));
-            lds_barrier();  // stage kt is in LDS; every math wave is done with stage kt - 1
-            if (kt + NS - 1 < nkt) issue(kt + NS - 1, (kt + NS - 1) % NS);
-        }
+        if (use_lo) stream(std::integral_constant<bool, Sh::LO>{});
+        else stream(std::false_type{});
         lds_barrier();  // the math waves' epilogue barrier
         return;
     }
@@ -233,24 +245,42 @@ __global__ __launch_bounds__(64 * (kGemmMath + kGemmDma)) void k_gemm16(GemmArgs
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
-    for (int kt = 0; kt < nkt; ++kt) {
-        lds_barrier();  // stage kt has landed (the DMA waves waited for it)
-        const uint8_t *st = smem + (kt % NS) * Sh::Stage;
+    auto compute = [&](auto lo_tag) __attribute__((always_inline)) {
+        constexpr bool kLo = decltype(lo_tag)::value;
+        int slot = 0;
+        for (int kt = 0; kt < nkt; ++kt) {
+            lds_barrier();  // stage kt has landed (the DMA waves waited for it)
+            const uint8_t *st = smem + slot * Sh::Stage;
+            slot = slot + 1 == NS ? 0 : slot + 1;
 #pragma unroll
-        for (int ks = 0; ks < BK / 32; ++ks) {
-            const uint8_t *sa = st + wm * (TM * 16) * RowB + frd[ks];
-            const uint8_t *sb = st + Sh::ATile + wn * (TN * 16) * RowB + frd[ks];
-            v8bf bo[TN], ao[TM];
+            for (int ks = 0; ks < BK / 32; ++ks) {
+                const uint8_t *sa = st + wm * (TM * 16) * RowB + frd[ks];
+                const uint8_t *sb = st + Sh::ATile + wn * (TN * 16) * RowB + frd[ks];
+                v8bf bo[TN], ao[TM], al[kLo ? TM : 1];
 #pragma unroll
-            for (int j = 0; j < TN; ++j) bo[j] = *(const v8bf *)(sb + j * 16 * RowB);
+                for (int j = 0; j < TN; ++j) bo[j] = *(const v8bf *)(sb + j * 16 * RowB);
 #pragma unroll
-            for (int i = 0; i < TM; ++i) ao[i] = *(const v8bf *)(sa + i * 16 * RowB);
+                for (int i = 0; i < TM; ++i) ao[i] = *(const v8bf *)(sa + i * 16 * RowB);
+                if constexpr (kLo) {
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+                    for (int i = 0; i < TM; ++i)
+                        al[i] = *(const v8bf *)(sa + Sh::ATile + Sh::BTile + i * 16 * RowB);
+                }
 #pragma unroll
-                for (int j = 0; j < TN; ++j) acc[i][j] = mfma16<F16>(ao[i], bo[j], acc[i][j]);
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) acc[i][j] = mfma16<F16>(ao[i], bo[j], acc[i][j]);
+                if constexpr (kLo) {
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+#pragma unroll
+                        for (int j = 0; j < TN; ++j) acc[i][j] = mfma16<F16>(al[i], bo[j], acc[i][j]);
+                }
+            }
         }
-    }
+    };
+    if (use_lo) compute(std::integral_constant<bool, Sh::LO>{});
+    else compute(std::false_type{});
     // Epilogue. D layout: lane (g, n) of tile (i, j) holds rows 4g + r, column n. Row-major
     // outputs go through a per-wave LDS buffer (16 rows x 64 columns per tile row i): lane l
     // then takes columns 4 (l % 16) .. + 3 of rows l / 16 + 4 q, q = 0..3, so the 16 lanes of a
@@ -372,23 +402,67 @@ __global__ __launch_bounds__(64 * (kGemmMath + kGemmDma)) void k_gemm16(GemmArgs
     }
 }
 
-// C = A . [B0; B1]^T with N0 + N1 output columns (N1 = 0: a single weight matrix). One block
-// per CU: the 256 x 256 tile is used unless 256 x 128 tiles (half the work each) need fewer
-// than twice as many rounds over the 256 CUs.
+// C = A . [B0; B1]^T with N0 + N1 output columns (N1 = 0: a single weight matrix).
+//
+// The tile shape goes by the number of tiles the call gives: a launch takes as many rounds of its
+// blocks as 256 CUs need, and a round of a shape takes about the same time whatever the number of
+// its blocks, so the shape with the smallest rounds x time per round runs. Below a few hundred
+// tokens a large tile leaves most CUs idle and a block's time is the latency of its k loop, which
+// small tiles hide with deeper rings; above a few thousand the bytes a CU takes in per MFMA decide
+// for the large ones. Measured time per round in us (stand-alone launches, K = 2048 for q | kv_a
+// and o_proj, 512 for kv_b); tokens -> us of the chosen shape, in brackets that of the 256-row
+// tiles with two passes over k that every size took before:
+//   q | kv_a  37: 11.4 (46)  250: 15.5 (50)  1181: 45 (55)  4096: 106 (134)  16000: 405
+//   kv_b      37: 5.6 (17)   250: 6.1 (21)   1181: 19 (24)  4096: 43 (50)    16000: 166 (171)
+//   o_proj    37: 8.2 (24)   250: 8.8 (24)   1181: 19 (27)  4096: 33 (38)    16000: 109 (118)
+template <class Sh, int EPI, bool F16>
+static hipError_t gemm_launch(hipStream_t st, const GemmArgs &a, const GemmEpi &e, int tiles) {
+    hipLaunchKernelGGL((k_gemm16<Sh, EPI, F16>), dim3(tiles), dim3(Sh::Threads), 0, st, a, e);
+    return hipGetLastError();
+}
+
+enum { kTile64x64 = 0, kTile128x64, kTile128x128, kTile192x128, kTile256x128, kTile256x256, kGemmTiles };
+
+static int gemm_pick(int epi, int M, int N0, int N1, int *tiles) {
+    static const int bm[kGemmTiles] = {64, 128, 128, 192, 256, 256}, bn[kGemmTiles] = {64, 64, 128, 128, 128, 256};
+    // [epilogue]: us per round of 256 blocks (64 x 64: two blocks fit a CU, us up to 256 blocks; a
+    // round of 512 takes kTwo us)
+    static const float cost[3][kGemmTiles] = {{11.0f, 13.0f, 19.0f, 24.0f, 31.0f, 52.0f},
+                                              {15.0f, 22.0f, 29.0f, 45.0f, 52.0f, 101.0f},
+                                              {6.0f, 9.2f, 13.5f, 18.5f, 23.0f, 40.0f}};
+    static const float kTwo[3] = {20.0f, 24.0f, 9.8f};
+    int best = 0;
+    float tbest = 0.0f;
+    for (int c = 0; c < kGemmTiles; ++c) {
+        const int n = (M + bm[c] - 1) / bm[c] * ((N0 + bn[c] - 1) / bn[c] + (N1 + bn[c] - 1) / bn[c]);
+        const float t = c == kTile64x64 ? (n <= 256 ? cost[epi][c] : kTwo[epi] * std::max(1.0f, (n + 64) / 512.0f))
+                                        : cost[epi][c] * (float)((n + 255) / 256);
+        if (c == 0 || t < tbest) {
+            best = c;
+            tbest = t;
+            *tiles = n;
+        }
+    }
+    return best;
+}
+
 template <int EPI, bool F16 = false>
 static hipError_t gemm(hipStream_t st, const uint16_t *Ah, const uint16_t *Al, const int *flag,
                        int lda, const uint16_t *B0, int N0, const uint16_t *B1, int N1, int ldb,
                        float *C, int ldc, int M, int K, const GemmEpi &e) {
     GemmArgs a{Ah, Al, B0, B1 ? B1 : B0, C, flag, M, N0, N1, K, lda, ldb, ldc};
-    const int tm = (M + kGBm - 1) / kGBm;
-    const int t256 = tm * ((N0 + 255) / 256 + (N1 + 255) / 256);
-    const int t128 = tm * ((N0 + 127) / 128 + (N1 + 127) / 128);
-    const bool big = 2 * ((t256 + 255) / 256) <= (t128 + 255) / 256;
     if (K % 64) return hipErrorInvalidValue;
-    constexpr int nt = 64 * (kGemmMath + kGemmDma);
-    if (big) hipLaunchKernelGGL((k_gemm16<256, EPI, F16>), dim3(t256), dim3(nt), 0, st, a, e);
-    else hipLaunchKernelGGL((k_gemm16<128, EPI, F16>), dim3(t128), dim3(nt), 0, st, a, e);
-    return hipGetLastError();
+    constexpr bool LO = !F16;  // the fp16 product has no lo operand
+    if (!LO && Al) return hipErrorInvalidValue;
+    int tiles = 0;
+    switch (gemm_pick(EPI, M, N0, N1, &tiles)) {
+    case kTile64x64: return gemm_launch<GemmCfg<64, 64, 64, 4, 2, LO>, EPI, F16>(st, a, e, tiles);
+    case kTile128x64: return gemm_launch<GemmCfg<128, 64, 64, 4, 1, LO>, EPI, F16>(st, a, e, tiles);
+    case kTile128x128: return gemm_launch<GemmCfg<128, 128, 64, 8, 1, LO>, EPI, F16>(st, a, e, tiles);
+    case kTile192x128: return gemm_launch<GemmCfg<192, 128, 64, 8, 1, LO>, EPI, F16>(st, a, e, tiles);
+    case kTile256x128: return gemm_launch<GemmCfg<256, 128, 64, 8, 1, LO>, EPI, F16>(st, a, e, tiles);
+    default: return gemm_launch<GemmCfg<256, 256, LO ? 32 : 64, 8, 1, LO>, EPI, F16>(st, a, e, tiles);
+    }
 }
 
 // ================================================================ epilogues ============
