@@ -116,6 +116,18 @@ __device__ __forceinline__ uint32_t f16_to_bf8(_Float16 x) {
     return ((h >> 8) & 0x80u) | (m > 0x7b7fu ? 0x7bu : (m + 0x80u) >> 8);
 }
 
+// Four fp16 values -> four bf8 bytes with the hardware conversion (round to nearest even, one
+// instruction per pair), saturating as f16_to_bf8.
+typedef short v2s __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t f16x4_to_bf8(v4h x) {
+    const v4h top = {(_Float16)57344.0f, (_Float16)57344.0f, (_Float16)57344.0f, (_Float16)57344.0f};
+    x = __builtin_elementwise_max(__builtin_elementwise_min(x, top), -top);
+    v2s r = {0, 0};
+    r = __builtin_amdgcn_cvt_scalef32_pk_bf8_f16(r, __builtin_shufflevector(x, x, 0, 1), 1.0f, false);
+    r = __builtin_amdgcn_cvt_scalef32_pk_bf8_f16(r, __builtin_shufflevector(x, x, 2, 3), 1.0f, true);
+    return __builtin_bit_cast(uint32_t, r);
+}
+
 // K8 row (384 bytes) of a key: 24 slots of 16 bytes, slot (part, k-block pair p, lane group g)
 // at 12 part + 4 p + g holding the bf8 of dims 32 kb + 8 g + e for kb = 2p, 2p + 1, e = 0 .. 7 in
 // that order: part 0 the fp16 hi parts, part 1 the lo parts x 2^11 (kK8Lo bytes further). A

@@ -680,9 +680,10 @@ __global__ __launch_bounds__(256) void k_kva_pack(KvaPackArgs a) {
 
 // ================================================================ flash attention ======
 
-// Causal attention for one head and 128 queries: 4 waves x 32 queries (two 16-query tiles
-// u = 0, 1), keys in tiles of 64. QD = 192, DV = 128. Operands are fp16 (11 significant bits,
-// ample range for these values): Q and K as hi + lo pairs, V and P rounded once.
+// Causal attention for one head and 128 queries: 8 waves, wave w taking queries 32 (w % 4) .. + 31
+// (two 16-query tiles u = 0, 1) and half w / 4 of every 64-key tile. QD = 192, DV = 128. Operands
+// are fp16 (11 significant bits, ample range for these values): Q and K as hi + lo pairs, V and P
+// rounded once.
 //
 // Scores are computed transposed, S^T = K Q^T (A = K from LDS, B = Q^T from registers), as
 // Kh Qh (v_mfma_f32_16x16x32_f16) plus the correction Kh Ql + Kl Qh as one bf8 product over
@@ -693,21 +694,35 @@ __global__ __launch_bounds__(256) void k_kva_pack(KvaPackArgs a) {
 // |K||Q| even for large logits, where a single rounding of K would be amplified by the logit
 // size (the Kl Ql term is below 2^-22). Lane (g, n) then holds
 // S^T[key 16t + 4g + i][query n], exactly the values it must supply as the B operand of
-// O^T = V^T P^T when the k-slots of a 32-key chunk c are ordered (16-key tile 2c: i = 0..3,
-// tile 2c+1: i = 0..3) per lane group g; V^T is stored with its keys permuted to that order
+// O^T = V^T P^T when the k-slots of a 32-key chunk are ordered (16-key tile 0: i = 0..3,
+// tile 1: i = 0..3) per lane group g; V^T is stored with its keys permuted to that order
 // (kv_b GEMM), so P never leaves the registers. Softmax is online with a lazy reference max
 // per query: it moves only when a tile's max exceeds it by more than 8 (log2 units), so
 // p <= 256 and most tiles skip the rescale.
 //
-// K and V tiles stream through LDS by global_load_lds_dwordx4 DMA into two offset rings:
-// step j computes QK of tile j+1 (K ring) and softmax + PV of tile j (V ring) while K of
-// tile j+2 and V of tile j+1 are in flight. The 16-byte slots of each LDS row are XOR-
-// swizzled by the row so that the fragment reads are free of bank conflicts.
+// The two waves of a SIMD (w and w + 4) take the two key halves with separate running maxima and
+// sums, and work half a step apart: in step j the first computes QK, softmax and PV of tile j, the
+// second softmax and PV of tile j - 1 and then QK of tile j, so one's softmax runs under the
+// other's MFMAs. K tiles stream through a two-slot LDS ring and V tiles through a three-slot one
+// (step j + 1 still reads V of tile j), filled by global_load_lds_dwordx4 DMA one step ahead; the
+// waves of the second half issue theirs at the start of a step and those of the first after their
+// QK, each under the other's MFMAs (the 64 KB take a quarter of a step to issue). The halves are
+// merged through LDS at the end. The 16-byte slots of each LDS row are XOR-swizzled by the row so
+// that the fragment reads are free of bank conflicts.
+//
+// Bound by the serial chain of a wave's step (LDS reads -> MFMAs -> softmax -> MFMAs) rather than
+// by a unit: without the DMA 1577 us at 16000 tokens, MFMA busy for about 930 of them. Measured
+// alone (us, 37 / 1181 / 4096 / 16000 tokens): 11.2 / 46.0 / 161 / 1944 with one wave per SIMD
+// (32 queries, all 64 keys, QK of the next tile interleaved with the softmax by hand), 11.6 / 44.6
+// / 160 / 1992 with two, 11.1 / 41.0 / 148 / 1787 with the cross-lane max taken only when it moves,
+// 10.9 / 37.5 / 144 / 1763 with the DMA of the two halves apart.
 constexpr int kFQ = 128, kFK = 64;
 constexpr int kFKB = kFK * 192 * 2;  // K tile (hi or lo): 64 rows x 384 B
 constexpr int kFVB = 128 * kFK * 2;  // V^T tile: 128 rows x 128 B
-constexpr int kFSmem = 2 * 2 * kFKB + 2 * kFVB;
+constexpr int kFSmem = 2 * 2 * kFKB + 3 * kFVB;
 constexpr float kFLazy = 8.0f;       // log2 headroom of the lazy max
+constexpr float kFNone = -1e30f;     // running max of a key half that has seen no key yet (finite:
+                                     // differences of it and of itself stay numbers)
 
 struct FlashArgs {
     const _Float16 *qh, *kh;                 // Q, K hi: [NH, Sp, 192]
@@ -725,6 +740,12 @@ struct FlashArgs {
 // row-max logits up to ~150 give 3e-4, ~500 give 6e-4, ~1450 give 1.7e-3, ~4400 give 2.3e-3.
 constexpr float kFLogitMax = 512.0f;
 
+// v_max3_f32 as one instruction (fmaxf makes the compiler quiet each operand first).
+__device__ __forceinline__ float max3(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
 // Max / sum over the four lanes n, n + 16, n + 32, n + 48 (one per 16-lane row).
 __device__ __forceinline__ float xrow_max(float v) {
     auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -739,12 +760,12 @@ __device__ __forceinline__ float xrow_sum(float v) {
     return __uint_as_float(q[0]) + __uint_as_float(q[1]);
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_flash_prefill(FlashArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t smem[kFSmem];
     const uint32_t sbase = lds_addr(smem);
     const int tid = threadIdx.x, l = tid & 63, n = l & 15, g = l >> 4;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), half = w >> 2;
     // kernel arguments as locals (the lambdas below must not capture the argument block)
     const int S = a.S, Sp = a.Sp, NH = a.NH, ldo = a.ldo;
     const float sl2 = a.sl2;
@@ -761,8 +782,40 @@ void k_flash_prefill(FlashArgs a) {
         h = (int)blockIdx.x % NH;
     }
     const int nt = 2 * qt + 2;  // key tiles 0 .. nt-1 (the last two straddle the diagonal)
-    const int qw = qt * kFQ + 32 * w;
+    const int qw = qt * kFQ + 32 * (w & 3);
     const size_t hq = (size_t)h * Sp;
+
+    // DMA sources. K tile: wave w fills LDS slots (3w + i) * 64 + l (16 B each) of the
+    // 1536-slot tile; slot (row, s') holds logical slot s = s' ^ (row & 7) (within groups
+    // of 8). V^T tile: slots (2w + i) * 64 + l of 1024; row d, slot s' holds s' ^ (d & 7).
+    const uint8_t *gkh = (const uint8_t *)(a.kh + hq * 192);
+    const uint8_t *gkl = a.k8 + hq * 384;
+    const uint8_t *gv = (const uint8_t *)(a.vt + (size_t)h * 128 * Sp);
+    uint32_t koff[3], voff[2];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int p = (3 * w + i) * 64 + l, row = p / 24, sp = p % 24;
+        koff[i] = row * 384 + 16 * ((sp & ~7) | ((sp & 7) ^ (row & 7)));
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int p = (2 * w + i) * 64 + l, d = p >> 3, sp = p & 7;
+        voff[i] = (uint32_t)d * Sp * 2 + 16 * (sp ^ (d & 7));
+    }
+    // LDS: K ring [2][hi, lo], then V ring [3]; vs: V slot of tile t
+    auto issue = [&](int t, int vs) __attribute__((always_inline)) {
+        const uint32_t kd = sbase + (t & 1) * 2 * kFKB + (uint32_t)(3 * w) * 1024;
+        const uint32_t vd = sbase + 4 * kFKB + vs * kFVB + (uint32_t)(2 * w) * 1024;
+        const size_t so = (size_t)t * kFK * 384;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            dma_b128_s(gkh + so, koff[i], kd + i * 1024);
+            dma_b128_s(gkl + so, koff[i], kd + kFKB + i * 1024);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) dma_b128_s(gv + (size_t)t * 128, voff[i], vd + i * 1024);
+    };
+    issue(0, 0);
 
     // Q^T B operands: query qw + 16u + n, dims 32kb + 8g .. +7: hi as fp16 (main pass), lo as
     // its bf8(lo x 2^11) bytes (the correction operand below, written so by the q GEMM)
@@ -778,64 +831,16 @@ void k_flash_prefill(FlashArgs a) {
             qb[u][kb] = *(const uint2 *)(pl + 32 * kb);
         }
     }
+    // LDS fragment offsets. K (A operand): row 32 half + 16t + n, logical slot 4kb + g.
+    // V^T (A operand): row 16dt + n, logical slot 4 half + g.
+    int krd[6];
+#pragma unroll
+    for (int kb = 0; kb < 6; ++kb)
+        krd[kb] = (32 * half + n) * 384 + 16 * (8 * (kb >> 1) + ((4 * (kb & 1) + g) ^ (n & 7)));
+    const int vrd = n * 128 + 16 * ((4 * half + g) ^ (n & 7));
+    // K8 (A operand of correction MFMA m): the same row, logical slots 8m + g and 8m + 4 + g,
+    // which are the slots of kb = 2m and 2m + 1
 
-    // DMA sources. K tile: wave w fills LDS slots (6w + i) * 64 + l (16 B each) of the
-    // 1536-slot tile; slot (row, s') holds logical slot s = s' ^ (row & 7) (within groups
-    // of 8). V^T tile: slots (4w + i) * 64 + l of 1024; row d, slot s' holds s' ^ (d & 7).
-    const uint8_t *gkh = (const uint8_t *)(a.kh + hq * 192);
-    const uint8_t *gkl = a.k8 + hq * 384;
-    const uint8_t *gv = (const uint8_t *)(a.vt + (size_t)h * 128 * Sp);
-    uint32_t koff[6], voff[4];
-#pragma unroll
-    for (int i = 0; i < 6; ++i) {
-        const int p = (6 * w + i) * 64 + l, row = p / 24, sp = p % 24;
-        koff[i] = row * 384 + 16 * ((sp & ~7) | ((sp & 7) ^ (row & 7)));
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int p = (4 * w + i) * 64 + l, d = p >> 3, sp = p & 7;
-        voff[i] = (uint32_t)d * Sp * 2 + 16 * (sp ^ (d & 7));
-    }
-    // LDS: K ring [2][hi, lo], then V ring [2]
-    auto issue_k = [&](int t) __attribute__((always_inline)) {
-        const uint32_t dst = sbase + (t & 1) * 2 * kFKB + (uint32_t)(6 * w) * 1024;
-        const size_t so = (size_t)t * kFK * 384;
-#pragma unroll
-        for (int i = 0; i < 6; ++i) {
-            dma_b128(gkh + so + koff[i], dst + i * 1024);
-            dma_b128(gkl + so + koff[i], dst + kFKB + i * 1024);
-        }
-    };
-    auto issue_v = [&](int t) __attribute__((always_inline)) {
-        const uint32_t dst = sbase + 4 * kFKB + (t & 1) * kFVB + (uint32_t)(4 * w) * 1024;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) dma_b128(gv + (size_t)t * 128 + voff[i], dst + i * 1024);
-    };
-    // LDS fragment offsets. K (A operand): row 16t + n, logical slot 4kb + g.
-    // V^T (A operand): row 16dt + n, logical slot 4c + g.
-    int krd[6], vrd[2];
-#pragma unroll
-    for (int kb = 0; kb < 6; ++kb) krd[kb] = n * 384 + 16 * (8 * (kb >> 1) + ((4 * (kb & 1) + g) ^ (n & 7)));
-#pragma unroll
-    for (int c = 0; c < 2; ++c) vrd[c] = n * 128 + 16 * ((4 * c + g) ^ (n & 7));
-    // K8 (A operand of correction MFMA m): row 16t + n, logical slots 8m + g and 8m + 4 + g
-    int f8rd[3][2];
-#pragma unroll
-    for (int m = 0; m < 3; ++m)
-#pragma unroll
-        for (int h2 = 0; h2 < 2; ++h2) {
-            const int ls = 8 * m + 4 * h2 + g;
-            f8rd[m][h2] = n * 384 + 16 * ((ls & ~7) | ((ls & 7) ^ (n & 7)));
-        }
-
-    issue_k(0);
-    issue_k(1);
-    issue_v(0);
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int kb = 0; kb < 6; ++kb) asm volatile("" : "+v"(qa[u][kb]), "+v"(qb[u][kb].x), "+v"(qb[u][kb].y));
-    wait_vmcnt<0>();
     // correction operands: per u, 96 bytes = bf8(Ql 2^11) then bf8(Qh), each in (k-block,
     // element) order, so that byte p meets byte p of the lane group's K8 bytes (hi, then lo);
     // MFMA m takes bytes 32m .. 32m+31
@@ -847,9 +852,9 @@ void k_flash_prefill(FlashArgs a) {
         for (int kb = 0; kb < 6; ++kb)
 #pragma unroll
             for (int hf = 0; hf < 2; ++hf) {
-                uint32_t hi = 0;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) hi |= f16_to_bf8(qa[u][kb][4 * hf + i]) << (8 * i);
+                const v8h &q = qa[u][kb];
+                const uint32_t hi = hf == 0 ? f16x4_to_bf8(__builtin_shufflevector(q, q, 0, 1, 2, 3))
+                                            : f16x4_to_bf8(__builtin_shufflevector(q, q, 4, 5, 6, 7));
                 wd[2 * kb + hf] = hf == 0 ? qb[u][kb].x : qb[u][kb].y;
                 wd[12 + 2 * kb + hf] = hi;
             }
@@ -858,261 +863,176 @@ void k_flash_prefill(FlashArgs a) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) q8[u][m][j] = (int)wd[8 * m + j];
     }
-    // the query operands live in AGPRs (MFMA reads its A/B operands from either file), which
-    // leaves the VGPRs to the score accumulators the softmax reads
+    // a use of every operand here, so that the compiler's wait for their loads stands before the
+    // loop: inside it, it would wait for the tile in flight as well, in every step
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
 #pragma unroll
-        for (int kb = 0; kb < 6; ++kb) asm volatile("" : "+a"(qa[u][kb]));
+        for (int kb = 0; kb < 6; ++kb) asm volatile("" : "+v"(qa[u][kb]));
 #pragma unroll
-        for (int m = 0; m < 3; ++m) asm volatile("" : "+a"(q8[u][m]));
+        for (int m = 0; m < 3; ++m) asm volatile("" : "+v"(q8[u][m]));
     }
-    lds_barrier();
 
-    // Step j: QK of tile j+1 (unless it is the last step) with the softmax of tile j, the DMA
-    // of K(j+2) and V(j+1), and the reads of tile j's V fragments spread over its MFMAs, then PV
-    // of tile j. With one wave per SIMD, VALU, DMA-issue and LDS instructions run under the
-    // MFMAs only when they are interleaved with them in the wave's instruction stream, so the
-    // step is laid out as 18 groups of eight independent QK MFMAs (k-block kb, pass p) separated
-    // by scheduling fences, each carrying its share of the other work, and the scheduler is asked
-    // to alternate MFMAs and VALU within a group. Each QK accumulator receives its products in
-    // the order Kh Qh for kb = 0 .. 5, then the corrections m = 0 .. 2.
-    float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
+    float m_run[2] = {kFNone, kFNone}, l_run[2] = {0.f, 0.f};
     v4f acc[8][2];
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
         for (int u = 0; u < 2; ++u) acc[dt][u] = v4f{0.f, 0.f, 0.f, 0.f};
+    v4f sc[2][2];
 
-    v4f sc[4][2];
-    auto load_kh = [&](const uint8_t *kt, int kb, v8h (&kh)[4]) __attribute__((always_inline)) {
+    // scores of tile j (K slot j & 1): each accumulator receives its products in the order Kh Qh
+    // for kb = 0 .. 5, then the corrections m = 0 .. 2
+    auto qk = [&](int j) __attribute__((always_inline)) {
+        const uint8_t *kt = smem + (j & 1) * 2 * kFKB;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) kh[t] = *(const v8h *)(kt + t * 16 * 384 + krd[kb]);
-    };
-    auto load_k8 = [&](const uint8_t *kt, int m, v8i (&k8)[4]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const v4i x0 = *(const v4i *)(kt + kFKB + t * 16 * 384 + f8rd[m][0]);
-            const v4i x1 = *(const v4i *)(kt + kFKB + t * 16 * 384 + f8rd[m][1]);
-            k8[t] = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
-        }
-    };
-    auto qk_main = [&](v4f (&s)[4][2], const v8h (&kf)[4], int kb) __attribute__((always_inline)) {
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int u = 0; u < 2; ++u) s[t][u] = mfma_f16(kf[t], qa[u][kb], s[t][u]);
-    };
-    auto qk_corr = [&](v4f (&s)[4][2], const v8i (&kf)[4], int m) __attribute__((always_inline)) {
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int u = 0; u < 2; ++u) s[t][u] = mfma_bf8_s11(kf[t], q8[u][m], s[t][u]);
-    };
-    {  // QK of tile 0
-        const uint8_t *kt = smem;
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int u = 0; u < 2; ++u) sc[t][u] = v4f{0.f, 0.f, 0.f, 0.f};
+        auto load_k8 = [&](int m, int t) __attribute__((always_inline)) {
+            const v4i x0 = *(const v4i *)(kt + kFKB + t * 16 * 384 + krd[2 * m]);
+            const v4i x1 = *(const v4i *)(kt + kFKB + t * 16 * 384 + krd[2 * m + 1]);
+            return __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
+        };
 #pragma unroll
         for (int kb = 0; kb < 6; ++kb) {
-            v8h kh[4];
-            load_kh(kt, kb, kh);
-            qk_main(sc, kh, kb);
+            v8h kf[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) kf[t] = *(const v8h *)(kt + t * 16 * 384 + krd[kb]);
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) sc[t][u] = mfma_f16(kf[t], qa[u][kb], sc[t][u]);
         }
 #pragma unroll
         for (int m = 0; m < 3; ++m) {
-            v8i k8[4];
-            load_k8(kt, m, k8);
-            qk_corr(sc, k8, m);
-        }
-    }
-
-    auto step = [&](auto mask_tag, auto next_tag, int j) __attribute__((always_inline)) {
-        constexpr bool kMask = decltype(mask_tag)::value;
-        constexpr bool kNext = decltype(next_tag)::value;
-        wait_vmcnt<0>();
-        lds_barrier();
-        const bool dk = j + 2 < nt, dv = j + 1 < nt;
-        const uint32_t kdst = sbase + (j & 1) * 2 * kFKB + (uint32_t)(6 * w) * 1024;  // K(j+2)
-        const size_t kso = (size_t)(j + 2) * kFK * 384;
-        const uint32_t vdst = sbase + 4 * kFKB + ((j + 1) & 1) * kFVB + (uint32_t)(4 * w) * 1024;  // V(j+1)
-        auto dma_k = [&](int i) __attribute__((always_inline)) {
-            if (dk) {
-                dma_b128_s(gkh + kso, koff[i], kdst + i * 1024);
-                dma_b128_s(gkl + kso, koff[i], kdst + kFKB + i * 1024);
-            }
-        };
-        auto dma_v = [&](int i) __attribute__((always_inline)) {
-            if (dv) dma_b128_s(gv + (size_t)(j + 1) * 128, voff[i], vdst + i * 1024);
-        };
-        // softmax of tile j in pieces (per 16-query tile u: A mask + local max, B row max and
-        // reference max, C(t) weights of key tile t, D denominator)
-        const int k0 = j * kFK;
-        float mloc[2], mnew[2], alpha[2], ps[2];
-        bool moved = false;
-        v8h pb[2][2];
-        auto smA = [&](int u) __attribute__((always_inline)) {
-            const int q = qw + 16 * u + n;
-            float mx = -INFINITY;
+            v8i kf[2];
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
+            for (int t = 0; t < 2; ++t) kf[t] = load_k8(m, t);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float v = sc[t][u][i];
-                    if constexpr (kMask) {
-                        const int key = k0 + 16 * t + 4 * g + i;
-                        if (key > q || key >= S) v = -INFINITY;
-                        sc[t][u][i] = v;
-                    }
-                    mx = fmaxf(mx, v);
-                }
-            mloc[u] = mx;
-        };
-        auto smB = [&](int u) __attribute__((always_inline)) {
-            const float mx = xrow_max(mloc[u]) * sl2;
-            const float mref = m_run[u];
-            const bool mv = mx > mref + kFLazy;
-            mnew[u] = mv ? mx : mref;
-            alpha[u] = __builtin_amdgcn_exp2f(mref - mnew[u]);
-            m_run[u] = mnew[u];
-            moved |= mv;
-            ps[u] = 0.f;
-        };
-        auto smC = [&](int u, int t) __attribute__((always_inline)) {
+            for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float p = __builtin_amdgcn_exp2f(fmaf(sc[t][u][i], sl2, -mnew[u]));
-                ps[u] += p;
-                pb[u][t >> 1][4 * (t & 1) + i] = (_Float16)p;
-            }
-        };
-        auto smD = [&](int u) __attribute__((always_inline)) { l_run[u] = fmaf(l_run[u], alpha[u], ps[u]); };
-        // V fragments of tile j: row 16 dt + n, logical slot 4c + g
-        const uint8_t *vt = smem + 4 * kFKB + (j & 1) * kFVB;
-        v8h vv[2][8];
-        auto load_v = [&](int f) __attribute__((always_inline)) {
-            vv[f >> 3][f & 7] = *(const v8h *)(vt + (f & 7) * 16 * 128 + vrd[f >> 3]);
-        };
-        // the work carried by group gi (gi < 6: main pass kb = gi, eight MFMAs of 16 cycles;
-        // gi = 6 .. 8: correction m = gi - 6, eight MFMAs of 32 cycles)
-        auto extra = [&](int gi) __attribute__((always_inline)) {
-            switch (gi) {
-            case 0: smA(0); dma_k(0); dma_k(1); break;
-            case 1: smB(0); dma_k(2); dma_k(3); break;
-            case 2: smC(0, 0); smC(0, 1); dma_k(4); dma_k(5); break;
-            case 3: smC(0, 2); smC(0, 3); smD(0); dma_v(0); dma_v(1); break;
-            case 4: smA(1); dma_v(2); dma_v(3); break;
-            case 5: smB(1); load_v(0); load_v(1); break;
-            case 6: smC(1, 0); smC(1, 1); load_v(2); load_v(3); load_v(4); load_v(5); break;
-            case 7: smC(1, 2); smC(1, 3); smD(1); load_v(6); load_v(7); load_v(8); load_v(9); break;
-            case 8: load_v(10); load_v(11); load_v(12); load_v(13); load_v(14); load_v(15); break;
-            default: break;
-            }
-        };
-        if constexpr (kNext) {
-            const uint8_t *kt = smem + ((j + 1) & 1) * 2 * kFKB;  // K tile j+1
-            v4f sn[4][2];
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int u = 0; u < 2; ++u) sn[t][u] = v4f{0.f, 0.f, 0.f, 0.f};
-            v8h kh[2][4];
-            v8i k8[2][4];
-            load_kh(kt, 0, kh[0]);
-#pragma unroll
-            for (int kb = 0; kb < 6; ++kb) {
-                const int cb = kb & 1;
-                if (kb + 1 < 6) load_kh(kt, kb + 1, kh[cb ^ 1]);
-                if (kb == 4) load_k8(kt, 0, k8[0]);
-                if (kb == 5) load_k8(kt, 1, k8[1]);
-                __builtin_amdgcn_sched_barrier(0);
-                qk_main(sn, kh[cb], kb);
-                extra(kb);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-                    __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);  // up to three VALU
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-#pragma unroll
-            for (int m = 0; m < 3; ++m) {
-                if (m == 1) load_k8(kt, 2, k8[0]);  // k8[0] is free once correction 0 has issued
-                __builtin_amdgcn_sched_barrier(0);
-                qk_corr(sn, k8[m & 1], m);
-                extra(6 + m);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-                    __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // up to six VALU
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            // the softmax results stay in the groups above (the compiler would otherwise sink
-            // them past the rescale branch, to their uses)
-            asm volatile("" ::"v"(pb[0][0]), "v"(pb[0][1]), "v"(pb[1][0]), "v"(pb[1][1]), "v"(l_run[0]),
-                         "v"(l_run[1]));
-            const bool any = __any(moved);
-            if (any) {
-#pragma unroll
-                for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) acc[dt][u] *= alpha[u];
-            }
-#pragma unroll
-            for (int c = 0; c < 2; ++c)
-#pragma unroll
-                for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) acc[dt][u] = mfma_f16(vv[c][dt], pb[u][c], acc[dt][u]);
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int u = 0; u < 2; ++u) sc[t][u] = sn[t][u];
-        } else {
-#pragma unroll
-            for (int gi = 0; gi < 9; ++gi) extra(gi);
-            if (__any(moved)) {
-#pragma unroll
-                for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) acc[dt][u] *= alpha[u];
-            }
-#pragma unroll
-            for (int c = 0; c < 2; ++c)
-#pragma unroll
-                for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) acc[dt][u] = mfma_f16(vv[c][dt], pb[u][c], acc[dt][u]);
+                for (int u = 0; u < 2; ++u) sc[t][u] = mfma_bf8_s11(kf[t], q8[u][m], sc[t][u]);
         }
     };
-    using F = std::false_type;
-    using T = std::true_type;
-    for (int j = 0; j < nt - 2; ++j) step(F{}, T{}, j);
-    step(T{}, T{}, nt - 2);
-    step(T{}, F{}, nt - 1);
-
-    // range check of each query row: the reference max m_run (log2 units, within kFLazy of the
-    // row's true max) and every output value (NaN or Inf from operands beyond the fp16 range)
-    bool bad = false;
+    // softmax of this wave's half of tile j and its share of O^T += V^T P^T (V slot vs)
+    auto smpv = [&](int j, int vs) __attribute__((always_inline)) {
+        const uint8_t *vt = smem + 4 * kFKB + vs * kFVB + vrd;
+        const int k0 = j * kFK + 32 * half;
+        if (k0 + 31 > qw) {  // the diagonal
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (k0 + 16 * t + 4 * g + i > qw + 16 * u + n) sc[t][u][i] = -INFINITY;
+        }
+        // The running max moves only when a score of the tile exceeds it by more than kFLazy, which
+        // each lane can tell from its own scores; the max over a query's four lanes is taken then.
+        float mx[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+            mx[u] = max3(max3(max3(sc[0][u][0], sc[0][u][1], sc[0][u][2]), sc[0][u][3], sc[1][u][0]),
+                         max3(sc[1][u][1], sc[1][u][2], sc[1][u][3]), sc[1][u][3]) * sl2;
+        if (__any((mx[0] > m_run[0] + kFLazy) | (mx[1] > m_run[1] + kFLazy))) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const float m = xrow_max(mx[u]);
+                const float mnew = m > m_run[u] + kFLazy ? m : m_run[u];
+                const float alpha = __builtin_amdgcn_exp2f(m_run[u] - mnew);
+                m_run[u] = mnew;
+                l_run[u] *= alpha;
+#pragma unroll
+                for (int dt = 0; dt < 8; ++dt) acc[dt][u] *= alpha;
+            }
+        }
+        v8h pb[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            float ps = 0.f;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float p = __builtin_amdgcn_exp2f(fmaf(sc[t][u][i], sl2, -m_run[u]));
+                    ps += p;
+                    pb[u][4 * t + i] = (_Float16)p;
+                }
+            l_run[u] += ps;
+        }
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) {
+            const v8h vv = *(const v8h *)(vt + dt * 16 * 128);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) acc[dt][u] = mfma_f16(vv, pb[u], acc[dt][u]);
+        }
+    };
+    // a tile whose first key of this half comes after this wave's last query adds nothing
+    auto live = [&](int j) __attribute__((always_inline)) { return j * kFK + 32 * half <= qw + 31; };
+
+    int vs = 0;  // V slot of tile j
+    if (half == 0) {
+        for (int j = 0; j < nt; ++j) {
+            wait_vmcnt<0>();
+            lds_barrier();  // tile j is in LDS; every wave is done with K(j - 1) and V(j - 2)
+            const int vn = vs == 2 ? 0 : vs + 1;
+            if (live(j)) qk(j);
+            if (j + 1 < nt) issue(j + 1, vn);
+            if (live(j)) smpv(j, vs);
+            vs = vn;
+        }
+    } else {
+        int vp = 0;
+        for (int j = 0; j < nt; ++j) {
+            wait_vmcnt<0>();
+            lds_barrier();
+            const int vn = vs == 2 ? 0 : vs + 1;
+            if (j + 1 < nt) issue(j + 1, vn);
+            if (j > 0 && live(j - 1)) smpv(j - 1, vp);
+            if (live(j)) qk(j);
+            vp = vs;
+            vs = vn;
+        }
+        if (live(nt - 1)) smpv(nt - 1, vp);
+    }
+
+    // Merge of the two key halves: wave w gives query tile u = 1 - half to wave w ^ 4 and
+    // finishes tile u = half.
+    lds_barrier();  // the ring is free
+    float *xw = (float *)(smem + w * 9216), *xr = (float *)(smem + (w ^ 4) * 9216);
+    auto give = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) *(v4f *)(xw + 256 * dt + 4 * l) = acc[dt][u];
+        xw[2048 + l] = m_run[u];
+        xw[2112 + l] = l_run[u];
+    };
+    // range check of each query row: the reference max (log2 units, within kFLazy of the row's
+    // true max) and every output value (NaN or Inf from operands beyond the fp16 range)
+    bool bad = false;
+    auto finish = [&](int u) __attribute__((always_inline)) {
+        const float m1 = xr[2048 + l], m = fmaxf(m_run[u], m1);
+        const float a0 = __builtin_amdgcn_exp2f(m_run[u] - m), a1 = __builtin_amdgcn_exp2f(m1 - m);
         const int q = qw + 16 * u + n;
-        const float inv = 1.0f / xrow_sum(l_run[u]);
-        if (q >= S) continue;
-        bad |= !(fabsf(m_run[u]) <= kFLogitMax * 1.4426950408889634f);  // m_run = logit * log2(e)
+        const float inv = 1.0f / xrow_sum(l_run[u] * a0 + xr[2112 + l] * a1);
+        if (q >= S) return;
+        bad |= !(fabsf(m) <= kFLogitMax * 1.4426950408889634f);  // m = logit * log2(e)
         _Float16 *o = a.o + (size_t)q * ldo + (size_t)h * 128 + 4 * g;
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) {
-            const v4h ov = {(_Float16)(acc[dt][u][0] * inv), (_Float16)(acc[dt][u][1] * inv),
-                            (_Float16)(acc[dt][u][2] * inv), (_Float16)(acc[dt][u][3] * inv)};
+            const v4f s = acc[dt][u] * a0 + *(const v4f *)(xr + 256 * dt + 4 * l) * a1;
+            const v4h ov = {(_Float16)(s[0] * inv), (_Float16)(s[1] * inv), (_Float16)(s[2] * inv),
+                            (_Float16)(s[3] * inv)};
 #pragma unroll
             for (int i = 0; i < 4; ++i) bad |= !__builtin_isfinite((float)ov[i]);
             *(v4h *)(o + 16 * dt) = ov;
         }
-    }
+    };
+    if (half == 0) give(1);
+    else give(0);
+    lds_barrier();
+    if (half == 0) finish(0);
+    else finish(1);
     // any writer stores the same value; the readers are later kernels
     if (__builtin_amdgcn_ballot_w64(bad) != 0 && l == 0) {
         __hip_atomic_store(a.flag_call, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -1350,7 +1270,7 @@ hipError_t launch_prefill_all(hipStream_t st, const Dims &d, int S, float eps, c
             return e;
         FlashArgs fa{qh, kh, ql8, k8, vt, heads, flags + 1, range ? range->sticky : nullptr, S, Sp, d.NH, d.HO,
                      smscale * 1.4426950408889634f};
-        hipLaunchKernelGGL(k_flash_prefill, dim3(Sp / kFQ * d.NH), dim3(256), 0, st, fa);
+        hipLaunchKernelGGL(k_flash_prefill, dim3(Sp / kFQ * d.NH), dim3(512), 0, st, fa);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         // out = heads . o_proj^T in fp16 (heads rounded once, o_proj converted exactly), the
         // two scales undone (or NaN when the range flag of this call is up)
