@@ -67,6 +67,21 @@ def test_rmsnorm_bit_exact():
             np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32), err_msg=f"n={n} seed={seed}")
 
 
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 2047, 2049, 4096, 4097])
+def test_rmsnorm_sizes_bit_exact(n):
+    """The register form's edges (one value, whole and ragged 256-value rounds, its largest sizes) and
+    the looped form above 4096."""
+    for seed in range(4):
+        x = inputs.normal_f32(seed, "x", (n,)) * np.float32(0.5 + seed)
+        w = inputs.normal_bf16(seed, "w", (n,), mean=1.0, std=0.1)
+        a = np.full(n + 1, 7.0, np.float32)
+        b = np.zeros(n, np.float32)
+        L.kvl_rmsnorm_bf16(f32(a), f32(x), u16(w), n, np.float32(1e-5))
+        ORC.orc_rmsnorm_bf16(f32(b), f32(x), u16(w), n, np.float32(1e-5))
+        np.testing.assert_array_equal(a[:n].view(np.uint32), b.view(np.uint32), err_msg=f"n={n} seed={seed}")
+        assert a[n] == 7.0
+
+
 def pack_gpu(lat, rope, pos, theta):
     n, R = lat.shape
     DR = rope.shape[1]
