@@ -2076,6 +2076,49 @@ __device__ __forceinline__ void fq_wait_all(const FqArgs &f, const unsigned *fla
     __syncthreads();
 }
 
+// The projection's operand normalised in place (FqArgs::xnorm): wave w forms the RMS factor of
+// sequence w over its 2048 columns, adding k_rmsnorm's values in k_rmsnorm's order (the sums of its
+// threads l, l + 64, l + 128, l + 192, their tree, then the lanes), and every lane scales its own
+// columns, so the operand equals that kernel's output bit for bit. Every workgroup reads all of x (64
+// KB, from its XCD's L2) beside its 64 KB of weights. Decode stack (27 layers, 8 x 32K rows): the
+// launch grows by 2 us and the norm's launch goes, 1539 -> 1513 us. inv: 8 floats of LDS.
+__device__ __forceinline__ void fq_norm_x(const FqArgs &f, int B, int kq, v4f (&xa)[2], v4f (&xb)[2], float *inv) {
+    const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, n = l & 15, g = l >> 4;
+    const float *xr = f.x + (size_t)min(w, B - 1) * f.ldx;
+    float v[4][8];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[q][i] = xr[l + 64 * q + 256 * i];
+    v4i wt[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) wt[j] = *(const v4i *)(f.xnorm + kq * 512 + (w + 8 * j) * 32 + g * 8);
+    double ss[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        ss[q] = 0.0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ss[q] += (double)v[q][i] * (double)v[q][i];
+    }
+    double t = (ss[0] + ss[2]) + (ss[1] + ss[3]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) t += __shfl_down(t, o);
+    const float mean_sq = (float)(lane_f64(t, 0) / 2048.0);
+    const float r = 1.0f / sqrtf(mean_sq + f.eps);
+    if (l == 0) inv[w] = r;
+    __syncthreads();
+    const float s = inv[n & 7];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t a = (uint32_t)wt[j][e >> 1], b = (uint32_t)wt[j][2 + (e >> 1)];
+            xa[j][e] = (xa[j][e] * s) * __uint_as_float(e & 1 ? a & 0xffff0000u : a << 16);
+            xb[j][e] = (xb[j][e] * s) * __uint_as_float(e & 1 ? b & 0xffff0000u : b << 16);
+        }
+    __syncthreads();  // inv lies in the products' reduction buffer
+}
+
 // The q_proj | kv_a projection block of k_gemv_ksplit<1, 1> with this workgroup's index (B <= 8
 // sequences, in = 2048, the same XCD-aware block -> (row block, k quarter) map), by the 512
 // threads of a fused attention workgroup: wave w does that kernel's waves w and w + 8 (k-blocks
@@ -2110,6 +2153,7 @@ __device__ __forceinline__ void fq_gemv(const FqArgs &f, int B, uint8_t *lds) {
         xa[j] = *(const v4f *)(xr + kbase);
         xb[j] = *(const v4f *)(xr + kbase + 4);
     }
+    if (f.xnorm) fq_norm_x(f, B, kq, xa, xb, (float *)lds);
     v4f acc[2][4];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {

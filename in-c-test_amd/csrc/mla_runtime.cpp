@@ -953,6 +953,13 @@ int prepare_groups(int fmt, const Dims &d, float theta, S *const *states, int B,
     return 0;
 }
 
+// Norm of the inputs of a decode group: x is n = RMSNorm(d_x, w) instead of d_x. buf: a group's
+// rows [<= kMaxBatch, H], used where the projection does not normalise its operand itself.
+struct InNorm {
+    const uint16_t *w;
+    float *buf;
+};
+
 // One decode step for a group of B <= kMaxBatch sequences whose mirrors are synced.
 // d_x: device input rows [B,H]; d_out: device output rows [B,H]. Rows appended on the device
 // at each pos; staged copies in w.rows. solo: see plan_group.
@@ -960,7 +967,7 @@ int prepare_groups(int fmt, const Dims &d, float theta, S *const *states, int B,
 // nothing is allocated (the RoPE table must already cover the positions).
 int decode_group(int fmt, const Dims &d, float eps, float theta, const DevWeights &dw,
                  const SeqIn *seqs, int B, const float *d_x, float *d_out, bool residual,
-                 DecodeWork &w, bool solo = false, size_t part_cap = 0) {
+                 DecodeWork &w, bool solo = false, size_t part_cap = 0, const InNorm *in_norm = nullptr) {
     Ctx &c = ctx();
     hipStream_t st = c.stream;
     int maxpos = 0;
@@ -1020,6 +1027,10 @@ int decode_group(int fmt, const Dims &d, float eps, float theta, const DevWeight
     const bool fuse = fuse_base && (B >= 2 || (pfuse_ok && comb_mode != 0));
     const bool pfuse = fuse && pfuse_ok;
     const int comb = fuse ? comb_mode : 0;
+    if (in_norm && !pfuse) {  // else the projection tasks normalise x themselves (FqArgs::xnorm)
+        HIP_TRY(launch_rmsnorm(st, in_norm->buf, d_x, in_norm->w, d.H, B, eps));
+        d_x = in_norm->buf;
+    }
     {
         // q_proj | kv_a: k split over kGemvKs blocks where the shape allows (the consumers
         // add the partials), else one pass
@@ -1091,6 +1102,7 @@ int decode_group(int fmt, const Dims &d, float eps, float theta, const DevWeight
             if (pfuse) {
                 fq.gemv = 1;
                 fq.x = d_x;
+                fq.xnorm = in_norm ? in_norm->w : nullptr;
                 fq.wq = dw.q;
                 fq.wkva = dw.kva;
                 fq.ldx = d.H;
@@ -1250,7 +1262,7 @@ int decode_host(float *out, const float *x, const int *positions, int B, const K
 
 template <class S>
 int decode_device(float *d_out, const float *d_x, int B, const KvlMlaConfig *cfg, const KvlMlaBF16 *w,
-                  S *const *states, unsigned flags);
+                  S *const *states, unsigned flags, const InNorm *in_norm = nullptr);
 
 // The attention half of a decoder layer (src/generate.c:34-67, attention_token) for a batch,
 // stream-ordered over device buffers: n1 = RMSNorm(h, input_norm) (src/ops.c:76-83 rounding),
@@ -1274,7 +1286,7 @@ int attention_layer_device(float *d_h, float *d_n2, int B, const KvlMlaConfig *c
     const int H = cfg->hidden_size;
     const uint16_t *din = nullptr, *dpost = nullptr;
     if (dev_weight(input_norm, (size_t)H, &din) != 0 || dev_weight(post_norm, (size_t)H, &dpost) != 0) return -1;
-    const size_t need = (size_t)B * H * sizeof(float);
+    const size_t need = (size_t)std::min(B, kMaxBatch) * H * sizeof(float);
     if (c.layer.bytes < need) {
         if (c.capturing) {
             set_err("layer workspace growth during graph capture");
@@ -1282,9 +1294,8 @@ int attention_layer_device(float *d_h, float *d_n2, int B, const KvlMlaConfig *c
         }
         if (dev_reserve(c.layer, need) != 0) return -1;
     }
-    float *n1 = (float *)c.layer.p;
-    HIP_TRY(launch_rmsnorm(c.stream, n1, d_h, din, H, B, cfg->rms_eps));
-    if (decode_device(d_h, n1, B, cfg, w, states, flags | KVL_MLA_RESIDUAL) != 0) return -1;
+    const InNorm in{din, (float *)c.layer.p};
+    if (decode_device(d_h, d_h, B, cfg, w, states, flags | KVL_MLA_RESIDUAL, &in) != 0) return -1;
     HIP_TRY(launch_rmsnorm(c.stream, d_n2, d_h, dpost, H, B, cfg->rms_eps));
     return 0;
 }
@@ -1349,7 +1360,7 @@ int decode_block(float *out, const float *x, int count, int start, const KvlMlaC
 // Stream-ordered decode over device buffers (bound weights, synced mirrors).
 template <class S>
 int decode_device(float *d_out, const float *d_x, int B, const KvlMlaConfig *cfg,
-                  const KvlMlaBF16 *w, S *const *states, unsigned flags) {
+                  const KvlMlaBF16 *w, S *const *states, unsigned flags, const InNorm *in_norm) {
     Dims d;
     if (!d_out || !d_x || B <= 0 || !states || !weights_ok(w) || !dims_of(cfg, d)) {
         set_err("invalid arguments");
@@ -1378,7 +1389,8 @@ int decode_device(float *d_out, const float *d_x, int B, const KvlMlaConfig *cfg
         SeqIn seqs[kMaxBatch];
         for (int i = 0; i < n; ++i) seqs[i] = {ms[g0 + i], states[g0 + i]->len};
         if (decode_group(fmt, d, cfg->rms_eps, cfg->rope_theta, dw, seqs, n, d_x + (size_t)g0 * d.H,
-                         d_out + (size_t)g0 * d.H, (flags & KVL_MLA_RESIDUAL) != 0, wk) != 0)
+                         d_out + (size_t)g0 * d.H, (flags & KVL_MLA_RESIDUAL) != 0, wk, false, 0,
+                         in_norm) != 0)
             return -1;
         if (!(flags & KVL_MLA_NO_ADVANCE)) {
             for (int i = 0; i < n; ++i) {

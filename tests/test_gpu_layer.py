@@ -130,3 +130,48 @@ def test_attention_layer_rejects_bad_arguments():
     L.kvl_mla_device_free(d)
     L.kvl_mla_device_free(e)
     L.kvl_mla_compressed_q8_state_free(C.byref(st))
+
+
+@pytest.mark.parametrize("lens", [[8300], [6000] * 8, [7000, 5100, 9000]], ids=["1", "8", "3"])
+def test_layer_norm_inside_the_projection_equals_its_launch(lens):
+    """Q8 decodes whose projection runs inside the attention launch normalise their input there; with
+    the projection in its own launch the norm is a launch too. Same sums in the same order: h and n2
+    are equal bit for bit, from hidden states of very different scale per sequence."""
+    cfg = inputs.config(**KIMI)
+    H, B = cfg.hidden_size, len(lens)
+    layer = inputs.make_layer(cfg, 0xA7)
+    w = layer.struct()
+    lib.check(L.kvl_mla_bind_weights(C.byref(cfg), C.byref(w)), "bind")
+    rng = np.random.default_rng(0xA7)
+    norms = [inputs.f32_to_bf16_bits(1.0 + 0.1 * rng.standard_normal(H).astype(np.float32)) for _ in range(2)]
+    h0 = np.ascontiguousarray(inputs.hidden(cfg, 0xA8, B) * (10.0 ** (np.arange(B) % 5 - 2))[:, None].astype(np.float32))
+    states = []
+    for i, n in enumerate(lens):
+        st = abi.KvlMlaCompressedQ8State()
+        lib.check(L.kvl_mla_compressed_q8_state_init(C.byref(st), C.byref(cfg), n + 1), "init")
+        lib.check(L.kvl_mla_compressed_q8_state_fill_synthetic(C.byref(st), 0, n, 0xA70 + i), "fill")
+        states.append(st)
+    arr = (C.POINTER(abi.KvlMlaCompressedQ8State) * B)(*[C.pointer(s) for s in states])
+    nb = h0.nbytes
+    d_h, d_n2 = L.kvl_mla_device_alloc(nb), L.kvl_mla_device_alloc(nb)
+    got = {}
+    for on in (1, 0):
+        prev = L.kvl_mla_set_fused_projection(on)
+        try:
+            lib.check(L.kvl_mla_copy_to_device(d_h, h0.ctypes.data, nb), "h2d")
+            lib.check(L.kvl_mla_attention_layer_q8_device(d_h, d_n2, B, C.byref(cfg), C.byref(w), u16(norms[0]),
+                                                          u16(norms[1]), arr, lib.NO_ADVANCE), "layer")
+            h, n2 = np.zeros_like(h0), np.zeros_like(h0)
+            lib.check(L.kvl_mla_copy_to_host(h.ctypes.data, d_h, nb), "d2h")
+            lib.check(L.kvl_mla_copy_to_host(n2.ctypes.data, d_n2, nb), "d2h")
+            got[on] = (h, n2)
+        finally:
+            L.kvl_mla_set_fused_projection(prev)
+    for a, b in zip(got[1], got[0]):
+        assert np.all(np.isfinite(a))
+        np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
+    L.kvl_mla_device_free(d_h)
+    L.kvl_mla_device_free(d_n2)
+    for s in states:
+        L.kvl_mla_compressed_q8_state_free(C.byref(s))
+    lib.check(L.kvl_mla_release_weights(C.byref(w)), "release")
