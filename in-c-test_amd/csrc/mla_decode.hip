@@ -435,29 +435,34 @@ __global__ __launch_bounds__(256) void k_kva_tok(KvaTokArgs a) {
 }
 
 // The same partials for in = 2048 (one 32-wide k-block per k_gemv_ksplit wave) as a tiled
-// GEMM: x hi, x lo and W stream through a 3-stage LDS ring by DMA (16-byte slot s of a 64-byte
+// GEMM: x hi, x lo and W stream through an LDS ring by DMA (16-byte slot s of a 64-byte
 // row r stored at s ^ ((r >> 1) & 3), so the 8 rows of one ds_read_b128 phase hit distinct
-// banks). Block: 128 tokens x 192 rows x one k quarter, 6 waves of 64 tokens x 64 rows (4 x 4
-// MFMA tiles); per 32-wide k step each tile takes one MFMA from a zero accumulator for the hi
+// banks). Block: one k quarter of 16 TU WT tokens x 16 TT WR rows, WT x WR waves of TU x TT
+// MFMA tiles; per 32-wide k step each tile takes one MFMA from a zero accumulator for the hi
 // and one for the lo half, added to the running sums in k order (the sums of k_gemv_ksplit's
 // waves 0..15). Tiles are numbered row block fastest, then quarter, then token block, and XCD
 // b % 8 takes a contiguous eighth of them, so the row blocks sharing a token block's
 // activations run under one L2.
-constexpr int kKvgNT = 2, kKvgNR = 3;  // waves along tokens, along rows
-constexpr int kKvgBT = 64 * kKvgNT, kKvgBR = 64 * kKvgNR;
+template <int TU_, int TT_, int WT_, int WR_, int NS_>
+struct KvgShape {
+    static constexpr int TU = TU_, TT = TT_, WT = WT_, WR = WR_, NS = NS_;  // NS: ring stages
+    static constexpr int BT = 16 * TU * WT, BR = 16 * TT * WR, NT = 64 * WT * WR;
+};
 
-__global__ __launch_bounds__(64 * kKvgNT * kKvgNR) void k_kva_gemm(KvaTokArgs a) {
-    constexpr int NWV = kKvgNT * kKvgNR, NT = 64 * NWV, BT = kKvgBT, BR = kKvgBR;
+template <class Sh>
+__global__ __launch_bounds__(Sh::NT) void k_kva_gemm(KvaTokArgs a) {
+    constexpr int TU = Sh::TU, TT = Sh::TT, NS = Sh::NS;
+    constexpr int NWV = Sh::WT * Sh::WR, NT = Sh::NT, BT = Sh::BT, BR = Sh::BR;
     constexpr int ROWB = 64, XPL = BT * ROWB, STAGE = 2 * XPL + BR * ROWB;
     constexpr int SLOTS = STAGE / 16, NI = (SLOTS + NT - 1) / NT, NMIN = SLOTS / NT;
-    static_assert(SLOTS % 64 == 0, "the ring is filled by whole waves");
-    __shared__ __attribute__((aligned(16))) uint8_t smem[3 * STAGE];
+    static_assert(SLOTS % 64 == 0 && NS >= 2 && NS <= 16 && NS * STAGE <= 160 * 1024, "the ring is filled by whole waves");
+    __shared__ __attribute__((aligned(16))) uint8_t smem[NS * STAGE];
     const uint32_t sbase = lds_addr(smem);
     const int tid = threadIdx.x, l = tid & 63, n = l & 15, g = l >> 4;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), wt = w % kKvgNT, wr = w / kKvgNT;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), wt = w % Sh::WT, wr = w / Sh::WT;
     const int nrb = (a.out + BR - 1) / BR, ntb = (a.S + BT - 1) / BT, nt = nrb * kGemvKs * ntb;
-    int tile = blockIdx.x;
-    if (nt % 8 == 0) tile = (tile & 7) * (nt / 8) + (tile >> 3);
+    const int xcd = blockIdx.x & 7, rem = nt & 7;
+    const int tile = xcd * (nt >> 3) + min(xcd, rem) + (int)(blockIdx.x >> 3);
     const int rb = tile % nrb, kq = (tile / nrb) % kGemvKs, tb = tile / nrb / kGemvKs;
     const int row0 = rb * BR, tok0 = tb * BT;
     auto swz = [](int row) { return (row >> 1) & 3; };
@@ -480,46 +485,46 @@ __global__ __launch_bounds__(64 * kKvgNT * kKvgNR) void k_kva_gemm(KvaTokArgs a)
         src[i] = (const uint8_t *)(rp + kq * 512 + 8 * s);
     }
     auto issue = [&](int j) __attribute__((always_inline)) {
-        const uint32_t dst = sbase + (j % 3) * STAGE + (uint32_t)w * 1024;
+        const uint32_t dst = sbase + (j % NS) * STAGE + (uint32_t)w * 1024;
 #pragma unroll
         for (int i = 0; i < NI; ++i)
             if (i < NMIN || (i * NWV + w) * 64 < SLOTS) dma_b128(src[i] + (size_t)j * 64, dst + i * (NWV * 1024));
     };
-    int fx[4], fw[4];  // fragment offsets: row 16 u + n of the wave's tile, logical slot g
+    int fx[TU], fw[TT];  // fragment offsets: row 16 u + n of the wave's tile, logical slot g
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int row = 64 * wt + 16 * u + n;
+    for (int u = 0; u < TU; ++u) {
+        const int row = 16 * (TU * wt + u) + n;
         fx[u] = row * ROWB + 16 * (g ^ swz(row));
     }
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        const int row = 64 * wr + 16 * t + n;
+    for (int t = 0; t < TT; ++t) {
+        const int row = 16 * (TT * wr + t) + n;
         fw[t] = 2 * XPL + row * ROWB + 16 * (g ^ swz(row));
     }
-    v4f sh[4][4], sl[4][4];
-    issue(0);
-    issue(1);
+    v4f sh[TT][TU], sl[TT][TU];
+#pragma unroll
+    for (int j = 0; j < NS - 1; ++j) issue(j);
     auto step = [&](int j) __attribute__((always_inline)) {
-        // stage j has landed when only stage j + 1 may still be in flight (a wave issues NMIN
-        // or NMIN + 1 copies per stage; waiting for NMIN is exact or conservative)
-        if (j + 1 < 16) wait_vmcnt<NMIN>();
+        // stage j has landed when only the NS - 2 stages after it may still be in flight (a wave
+        // issues NMIN or NMIN + 1 copies per stage; waiting for NMIN each is exact or conservative)
+        if (j + NS - 1 <= 16) wait_vmcnt<(NS - 2) * NMIN>();
         else wait_vmcnt<0>();
         lds_barrier();  // also: every wave is done with stage j - 1, refilled next
-        if (j + 2 < 16) issue(j + 2);
-        const uint8_t *st = smem + (j % 3) * STAGE;
-        v8bf xh[4], xl[4], wv[4];
+        if (j + NS - 1 < 16) issue(j + NS - 1);
+        const uint8_t *st = smem + (j % NS) * STAGE;
+        v8bf xh[TU], xl[TU], wv[TT];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < TU; ++u) {
             xh[u] = *(const v8bf *)(st + fx[u]);
             xl[u] = *(const v8bf *)(st + XPL + fx[u]);
         }
 #pragma unroll
-        for (int t = 0; t < 4; ++t) wv[t] = *(const v8bf *)(st + fw[t]);
+        for (int t = 0; t < TT; ++t) wv[t] = *(const v8bf *)(st + fw[t]);
         const v4f z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+        for (int t = 0; t < TT; ++t)
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < TU; ++u) {
                 const v4f rh = mfma_bf16(wv[t], xh[u], z);
                 const v4f rl = mfma_bf16(wv[t], xl[u], z);
                 sh[t][u] = j == 0 ? rh : sh[t][u] + rh;
@@ -532,13 +537,13 @@ __global__ __launch_bounds__(64 * kKvgNT * kKvgNR) void k_kva_gemm(KvaTokArgs a)
     float *y = a.Y + (size_t)kq * a.pstride;
     const bool vec = (a.ldy & 3) == 0;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int tok = tok0 + 64 * wt + 16 * u + n;
+    for (int u = 0; u < TU; ++u) {
+        const int tok = tok0 + 16 * (TU * wt + u) + n;
         if (tok >= a.S) continue;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+        for (int t = 0; t < TT; ++t) {
             const v4f p = sh[t][u] + sl[t][u];  // lane (g, n): rows 4 g .. 4 g + 3, token n
-            const int r = row0 + 64 * wr + 16 * t + 4 * g;
+            const int r = row0 + 16 * (TT * wr + t) + 4 * g;
             float *yp = y + (size_t)tok * a.ldy + r;
             if (vec && r + 3 < a.out) {
                 *(v4f *)yp = p;
@@ -551,6 +556,14 @@ __global__ __launch_bounds__(64 * kKvgNT * kKvgNR) void k_kva_gemm(KvaTokArgs a)
     }
 }
 
+template <class Sh>
+static hipError_t kva_gemm_launch(hipStream_t st, const KvaTokArgs &a) {
+    const size_t tiles = (size_t)((a.out + Sh::BR - 1) / Sh::BR) * kGemvKs * ((a.S + Sh::BT - 1) / Sh::BT);
+    if (tiles > 0x7fffffff) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_kva_gemm<Sh>), dim3((unsigned)tiles), dim3(Sh::NT), 0, st, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_kva_tok(hipStream_t st, float *Y, size_t pstride, int ldy, const uint16_t *XH,
                           const uint16_t *XL, int S, const uint16_t *W, int out, int in) {
     if (!gemv_ksplit_ok(in, in) || S < 1 || out <= 0 || ldy < out || (S + 127) / 128 > 65535 ||
@@ -559,9 +572,14 @@ hipError_t launch_kva_tok(hipStream_t st, float *Y, size_t pstride, int ldy, con
         return hipErrorInvalidValue;
     KvaTokArgs a{Y, XH, XL, W, pstride, ldy, S, out, in};
     if (in == 2048) {
-        const size_t tiles = (size_t)((out + kKvgBR - 1) / kKvgBR) * kGemvKs * ((S + kKvgBT - 1) / kKvgBT);
-        if (tiles > 0x7fffffff) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(k_kva_gemm, dim3((unsigned)tiles), dim3(64 * kKvgNT * kKvgNR), 0, st, a);
+        // Small tiles while they do not outnumber the places for them (two blocks per CU), so that a
+        // short prompt spreads over the CUs; large ones take in fewer bytes per product. 64 x 64, 64 x
+        // 96, 128 x 192 (us): 9.5 / 11.8 / 17.1 at 37 tokens, 10.1 / 12.2 / 19.4 at 250, 12.5 / 13.4 /
+        // 19.8 at 512, 21.5 / 18.2 / 21.4 at 1181, 31.0 / 26.0 / 22.4 at 2048, - / 171 / 127 at 16000.
+        const long places = 512, tb = (S + 63) / 64 * (long)kGemvKs;
+        if (tb * ((out + 63) / 64) <= places) return kva_gemm_launch<KvgShape<2, 2, 2, 2, 6>>(st, a);
+        if (tb * ((out + 95) / 96) <= places) return kva_gemm_launch<KvgShape<2, 3, 2, 2, 4>>(st, a);
+        return kva_gemm_launch<KvgShape<4, 4, 2, 3, 3>>(st, a);
     } else {
         const dim3 grid((out + 63) / 64, kGemvKs, (S + 127) / 128);
         hipLaunchKernelGGL((k_kva_tok<2>), grid, dim3(256), 0, st, a);

@@ -525,8 +525,10 @@ __global__ __launch_bounds__(256) void k_kva_epi(KvaEpiArgs a) {
 // MFMA route, one wave per token t: latent = RMSNorm(kv_a[t, :R]) * w (as k_kva_epi) as
 // hi/lo bf16 [S, R] for the kv_b GEMM (whose lo pass always runs), and the rotated k_rope
 // (src/mla_prefill_streaming.c:131-138) into the rope part of K for every head, as the fp16
-// hi row and the K8 bytes (bf8 of hi and of lo x 2^11). Tokens S .. Sp-1 zero their Q, K, K8
-// and V^T entries, so padding keys contribute 0 * 0 in the flash kernel.
+// hi row and the K8 bytes (bf8 of hi and of lo x 2^11). The V^T entries of the padding keys S ..
+// Sp - 1 are zeroed (their weights are exactly 0 in the flash kernel, whose mask sets their scores
+// whatever Q and K hold there; rows of padding queries are not stored). Blocks past the tokens do
+// that: with every token's wave also zeroing Q, K and K8 of a padding token, 37 tokens took 9.6 us.
 struct KvaPackArgs {
     const float *y;  // [S, ldy] kv_a projection
     const uint16_t *norm;
@@ -546,22 +548,15 @@ struct KvaPackArgs {
 __global__ __launch_bounds__(256) void k_kva_pack(KvaPackArgs a) {
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.x_flag) *a.x_flag = 0;
-    if (t >= a.Sp) return;
     const int QD = a.DN + a.DR, half = a.DR / 2, R = a.R;
-    if (t >= a.S) {
-        const int tv = (t & ~31) | vt_perm(t & 31);
-        for (int h = 0; h < a.NH; ++h) {
-            const size_t qo = ((size_t)h * a.Sp + t) * QD;
-            for (int k = l; k < QD; k += 64) {
-                a.qh[qo + k] = 0;
-                a.ql8[qo + k] = 0;
-                a.kh[qo + k] = 0;
-            }
-            for (int k = l; k < 96; k += 64) ((uint32_t *)(a.k8 + ((size_t)h * a.Sp + t) * 384))[k] = 0;
-            for (int d = l; d < a.DV; d += 64) a.vt[((size_t)h * a.DV + d) * a.Sp + tv] = 0;
-        }
+    const int tblocks = (a.S + 3) / 4;
+    if ((int)blockIdx.x >= tblocks) {  // padding keys of V^T: 16 rows (h, d) per wave, one key per lane
+        const int r0 = 16 * (t - 4 * tblocks);
+        for (int r = r0; r < min(r0 + 16, a.NH * a.DV); ++r)
+            for (int k = a.S + l; k < a.Sp; k += 64) a.vt[(size_t)r * a.Sp + (k & ~31) + vt_perm(k & 31)] = 0;
         return;
     }
+    if (t >= a.S) return;
     const float *kat = a.y + (size_t)t * a.ldy;
     if (R == 512 && a.DR == 64 && (a.DN & 63) == 0 && (a.ldy & 3) == 0 && (a.pstride & 3) == 0) {
         // lane l: latent columns 8l .. 8l+7 (16-byte loads and stores); the rotated RoPE key
@@ -1261,7 +1256,8 @@ hipError_t launch_prefill_all(hipStream_t st, const Dims &d, int S, float eps, c
         }
         KvaPackArgs ka{ykva, wnorm, cs, lath, latl, qh, ql8, kh, k8, vt, (size_t)S * d.KVO, np,
                        S, Sp, d.NH, d.KVO, d.R, d.DN, d.DR, d.DV, eps, flags + 0};
-        hipLaunchKernelGGL(k_kva_pack, dim3((Sp + 3) / 4), dim3(256), 0, st, ka);
+        const int vpad = Sp > S ? (d.NH * d.DV + 63) / 64 : 0;
+        hipLaunchKernelGGL(k_kva_pack, dim3((S + 3) / 4 + vpad), dim3(256), 0, st, ka);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         // kv_b (-> K nope part as fp16 hi + K8, V^T scaled by vscale)
         ep.vscale = vscale;

@@ -187,3 +187,32 @@ def test_fused_rejects_bad_arguments():
     assert L.kvl_mla_prefill_compressed_q8_state_bf16(f32(out), f32(x), 2, C.byref(cfg), C.byref(w), C.byref(st)) == -1
     assert st.len == 2
     free_state(G, "q8", st)
+
+
+_long_rows = {}
+
+
+def f32_rows(S):
+    """FP32 state rows of the first S tokens of one 2000-token input (bit patterns)."""
+    cfg = inputs.config(**inputs.KIMI)
+    layer = inputs.make_layer(cfg, 0xD7)
+    w = layer.struct()
+    x = np.ascontiguousarray(inputs.hidden(cfg, 0xD7, 2000)[:S])
+    st = abi.KvlMlaCompressedState()
+    lib.check(L.kvl_mla_compressed_state_init(C.byref(st), C.byref(cfg), S), "init")
+    lib.check(L.kvl_mla_compressed_state_prefill_bf16(f32(x), S, C.byref(cfg), C.byref(w), C.byref(st)), "prefill")
+    lat = np.ctypeslib.as_array(st.latent, (S, 512)).copy().view(np.uint32)
+    key = np.ctypeslib.as_array(st.rope, (S, 64)).copy().view(np.uint32)
+    L.kvl_mla_compressed_state_free(C.byref(st))
+    return lat, key
+
+
+@pytest.mark.parametrize("S", [1, 63, 65, 512, 832, 896, 897, 1344, 1345])
+def test_rows_do_not_depend_on_the_prompt_length(S):
+    """A row depends on its token alone, in one summation order: the rows of a shorter prompt equal
+    those of a longer one bit for bit at the edges of the three tile shapes of the kv_a projection
+    (64 x 64 up to 896 tokens, 64 x 96 up to 1344, 128 x 192)."""
+    if 2000 not in _long_rows:
+        _long_rows[2000] = f32_rows(2000)
+    for got, full in zip(f32_rows(S), _long_rows[2000]):
+        np.testing.assert_array_equal(got, full[:S])
