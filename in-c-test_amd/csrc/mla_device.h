@@ -145,6 +145,20 @@ __device__ __forceinline__ void split_f16(float x, _Float16 &hi, _Float16 &lo) {
     hi = (_Float16)x;
     lo = (_Float16)(x - (float)hi);
 }
+// Four values at once; the bf8 bytes of four lo parts x 2^11 (a power of two: exact in fp16).
+__device__ __forceinline__ void split4_f16(const v4f &x, v4h &hi, v4h &lo) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        _Float16 h, l;
+        split_f16(x[i], h, l);
+        hi[i] = h;
+        lo[i] = l;
+    }
+}
+__device__ __forceinline__ uint32_t bf8_lo_s11(const v4h &lo) {
+    const _Float16 s = (_Float16)2048.0f;
+    return f16x4_to_bf8(lo * v4h{s, s, s, s});
+}
 __device__ __forceinline__ void split8_f16(const float *x, v8h &hi, v8h &lo) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {

@@ -74,7 +74,7 @@ __global__ __launch_bounds__(256) void k_split(const float *src, int ld_src, uin
 // columns of C may come from two weight matrices (B0 for n < N0, B1 for the N1 after it),
 // so the q and kv_a projections of the same tokens run as one launch.
 //
-// Block tile BM x BN, MW math waves in a WM x WN grid, each owning (BM / WM) x 64 columns of
+// Block tile BM x BN, MW math waves in a WM x WN grid, each owning (BM / WM) x 16 TN columns of
 // v_mfma_f32_16x16x32 tiles. With LO a stage of the LDS ring holds a k step of Ah, of Al and of
 // B, so each B tile is taken in once for both parts (two passes over k took in 4/3 of the
 // bytes); the Al part is neither fetched nor multiplied when *lo_flag says that it is zero.
@@ -94,7 +94,8 @@ struct GemmCfg {
     static constexpr int BM = BM_, BN = BN_, BK = BK_, MW = MW_, BPC = BPC_;  // BPC: blocks per CU
     static constexpr bool LO = LO_;
     static constexpr int RowB = BK * 2, Spr = BK / 8;  // 16-byte slots per row
-    static constexpr int WN = BN / 64, WM = MW / WN, TM = BM / WM / 16, TN = 4;
+    static constexpr int TN = BN >= 64 ? 4 : BN / 16;  // 16-column tiles per wave
+    static constexpr int WN = BN / (16 * TN), WM = MW / WN, TM = BM / WM / 16;
     static constexpr int ATile = BM * RowB, BTile = BN * RowB;
     static constexpr int Stage = (LO ? 2 : 1) * ATile + BTile;
     static constexpr int Fit = (160 * 1024 / BPC) / Stage;
@@ -111,6 +112,8 @@ struct GemmArgs {
     float *C;
     const int *lo_flag;
     int M, N0, N1, K, lda, ldb, ldc;
+    int ks;          // kEpiPart: k ranges, range s written to C + s * pstride
+    size_t pstride;
 };
 
 // Epilogues. kEpiPlain: C fp32. kEpiQ (q | kv_a projection): the N0 = NH * QD q columns go
@@ -119,7 +122,8 @@ struct GemmArgs {
 // (kv_b projection): k_nope -> K hi [NH, Sp, QD] fp16 and K8 [NH, Sp, 384 bytes] (bf8 of the
 // hi parts and of the lo parts x 2^11, k8_hi_byte order), values -> V^T [NH, DV, Sp] fp16 with
 // the keys of each 32-key group in vt_perm order.
-enum { kEpiPlain = 0, kEpiQ = 1, kEpiKV = 2 };
+// kEpiPart: the fp32 sums of one of a.ks ranges of k (k_kva_pack adds them in order).
+enum { kEpiPlain = 0, kEpiQ = 1, kEpiKV = 2, kEpiPart = 3 };
 struct GemmEpi {
     _Float16 *qh, *kh;
     uint8_t *ql8;  // bf8(Q lo x 2^11), the flash kernel's correction operand (kEpiQ)
@@ -131,6 +135,36 @@ struct GemmEpi {
     float alpha = 1.0f;              // kEpiPlain: C = alpha * acc (a power of two)
     const int *nan_flag = nullptr;   // kEpiPlain: C = NaN when *nan_flag != 0
 };
+
+// Columns nl0 .. nl0 + 3 (nl0 % 4 == 0) of token t of the q projection into Q (kEpiQ). Q (50 MB at
+// 4096 tokens) is read once, by the flash kernel's workgroup of its query tile: non-temporal stores
+// keep it from evicting the K/V and weight lines the next kernels reuse (q GEMM 78 -> 70 us, kv_b
+// GEMM 44 -> 40 us). Q hi as fp16 and Q lo only as the bf8 byte the flash kernel's correction takes
+// (bf8(lo x 2^11)): 37.5 instead of 50 MB written at 4096 tokens.
+__device__ __forceinline__ void store_q4(const GemmEpi &e, int t, int nl0, const v4f &x) {
+    const int QD = e.DN + e.DR, half = e.DR / 2;
+    const int h = nl0 / QD, k0 = nl0 % QD;
+    const size_t o = ((size_t)h * e.Sp + t) * QD;
+    if (k0 < e.DN) {
+        v4h hi, lo;
+        split4_f16(x, hi, lo);
+        __builtin_nontemporal_store(hi, (v4h *)(e.qh + o + k0));
+        __builtin_nontemporal_store(bf8_lo_s11(lo), (uint32_t *)(e.ql8 + o + k0));
+        return;
+    }
+    // pairs (x.x, x.y), (x.z, x.w) of rope indices i2, i2 + 1
+    const int i2 = (k0 - e.DN) >> 1;
+    const float2 *cs = e.cs + (size_t)t * half + i2;
+    const float2 c0 = cs[0], c1 = cs[1];
+    const v4f r = {x.x * c0.x - x.y * c0.y, x.z * c1.x - x.w * c1.y, x.y * c0.x + x.x * c0.y, x.w * c1.x + x.z * c1.y};
+    v4h hi, lo;
+    split4_f16(r, hi, lo);
+    const uint32_t l8 = bf8_lo_s11(lo);
+    __builtin_nontemporal_store(__builtin_shufflevector(hi, hi, 0, 1), (v2h *)(e.qh + o + e.DN + i2));
+    __builtin_nontemporal_store((uint16_t)l8, (uint16_t *)(e.ql8 + o + e.DN + i2));
+    __builtin_nontemporal_store(__builtin_shufflevector(hi, hi, 2, 3), (v2h *)(e.qh + o + e.DN + half + i2));
+    __builtin_nontemporal_store((uint16_t)(l8 >> 16), (uint16_t *)(e.ql8 + o + e.DN + half + i2));
+}
 
 // Position of key k (0..31 within its 32-key group) in the permuted V^T rows: the 8 keys
 // lane group g of the flash kernel holds for one PV chunk are 4g .. 4g+3 and 16+4g .. 16+4g+3.
@@ -165,11 +199,12 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
     const int wm = w / Sh::WN, wn = w % Sh::WN;
     const int M = a.M, N0 = a.N0, N1 = a.N1, K = a.K, lda = a.lda, ldb = a.ldb;
     const int tn0 = (N0 + BN - 1) / BN, tn = tn0 + (N1 + BN - 1) / BN;
-    const int tm = (M + BM - 1) / BM, ntiles = tm * tn;
+    const int tm = (M + BM - 1) / BM, ks = EPI == kEpiPart ? a.ks : 1, ntiles = tm * tn * ks;
     // Tiles in row-major order, XCD b % 8 taking a contiguous eighth of them (blocks of one XCD
     // share A rows in its L2).
     const int xcd = blockIdx.x & 7, per = ntiles >> 3, rem = ntiles & 7;
-    const int tile = xcd * per + min(xcd, rem) + (blockIdx.x >> 3);
+    const int task = xcd * per + min(xcd, rem) + (blockIdx.x >> 3);
+    const int tile = EPI == kEpiPart ? task / ks : task, kr = EPI == kEpiPart ? task % ks : 0;
     const int mt = tile / tn, nt = tile % tn;
     const bool seg1 = nt >= tn0;
     const uint16_t *B = seg1 ? a.B1 : a.B0;
@@ -179,7 +214,7 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
     const int m0 = mt * BM;
     const bool use_lo = Sh::LO && a.Al && (!a.lo_flag || *a.lo_flag);
 
-    const int nkt = K / BK;
+    const int nkt = K / BK / ks, kt0 = kr * nkt;  // this block's k steps (ks divides K / BK)
     constexpr int NS = Sh::Stages;
     if (w >= Sh::MW) {
         // DMA wave dw: instruction i fills slot (4i + dw) * 64 + l of a tile: row p / Spr,
@@ -206,7 +241,7 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
             constexpr bool kLo = decltype(lo_tag)::value;
             auto issue = [&](int kt, int stage) __attribute__((always_inline)) {
                 const uint32_t dst = sbase + stage * Sh::Stage + (uint32_t)dw * 1024;
-                const size_t ko = (size_t)kt * RowB;
+                const size_t ko = (size_t)(kt0 + kt) * RowB;
 #pragma unroll
                 for (int i = 0; i < NA; ++i) dma_b128_s(gah + ko, aoff[i], dst + i * (kGemmDma * 1024));
 #pragma unroll
@@ -287,8 +322,28 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
     // row write its 64 columns as one contiguous run (scattered 16-byte pieces per lane cost
     // ~10 us more per launch at these sizes), and the rope pairs (2p, 2p+1) sit in one lane.
     // The V^T part of kEpiKV wants 4 consecutive tokens per lane, which the D layout gives.
-    const int QD = e.DN + e.DR, KH = e.DN + e.DV, half = e.DR / 2;
-    static_assert(TN == 4, "the staged epilogue assumes 64 columns per wave");
+    if constexpr (TN < 4) {
+        // narrow tiles (kEpiPlain): stored from the D layout, 64-byte runs
+        static_assert(TN == 4 || EPI == kEpiPlain, "the staged epilogue assumes 64 columns per wave");
+        lds_barrier();  // the DMA waves' last barrier
+        float al = e.alpha;
+        if (e.nan_flag && __hip_atomic_load(e.nan_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            al = __builtin_nanf("");
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int c = c0 + wn * TN * 16 + 16 * j + n;
+                if (c - c0 + nb0 >= Nseg) continue;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int t = m0 + wm * TM * 16 + 16 * i + 4 * g + r;
+                    if (t < M) a.C[(size_t)t * a.ldc + c] = acc[i][j][r] * al;
+                }
+            }
+        return;
+    } else {
+    const int QD = e.DN + e.DR, KH = e.DN + e.DV;
     lds_barrier();  // every wave is done with the ring
     float *ep = (float *)smem + w * (16 * 68);
     const int cw = wn * 64;                      // wave's first column within the tile
@@ -333,72 +388,25 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
         for (int q = 0; q < 4; ++q) {
             const int t = rbase + rr + 4 * q;
             if (t >= M) continue;
-            const float v[4] = {vq[q].x, vq[q].y, vq[q].z, vq[q].w};
-            if (EPI == kEpiPlain || (EPI == kEpiQ && seg1)) {
-                float *dst = EPI == kEpiPlain ? a.C + (size_t)t * a.ldc + c0 + cw + cc : a.C + (size_t)t * a.ldc + nl0;
+            if (EPI == kEpiPlain || EPI == kEpiPart || (EPI == kEpiQ && seg1)) {
+                float *dst = EPI == kEpiPlain  ? a.C + (size_t)t * a.ldc + c0 + cw + cc
+                             : EPI == kEpiPart ? a.C + kr * a.pstride + (size_t)t * a.ldc + c0 + cw + cc
+                                               : a.C + (size_t)t * a.ldc + nl0;
                 *(v4f *)dst = EPI == kEpiPlain ? vq[q] * alpha : vq[q];
             } else if (EPI == kEpiQ) {
-                // Q (50 MB at 4096 tokens) is read once, by the flash kernel's workgroup of its
-                // query tile: non-temporal stores keep it from evicting the K/V and weight
-                // lines the next kernels reuse (q GEMM 78 -> 70 us, kv_b GEMM 44 -> 40 us)
-                const int h = nl0 / QD, k0 = nl0 % QD;
-                const size_t o = ((size_t)h * e.Sp + t) * QD;
-                // Q hi as fp16 and Q lo only as the bf8 byte the flash kernel's correction takes
-                // (bf8(lo x 2^11)): 37.5 instead of 50 MB written at 4096 tokens
-                if (k0 < e.DN) {
-                    v4h hi;
-                    uint32_t l8 = 0;
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        _Float16 hh, ll;
-                        split_f16(v[u], hh, ll);
-                        hi[u] = hh;
-                        l8 |= bf8_lo_s11(ll) << (8 * u);
-                    }
-                    __builtin_nontemporal_store(hi, (v4h *)(e.qh + o + k0));
-                    __builtin_nontemporal_store(l8, (uint32_t *)(e.ql8 + o + k0));
-                } else {
-                    // pairs (ev, od) = (v[2p], v[2p+1]) of rope index i2 + p
-                    const int i2 = (k0 - e.DN) >> 1;
-                    const float2 *cs = e.cs + (size_t)t * half + i2;
-                    v2h h0, h1;
-                    uint16_t l0 = 0, l1 = 0;
-#pragma unroll
-                    for (int p = 0; p < 2; ++p) {
-                        const float2 c = cs[p];
-                        const float ev = v[2 * p], od = v[2 * p + 1];
-                        _Float16 hh, ll;
-                        split_f16(ev * c.x - od * c.y, hh, ll);
-                        h0[p] = hh;
-                        l0 |= (uint16_t)(bf8_lo_s11(ll) << (8 * p));
-                        split_f16(od * c.x + ev * c.y, hh, ll);
-                        h1[p] = hh;
-                        l1 |= (uint16_t)(bf8_lo_s11(ll) << (8 * p));
-                    }
-                    __builtin_nontemporal_store(h0, (v2h *)(e.qh + o + e.DN + i2));
-                    __builtin_nontemporal_store(l0, (uint16_t *)(e.ql8 + o + e.DN + i2));
-                    __builtin_nontemporal_store(h1, (v2h *)(e.qh + o + e.DN + half + i2));
-                    __builtin_nontemporal_store(l1, (uint16_t *)(e.ql8 + o + e.DN + half + i2));
-                }
+                store_q4(e, t, nl0, vq[q]);
             } else {  // kEpiKV, k_nope columns
                 const int h = nl0 / KH, k0 = nl0 % KH;
                 const size_t o = ((size_t)h * e.Sp + t) * QD + k0;
-                v4h hi;
-                uint32_t h8 = 0, l8 = 0;
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    _Float16 hh, ll;
-                    split_f16(v[u], hh, ll);
-                    hi[u] = hh;
-                    h8 |= f16_to_bf8(hh) << (8 * u);
-                    l8 |= bf8_lo_s11(ll) << (8 * u);
-                }
+                v4h hi, lo;
+                split4_f16(vq[q], hi, lo);
                 *(v4h *)(e.kh + o) = hi;
                 uint8_t *row = e.k8 + ((size_t)h * e.Sp + t) * 384 + k8_hi_byte(k0);
-                *(uint32_t *)row = h8;
-                *(uint32_t *)(row + kK8Lo) = l8;
+                *(uint32_t *)row = f16x4_to_bf8(hi);
+                *(uint32_t *)(row + kK8Lo) = bf8_lo_s11(lo);
             }
         }
+    }
     }
 }
 
@@ -422,6 +430,25 @@ static hipError_t gemm_launch(hipStream_t st, const GemmArgs &a, const GemmEpi &
 }
 
 enum { kTile64x64 = 0, kTile128x64, kTile128x128, kTile192x128, kTile256x128, kTile256x256, kGemmTiles };
+
+// K ranges of the q | kv_a projection of M tokens: 64 x 64 tiles with the whole of k take in 768 KB
+// each, at the 70 GB/s a CU takes in, so while their number leaves CUs idle k is split over 2 or 4
+// blocks, whose sums go through memory to k_kva_pack. Alone, whole k / 2 / 4 ranges (us): 10.3 / 6.8 / 5.0 at
+// 37 tokens (57 tiles), 11.6 / 8.1 / 8.4 at 100 (114), 12.8 / 12.3 / 12.0 at 192 (171).
+static int gemm_part_ks(int M, int N0, int N1, int K) {
+    const int tiles = (M + 63) / 64 * ((N0 + 63) / 64 + (N1 + 63) / 64);
+    const int ks = tiles <= 64 ? 4 : tiles <= 128 ? 2 : 1;
+    return K % (64 * ks) == 0 && N0 % 4 == 0 && N1 % 4 == 0 ? ks : 1;
+}
+
+static hipError_t gemm_part(hipStream_t st, const uint16_t *Ah, const uint16_t *Al, const int *flag, int lda,
+                            const uint16_t *B0, int N0, const uint16_t *B1, int N1, int ldb, float *C, int M, int K,
+                            int ks) {
+    GemmArgs a{Ah, Al, B0, B1 ? B1 : B0, C, flag, M, N0, N1, K, lda, ldb, N0 + N1, ks, (size_t)M * (N0 + N1)};
+    if (K % (64 * ks)) return hipErrorInvalidValue;
+    const int tiles = (M + 63) / 64 * ((N0 + 63) / 64 + (N1 + 63) / 64);
+    return gemm_launch<GemmCfg<64, 64, 64, 4, 2, true>, kEpiPart, false>(st, a, GemmEpi{}, tiles * ks);
+}
 
 static int gemm_pick(int epi, int M, int N0, int N1, int *tiles) {
     static const int bm[kGemmTiles] = {64, 128, 128, 192, 256, 256}, bn[kGemmTiles] = {64, 64, 128, 128, 128, 256};
@@ -450,11 +477,17 @@ template <int EPI, bool F16 = false>
 static hipError_t gemm(hipStream_t st, const uint16_t *Ah, const uint16_t *Al, const int *flag,
                        int lda, const uint16_t *B0, int N0, const uint16_t *B1, int N1, int ldb,
                        float *C, int ldc, int M, int K, const GemmEpi &e) {
-    GemmArgs a{Ah, Al, B0, B1 ? B1 : B0, C, flag, M, N0, N1, K, lda, ldb, ldc};
+    GemmArgs a{Ah, Al, B0, B1 ? B1 : B0, C, flag, M, N0, N1, K, lda, ldb, ldc, 1, 0};
     if (K % 64) return hipErrorInvalidValue;
     constexpr bool LO = !F16;  // the fp16 product has no lo operand
     if (!LO && Al) return hipErrorInvalidValue;
     int tiles = 0;
+    if constexpr (EPI == kEpiPlain) {
+        // half-width tiles while every one has a CU (o_proj up to 256 tokens): half the weights per
+        // block; 37 tokens 8.2 -> 6.4 us, 250 tokens 8.8 -> 8.1, beyond one round slower
+        tiles = (M + 63) / 64 * ((N0 + 31) / 32);
+        if (N1 == 0 && tiles <= 256) return gemm_launch<GemmCfg<64, 32, 64, 4, 2, LO>, EPI, F16>(st, a, e, tiles);
+    }
     switch (gemm_pick(EPI, M, N0, N1, &tiles)) {
     case kTile64x64: return gemm_launch<GemmCfg<64, 64, 64, 4, 2, LO>, EPI, F16>(st, a, e, tiles);
     case kTile128x64: return gemm_launch<GemmCfg<128, 64, 64, 4, 1, LO>, EPI, F16>(st, a, e, tiles);
@@ -543,6 +576,12 @@ struct KvaPackArgs {
     int np, S, Sp, NH, ldy, R, DN, DR, DV;
     float eps;
     int *x_flag;     // the x lo flag, cleared for the next prefill (its one reader has run)
+    // q (may be null): nq partials of the q projection [S, ldq], qpstride floats apart; blocks past
+    // the tokens and the padding add them in order and write Q (store_q4)
+    const float *q;
+    size_t qpstride;
+    int nq, ldq, pad_blocks;
+    GemmEpi qe;
 };
 
 __global__ __launch_bounds__(256) void k_kva_pack(KvaPackArgs a) {
@@ -550,6 +589,16 @@ __global__ __launch_bounds__(256) void k_kva_pack(KvaPackArgs a) {
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.x_flag) *a.x_flag = 0;
     const int QD = a.DN + a.DR, half = a.DR / 2, R = a.R;
     const int tblocks = (a.S + 3) / 4;
+    if ((int)blockIdx.x >= tblocks + a.pad_blocks) {
+        const int i = ((int)blockIdx.x - tblocks - a.pad_blocks) * 256 + threadIdx.x, per = a.NH * QD / 4;
+        if (i >= a.S * per) return;
+        const int tq = i / per, c = 4 * (i % per);
+        const float *q = a.q + (size_t)tq * a.ldq + c;
+        v4f v = *(const v4f *)q;
+        for (int p = 1; p < a.nq; ++p) v += *(const v4f *)(q + p * a.qpstride);
+        store_q4(a.qe, tq, c, v);
+        return;
+    }
     if ((int)blockIdx.x >= tblocks) {  // padding keys of V^T: 16 rows (h, d) per wave, one key per lane
         const int r0 = 16 * (t - 4 * tblocks);
         for (int r = r0; r < min(r0 + 16, a.NH * a.DV); ++r)
@@ -1177,6 +1226,9 @@ size_t prefill_bytes(const Dims &d, int S, bool generic) {
         add(2 * (size_t)S * d.H);                // x hi
         add(2 * (size_t)S * d.H);                // x lo
         add(4 * (size_t)S * d.KVO * (prefill_kva_exact(d) ? kGemvKs : 1));  // kv_a projection
+        // partials of a split q | kv_a projection (of q alone where a state fill asks for its own kv_a)
+        const int k0 = gemm_part_ks(S, d.QO, 0, d.H), k1 = gemm_part_ks(S, d.QO, d.KVO, d.H);
+        add(4 * (size_t)S * std::max(k0 > 1 ? k0 * d.QO : 0, k1 > 1 ? k1 * (d.QO + d.KVO) : 0));
         add(2 * (size_t)S * d.R);                // latent hi
         add(2 * (size_t)S * d.R);                // latent lo
         add(2 * (size_t)d.NH * Sp * d.QD);       // q hi (fp16)
@@ -1221,7 +1273,9 @@ hipError_t launch_prefill_all(hipStream_t st, const Dims &d, int S, float eps, c
         uint16_t *xl = (uint16_t *)take(2 * (size_t)S * d.H);
         const bool exact = kva && prefill_kva_exact(d);
         const int np = exact ? kGemvKs : 1;
+        const int qn1 = exact ? 0 : d.KVO, ks = gemm_part_ks(S, d.QO, qn1, d.H);
         float *ykva = (float *)take(4 * (size_t)S * d.KVO * np);
+        float *ypart = ks > 1 ? (float *)take(4 * (size_t)S * ks * (d.QO + qn1)) : nullptr;
         uint16_t *lath = (uint16_t *)take(2 * (size_t)S * d.R);
         uint16_t *latl = (uint16_t *)take(2 * (size_t)S * d.R);
         _Float16 *qh = (_Float16 *)take(2 * (size_t)d.NH * Sp * d.QD);
@@ -1242,22 +1296,25 @@ hipError_t launch_prefill_all(hipStream_t st, const Dims &d, int S, float eps, c
         // q (-> Q hi/lo, rotated) | kv_a (-> ykva). When the caller fills a state from this
         // kv_a, it is computed with the decode's k-split arithmetic (launch_kva_tok) so those
         // rows equal the rows a decode appends; otherwise it rides along in the q GEMM.
+        // A short prompt splits k (gemm_part_ks) and k_kva_pack adds the partials.
+        if (ks > 1) e = gemm_part(st, xh, xl, flags + 0, d.H, wq, d.QO, exact ? nullptr : wkva, qn1, d.H, ypart, S, d.H, ks);
+        else if (exact) e = gemm<kEpiQ>(st, xh, xl, flags + 0, d.H, wq, d.QO, nullptr, 0, d.H, nullptr, 0, S, d.H, ep);
+        else e = gemm<kEpiQ>(st, xh, xl, flags + 0, d.H, wq, d.QO, wkva, d.KVO, d.H, ykva, d.KVO, S, d.H, ep);
+        if (e != hipSuccess) return e;
         if (exact) {
-            if ((e = gemm<kEpiQ>(st, xh, xl, flags + 0, d.H, wq, d.QO, nullptr, 0, d.H, nullptr, 0, S, d.H,
-                                 ep)) != hipSuccess)
-                return e;
             if ((e = launch_kva_tok(st, ykva, (size_t)S * d.KVO, d.KVO, xh, xl, S, wkva, d.KVO, d.H)) !=
                 hipSuccess)
                 return e;
             if (kva) *kva = PrefillKva{ykva, d.KVO, np, (size_t)S * d.KVO};
-        } else if ((e = gemm<kEpiQ>(st, xh, xl, flags + 0, d.H, wq, d.QO, wkva, d.KVO, d.H, ykva, d.KVO, S,
-                                    d.H, ep)) != hipSuccess) {
-            return e;
         }
-        KvaPackArgs ka{ykva, wnorm, cs, lath, latl, qh, ql8, kh, k8, vt, (size_t)S * d.KVO, np,
-                       S, Sp, d.NH, d.KVO, d.R, d.DN, d.DR, d.DV, eps, flags + 0};
-        const int vpad = Sp > S ? (d.NH * d.DV + 63) / 64 : 0;
-        hipLaunchKernelGGL(k_kva_pack, dim3((S + 3) / 4 + vpad), dim3(256), 0, st, ka);
+        const int vpad = Sp > S ? (d.NH * d.DV + 63) / 64 : 0, ldq = d.QO + qn1;
+        const bool kpart = ks > 1 && !exact;  // kv_a is part of the split projection
+        KvaPackArgs ka{kpart ? ypart + d.QO : ykva, wnorm, cs, lath, latl, qh, ql8, kh, k8, vt,
+                       kpart ? (size_t)S * ldq : (size_t)S * d.KVO, kpart ? ks : np,
+                       S, Sp, d.NH, kpart ? ldq : d.KVO, d.R, d.DN, d.DR, d.DV, eps, flags + 0,
+                       ypart, (size_t)S * ldq, ks, ldq, vpad, ep};
+        const int qblocks = ks > 1 ? (int)(((size_t)S * (d.QO / 4) + 255) / 256) : 0;
+        hipLaunchKernelGGL(k_kva_pack, dim3((S + 3) / 4 + vpad + qblocks), dim3(256), 0, st, ka);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         // kv_b (-> K nope part as fp16 hi + K8, V^T scaled by vscale)
         ep.vscale = vscale;
