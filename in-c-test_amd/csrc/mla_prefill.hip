@@ -745,21 +745,25 @@ __global__ __launch_bounds__(256) void k_kva_pack(KvaPackArgs a) {
 // p <= 256 and most tiles skip the rescale.
 //
 // The two waves of a SIMD (w and w + 4) take the two key halves with separate running maxima and
-// sums, and work half a step apart: in step j the first computes QK, softmax and PV of tile j, the
-// second softmax and PV of tile j - 1 and then QK of tile j, so one's softmax runs under the
-// other's MFMAs. K tiles stream through a two-slot LDS ring and V tiles through a three-slot one
-// (step j + 1 still reads V of tile j), filled by global_load_lds_dwordx4 DMA one step ahead; the
-// waves of the second half issue theirs at the start of a step and those of the first after their
-// QK, each under the other's MFMAs (the 64 KB take a quarter of a step to issue). The halves are
-// merged through LDS at the end. The 16-byte slots of each LDS row are XOR-swizzled by the row so
-// that the fragment reads are free of bank conflicts.
+// sums, and work half a step apart, so that one's softmax runs under the other's MFMAs: both run
+// the same loop (QK of tile j, then its softmax and PV), the first passing the barrier of step j
+// before QK(j), the second that of step j + 1 after it. K tiles stream through a two-slot LDS ring
+// and V tiles through a three-slot one (the second half reads V one step later), filled by
+// global_load_lds_dwordx4 DMA one step ahead; each half issues its share after its QK, under the
+// other's MFMAs (the 64 KB take a quarter of a step to issue). The halves are merged through LDS at
+// the end. The 16-byte slots of each LDS row are XOR-swizzled by the row so that the fragment reads
+// are free of bank conflicts.
 //
-// Bound by the serial chain of a wave's step (LDS reads -> MFMAs -> softmax -> MFMAs) rather than
-// by a unit: without the DMA 1577 us at 16000 tokens, MFMA busy for about 930 of them. Measured
-// alone (us, 37 / 1181 / 4096 / 16000 tokens): 11.2 / 46.0 / 161 / 1944 with one wave per SIMD
-// (32 queries, all 64 keys, QK of the next tile interleaved with the softmax by hand), 11.6 / 44.6
-// / 160 / 1992 with two, 11.1 / 41.0 / 148 / 1787 with the cross-lane max taken only when it moves,
-// 10.9 / 37.5 / 144 / 1763 with the DMA of the two halves apart.
+// Bound by the serial chain of a wave's step (LDS reads -> MFMAs -> softmax -> MFMAs) and the DMA
+// rather than by one unit (16000 tokens: MFMA busy for about 930 us), short prompts by the prologue
+// and by fetching the code once. Measured alone (us, 37 / 1181 / 4096 / 16000 tokens):
+//   11.2 / 46.0 / 161 / 1944  one wave per SIMD (32 queries, all 64 keys), hand-interleaved
+//   11.6 / 44.6 / 160 / 1992  two, on the key halves
+//   11.1 / 41.0 / 148 / 1787  the cross-lane max taken only when it moves, bf8 by hardware
+//   10.9 / 37.5 / 144 / 1763  the DMA of the two halves apart
+//   11.0 / 36.5 / 139 / 1700  one loop for both, K fragments read two groups ahead (two copies of
+//                             the loop left the compiler too few registers for that)
+//   10.3 / 36.0 / 139 / 1687  V fragments read before the weights, one copy of the merge
 constexpr int kFQ = 128, kFK = 64;
 constexpr int kFKB = kFK * 192 * 2;  // K tile (hi or lo): 64 rows x 384 B
 constexpr int kFVB = 128 * kFK * 2;  // V^T tile: 128 rows x 128 B
@@ -861,14 +865,17 @@ void k_flash_prefill(FlashArgs a) {
     };
     issue(0, 0);
 
-    // Q^T B operands: query qw + 16u + n, dims 32kb + 8g .. +7: hi as fp16 (main pass), lo as
+    // Query tile u of a wave of the second half is tile 1 - u of the first: the merge below is then
+    // the same code for both (the kernel's first pass through its code is instruction fetch).
+    const int qu[2] = {qw + 16 * half + n, qw + 16 * (1 - half) + n};  // this lane's query of tile u
+    // Q^T B operands: query qu[u], dims 32kb + 8g .. +7: hi as fp16 (main pass), lo as
     // its bf8(lo x 2^11) bytes (the correction operand below, written so by the q GEMM)
     v8h qa[2][6];
     uint2 qb[2][6];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-        const _Float16 *ph = a.qh + (hq + qw + 16 * u + n) * 192 + 8 * g;
-        const uint8_t *pl = a.ql8 + (hq + qw + 16 * u + n) * 192 + 8 * g;
+        const _Float16 *ph = a.qh + (hq + qu[u]) * 192 + 8 * g;
+        const uint8_t *pl = a.ql8 + (hq + qu[u]) * 192 + 8 * g;
 #pragma unroll
         for (int kb = 0; kb < 6; ++kb) {
             qa[u][kb] = *(const v8h *)(ph + 32 * kb);
@@ -925,39 +932,46 @@ void k_flash_prefill(FlashArgs a) {
         for (int u = 0; u < 2; ++u) acc[dt][u] = v4f{0.f, 0.f, 0.f, 0.f};
     v4f sc[2][2];
 
-    // scores of tile j (K slot j & 1): each accumulator receives its products in the order Kh Qh
-    // for kb = 0 .. 5, then the corrections m = 0 .. 2
+    // Scores of tile j (K slot j & 1): each accumulator receives its products in the order Kh Qh
+    // for kb = 0 .. 5, then the corrections m = 0 .. 2. Six groups of four independent MFMAs and six
+    // of two (twice as long); each group is followed by the fragment reads of the next but one.
     auto qk = [&](int j) __attribute__((always_inline)) {
         const uint8_t *kt = smem + (j & 1) * 2 * kFKB;
+        v8h kf[2][2];
+        v8i k8[2];
+        auto load_kh = [&](int kb) __attribute__((always_inline)) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) kf[kb & 1][t] = *(const v8h *)(kt + t * 16 * 384 + krd[kb]);
+        };
+        auto load_k8 = [&](int c) __attribute__((always_inline)) {  // correction c / 2 of key tile c & 1
+            const uint8_t *r = kt + kFKB + (c & 1) * 16 * 384;
+            const v4i x0 = *(const v4i *)(r + krd[c & ~1]), x1 = *(const v4i *)(r + krd[c | 1]);
+            k8[c & 1] = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
+        };
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int u = 0; u < 2; ++u) sc[t][u] = v4f{0.f, 0.f, 0.f, 0.f};
-        auto load_k8 = [&](int m, int t) __attribute__((always_inline)) {
-            const v4i x0 = *(const v4i *)(kt + kFKB + t * 16 * 384 + krd[2 * m]);
-            const v4i x1 = *(const v4i *)(kt + kFKB + t * 16 * 384 + krd[2 * m + 1]);
-            return __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
-        };
+        load_kh(0);
+        load_kh(1);
 #pragma unroll
         for (int kb = 0; kb < 6; ++kb) {
-            v8h kf[2];
-#pragma unroll
-            for (int t = 0; t < 2; ++t) kf[t] = *(const v8h *)(kt + t * 16 * 384 + krd[kb]);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int u = 0; u < 2; ++u) sc[t][u] = mfma_f16(kf[t], qa[u][kb], sc[t][u]);
+                for (int u = 0; u < 2; ++u) sc[t][u] = mfma_f16(kf[kb & 1][t], qa[u][kb], sc[t][u]);
+            if (kb + 2 < 6) load_kh(kb + 2);
+            else load_k8(kb - 4);
         }
 #pragma unroll
-        for (int m = 0; m < 3; ++m) {
-            v8i kf[2];
+        for (int c = 0; c < 6; ++c) {
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int t = 0; t < 2; ++t) kf[t] = load_k8(m, t);
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int u = 0; u < 2; ++u) sc[t][u] = mfma_bf8_s11(kf[t], q8[u][m], sc[t][u]);
+            for (int u = 0; u < 2; ++u) sc[c & 1][u] = mfma_bf8_s11(k8[c & 1], q8[u][c >> 1], sc[c & 1][u]);
+            if (c + 2 < 6) load_k8(c + 2);
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
     // softmax of this wave's half of tile j and its share of O^T += V^T P^T (V slot vs)
     auto smpv = [&](int j, int vs) __attribute__((always_inline)) {
@@ -970,7 +984,7 @@ void k_flash_prefill(FlashArgs a) {
                 for (int u = 0; u < 2; ++u)
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                        if (k0 + 16 * t + 4 * g + i > qw + 16 * u + n) sc[t][u][i] = -INFINITY;
+                        if (k0 + 16 * t + 4 * g + i > qu[u]) sc[t][u][i] = -INFINITY;
         }
         // The running max moves only when a score of the tile exceeds it by more than kFLazy, which
         // each lane can tell from its own scores; the max over a query's four lanes is taken then.
@@ -991,6 +1005,10 @@ void k_flash_prefill(FlashArgs a) {
                 for (int dt = 0; dt < 8; ++dt) acc[dt][u] *= alpha;
             }
         }
+        v8h vv0[4];
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) vv0[dt] = *(const v8h *)(vt + dt * 16 * 128);
+        __builtin_amdgcn_sched_barrier(0);
         v8h pb[2];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
@@ -1007,76 +1025,68 @@ void k_flash_prefill(FlashArgs a) {
         }
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) {
-            const v8h vv = *(const v8h *)(vt + dt * 16 * 128);
 #pragma unroll
-            for (int u = 0; u < 2; ++u) acc[dt][u] = mfma_f16(vv, pb[u], acc[dt][u]);
+            for (int u = 0; u < 2; ++u) acc[dt][u] = mfma_f16(vv0[dt & 3], pb[u], acc[dt][u]);
+            if (dt < 4) vv0[dt] = *(const v8h *)(vt + (dt + 4) * 16 * 128);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
     // a tile whose first key of this half comes after this wave's last query adds nothing
     auto live = [&](int j) __attribute__((always_inline)) { return j * kFK + 32 * half <= qw + 31; };
 
+    // Both halves run one loop, QK(j) then softmax and PV of tile j; the second passes the barrier of
+    // step j + 1 between the two, the first before QK(j). Passing the barrier of step j: tile j is in
+    // LDS, and every wave is done with K(j - 1) and V(j - 2).
+    auto pass = [&]() __attribute__((always_inline)) {
+        wait_vmcnt<0>();
+        lds_barrier();
+    };
+    if (half) {
+        pass();
+        if (1 < nt) issue(1, 1);
+    }
     int vs = 0;  // V slot of tile j
-    if (half == 0) {
-        for (int j = 0; j < nt; ++j) {
-            wait_vmcnt<0>();
-            lds_barrier();  // tile j is in LDS; every wave is done with K(j - 1) and V(j - 2)
-            const int vn = vs == 2 ? 0 : vs + 1;
-            if (live(j)) qk(j);
-            if (j + 1 < nt) issue(j + 1, vn);
-            if (live(j)) smpv(j, vs);
-            vs = vn;
-        }
-    } else {
-        int vp = 0;
-        for (int j = 0; j < nt; ++j) {
-            wait_vmcnt<0>();
-            lds_barrier();
-            const int vn = vs == 2 ? 0 : vs + 1;
-            if (j + 1 < nt) issue(j + 1, vn);
-            if (j > 0 && live(j - 1)) smpv(j - 1, vp);
-            if (live(j)) qk(j);
-            vp = vs;
-            vs = vn;
-        }
-        if (live(nt - 1)) smpv(nt - 1, vp);
+    for (int j = 0; j < nt; ++j) {
+        const int v1 = vs == 2 ? 0 : vs + 1, v2 = v1 == 2 ? 0 : v1 + 1;
+        const int ti = j + 1 + half, vi = half ? v2 : v1;  // the tile this wave issues in this step
+        if (!half) pass();
+        if (live(j)) qk(j);
+        if (half && j + 1 < nt) pass();
+        if (ti < nt) issue(ti, vi);
+        if (live(j)) smpv(j, vs);
+        vs = v1;
     }
 
-    // Merge of the two key halves: wave w gives query tile u = 1 - half to wave w ^ 4 and
-    // finishes tile u = half.
+    // Merge of the two key halves: wave w gives its query tile 1 to wave w ^ 4, whose tile 0 that is,
+    // and finishes its own tile 0.
     lds_barrier();  // the ring is free
     float *xw = (float *)(smem + w * 9216), *xr = (float *)(smem + (w ^ 4) * 9216);
-    auto give = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt) *(v4f *)(xw + 256 * dt + 4 * l) = acc[dt][u];
-        xw[2048 + l] = m_run[u];
-        xw[2112 + l] = l_run[u];
-    };
+    for (int dt = 0; dt < 8; ++dt) *(v4f *)(xw + 256 * dt + 4 * l) = acc[dt][1];
+    xw[2048 + l] = m_run[1];
+    xw[2112 + l] = l_run[1];
+    lds_barrier();
     // range check of each query row: the reference max (log2 units, within kFLazy of the row's
-    // true max) and every output value (NaN or Inf from operands beyond the fp16 range)
+    // true max) and every output value (NaN or Inf from operands beyond the fp16 range: an
+    // exponent field of ones, which the addition carries into the sign bit)
     bool bad = false;
-    auto finish = [&](int u) __attribute__((always_inline)) {
-        const float m1 = xr[2048 + l], m = fmaxf(m_run[u], m1);
-        const float a0 = __builtin_amdgcn_exp2f(m_run[u] - m), a1 = __builtin_amdgcn_exp2f(m1 - m);
-        const int q = qw + 16 * u + n;
-        const float inv = 1.0f / xrow_sum(l_run[u] * a0 + xr[2112 + l] * a1);
-        if (q >= S) return;
-        bad |= !(fabsf(m) <= kFLogitMax * 1.4426950408889634f);  // m = logit * log2(e)
-        _Float16 *o = a.o + (size_t)q * ldo + (size_t)h * 128 + 4 * g;
+    const float m1 = xr[2048 + l], m = fmaxf(m_run[0], m1);
+    const float a0 = __builtin_amdgcn_exp2f(m_run[0] - m), a1 = __builtin_amdgcn_exp2f(m1 - m);
+    const float inv = 1.0f / xrow_sum(l_run[0] * a0 + xr[2112 + l] * a1);
+    if (qu[0] < S) {
+        uint32_t ones = 0;
+        _Float16 *o = a.o + (size_t)qu[0] * ldo + (size_t)h * 128 + 4 * g;
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) {
-            const v4f s = acc[dt][u] * a0 + *(const v4f *)(xr + 256 * dt + 4 * l) * a1;
+            const v4f s = acc[dt][0] * a0 + *(const v4f *)(xr + 256 * dt + 4 * l) * a1;
             const v4h ov = {(_Float16)(s[0] * inv), (_Float16)(s[1] * inv), (_Float16)(s[2] * inv),
                             (_Float16)(s[3] * inv)};
-#pragma unroll
-            for (int i = 0; i < 4; ++i) bad |= !__builtin_isfinite((float)ov[i]);
+            const uint2 ob = __builtin_bit_cast(uint2, ov);
+            ones |= ((ob.x & 0x7c007c00u) + 0x04000400u) | ((ob.y & 0x7c007c00u) + 0x04000400u);
             *(v4h *)(o + 16 * dt) = ov;
         }
-    };
-    if (half == 0) give(1);
-    else give(0);
-    lds_barrier();
-    if (half == 0) finish(0);
-    else finish(1);
+        bad = (ones & 0x80008000u) != 0 || !(fabsf(m) <= kFLogitMax * 1.4426950408889634f);  // m = logit * log2(e)
+    }
     // any writer stores the same value; the readers are later kernels
     if (__builtin_amdgcn_ballot_w64(bad) != 0 && l == 0) {
         __hip_atomic_store(a.flag_call, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
