@@ -89,19 +89,23 @@ __global__ __launch_bounds__(256) void k_split(const float *src, int ld_src, uin
 // and ldb multiples of 8.
 constexpr int kGemmDma = 4;  // DMA waves of a GEMM block
 
-template <int BM_, int BN_, int BK_, int MW_, int BPC_, bool LO_>
+// AF32 (with LO): A comes as fp32 (GemmArgs::Af) and the math waves split it (split8_cvt, the words
+// k_split makes of finite values): the bytes of the two planes, without the launch that writes them.
+template <int BM_, int BN_, int BK_, int MW_, int BPC_, bool LO_, bool AF32_ = false>
 struct GemmCfg {
     static constexpr int BM = BM_, BN = BN_, BK = BK_, MW = MW_, BPC = BPC_;  // BPC: blocks per CU
-    static constexpr bool LO = LO_;
+    static constexpr bool LO = LO_, AF32 = AF32_;
     static constexpr int RowB = BK * 2, Spr = BK / 8;  // 16-byte slots per row
     static constexpr int TN = BN >= 64 ? 4 : BN / 16;  // 16-column tiles per wave
     static constexpr int WN = BN / (16 * TN), WM = MW / WN, TM = BM / WM / 16;
     static constexpr int ATile = BM * RowB, BTile = BN * RowB;
-    static constexpr int Stage = (LO ? 2 : 1) * ATile + BTile;
+    static constexpr int Stage = (LO ? 2 : 1) * ATile + BTile;  // A hi, B, A lo; AF32: A, B
+    static constexpr int BOff = (AF32 ? 2 : 1) * ATile, ALo = ATile + BTile;
     static constexpr int Fit = (160 * 1024 / BPC) / Stage;
     static constexpr int Stages = Fit > 8 ? 8 : Fit;  // ring depth that fits
     static constexpr int Smem = Stages * Stage;
     static constexpr int Threads = 64 * (MW + kGemmDma);
+    static_assert(LO || !AF32, "fp32 A is split into hi and lo");
     static_assert(Stages >= 2 && TM >= 1 && WM * WN == MW && WM * TM * 16 == BM, "tile shape");
     static_assert(Smem >= MW * 16 * 68 * 4, "the epilogue's staging fits the ring");
     __device__ static int swz(int row) { return BK == 64 ? row & 7 : (row >> 1) & 3; }
@@ -114,6 +118,8 @@ struct GemmArgs {
     int M, N0, N1, K, lda, ldb, ldc;
     int ks;          // kEpiPart: k ranges, range s written to C + s * pstride
     size_t pstride;
+    const float *Af;  // fp32 A [M, lda] (GemmCfg::AF32)
+    int *clear;       // a word the launch clears (may be null)
 };
 
 // Epilogues. kEpiPlain: C fp32. kEpiQ (q | kv_a projection): the N0 = NH * QD q columns go
@@ -212,7 +218,8 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
     const int nb0 = seg1 ? (nt - tn0) * BN : nt * BN;  // first row of B in this tile
     const int c0 = seg1 ? N0 + nb0 : nb0;              // first column of C
     const int m0 = mt * BM;
-    const bool use_lo = Sh::LO && a.Al && (!a.lo_flag || *a.lo_flag);
+    const bool use_lo = Sh::LO && (Sh::AF32 || (a.Al && (!a.lo_flag || *a.lo_flag)));
+    if (a.clear && blockIdx.x == 0 && tid == 0) __hip_atomic_store(a.clear, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 
     const int nkt = K / BK / ks, kt0 = kr * nkt;  // this block's k steps (ks divides K / BK)
     constexpr int NS = Sh::Stages;
@@ -223,7 +230,14 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
         const int dw = w - Sh::MW;
         constexpr int NA = Sh::ATile / (kGemmDma * 1024), NB = Sh::BTile / (kGemmDma * 1024);
         static_assert(NA >= 1 && NB >= 1, "whole DMA instructions per tile");
-        uint32_t aoff[NA], boff[NB];
+        uint32_t aoff[(Sh::AF32 ? 2 : 1) * NA], boff[NB];
+        if constexpr (Sh::AF32) {
+#pragma unroll
+            for (int i = 0; i < 2 * NA; ++i) {  // fp32 rows: twice the slots, the low three bits swizzled
+                const int p = (kGemmDma * i + dw) * 64 + l, row = p / (2 * Spr), s = (p % (2 * Spr)) ^ (row & 7);
+                aoff[i] = (uint32_t)(min(m0 + row, M - 1) - m0) * lda * 4 + 16 * s;
+            }
+        } else
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
             const int p = (kGemmDma * i + dw) * 64 + l, row = p / Spr, s = (p % Spr) ^ Sh::swz(row);
@@ -234,8 +248,8 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
             const int p = (kGemmDma * i + dw) * 64 + l, row = p / Spr, s = (p % Spr) ^ Sh::swz(row);
             boff[i] = (uint32_t)(min(nb0 + row, Nseg - 1) - nb0) * ldb * 2 + 16 * s;
         }
-        const uint8_t *gah = (const uint8_t *)(a.Ah + (size_t)m0 * lda);
-        const uint8_t *gal = use_lo ? (const uint8_t *)(a.Al + (size_t)m0 * lda) : gah;
+        const uint8_t *gah = Sh::AF32 ? (const uint8_t *)(a.Af + (size_t)m0 * lda) : (const uint8_t *)(a.Ah + (size_t)m0 * lda);
+        const uint8_t *gal = use_lo && !Sh::AF32 ? (const uint8_t *)(a.Al + (size_t)m0 * lda) : gah;
         const uint8_t *gb = (const uint8_t *)(B + (size_t)nb0 * ldb);
         auto stream = [&](auto lo_tag) __attribute__((always_inline)) {
             constexpr bool kLo = decltype(lo_tag)::value;
@@ -243,13 +257,14 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
                 const uint32_t dst = sbase + stage * Sh::Stage + (uint32_t)dw * 1024;
                 const size_t ko = (size_t)(kt0 + kt) * RowB;
 #pragma unroll
-                for (int i = 0; i < NA; ++i) dma_b128_s(gah + ko, aoff[i], dst + i * (kGemmDma * 1024));
+                for (int i = 0; i < (Sh::AF32 ? 2 : 1) * NA; ++i)
+                    dma_b128_s(gah + (Sh::AF32 ? 2 * ko : ko), aoff[i], dst + i * (kGemmDma * 1024));
 #pragma unroll
-                for (int i = 0; i < NB; ++i) dma_b128_s(gb + ko, boff[i], dst + Sh::ATile + i * (kGemmDma * 1024));
-                if constexpr (kLo) {
+                for (int i = 0; i < NB; ++i) dma_b128_s(gb + ko, boff[i], dst + Sh::BOff + i * (kGemmDma * 1024));
+                if constexpr (kLo && !Sh::AF32) {
 #pragma unroll
                     for (int i = 0; i < NA; ++i)
-                        dma_b128_s(gal + ko, aoff[i], dst + Sh::ATile + Sh::BTile + i * (kGemmDma * 1024));
+                        dma_b128_s(gal + ko, aoff[i], dst + Sh::ALo + i * (kGemmDma * 1024));
                 }
             };
 #pragma unroll
@@ -264,7 +279,7 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
                 fill = fill + 1 == NS ? 0 : fill + 1;
             }
         };
-        if (use_lo) stream(std::integral_constant<bool, Sh::LO>{});
+        if (Sh::AF32 || use_lo) stream(std::integral_constant<bool, Sh::LO>{});
         else stream(std::false_type{});
         lds_barrier();  // the math waves' epilogue barrier
         return;
@@ -290,16 +305,26 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
 #pragma unroll
             for (int ks = 0; ks < BK / 32; ++ks) {
                 const uint8_t *sa = st + wm * (TM * 16) * RowB + frd[ks];
-                const uint8_t *sb = st + Sh::ATile + wn * (TN * 16) * RowB + frd[ks];
+                const uint8_t *sb = st + Sh::BOff + wn * (TN * 16) * RowB + frd[ks];
                 v8bf bo[TN], ao[TM], al[kLo ? TM : 1];
 #pragma unroll
                 for (int j = 0; j < TN; ++j) bo[j] = *(const v8bf *)(sb + j * 16 * RowB);
+                if constexpr (Sh::AF32) {
 #pragma unroll
-                for (int i = 0; i < TM; ++i) ao[i] = *(const v8bf *)(sa + i * 16 * RowB);
-                if constexpr (kLo) {
+                    for (int i = 0; i < TM; ++i) {
+                        const uint8_t *sf = st + (wm * TM * 16 + 16 * i + n) * 2 * RowB;
+                        const v4f x0 = *(const v4f *)(sf + 16 * ((8 * ks + 2 * g) ^ (n & 7)));
+                        const v4f x1 = *(const v4f *)(sf + 16 * ((8 * ks + 2 * g + 1) ^ (n & 7)));
+                        split8_cvt(x0, x1, ao[i], al[kLo ? i : 0]);
+                    }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) ao[i] = *(const v8bf *)(sa + i * 16 * RowB);
+                }
+                if constexpr (kLo && !Sh::AF32) {
 #pragma unroll
                     for (int i = 0; i < TM; ++i)
-                        al[i] = *(const v8bf *)(sa + Sh::ATile + Sh::BTile + i * 16 * RowB);
+                        al[i] = *(const v8bf *)(sa + Sh::ALo + i * 16 * RowB);
                 }
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
@@ -314,7 +339,7 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
             }
         }
     };
-    if (use_lo) compute(std::integral_constant<bool, Sh::LO>{});
+    if (Sh::AF32 || use_lo) compute(std::integral_constant<bool, Sh::LO>{});
     else compute(std::false_type{});
     // Epilogue. D layout: lane (g, n) of tile (i, j) holds rows 4g + r, column n. Row-major
     // outputs go through a per-wave LDS buffer (16 rows x 64 columns per tile row i): lane l
@@ -441,13 +466,22 @@ static int gemm_part_ks(int M, int N0, int N1, int K) {
     return K % (64 * ks) == 0 && N0 % 4 == 0 && N1 % 4 == 0 ? ks : 1;
 }
 
-static hipError_t gemm_part(hipStream_t st, const uint16_t *Ah, const uint16_t *Al, const int *flag, int lda,
-                            const uint16_t *B0, int N0, const uint16_t *B1, int N1, int ldb, float *C, int M, int K,
-                            int ks) {
-    GemmArgs a{Ah, Al, B0, B1 ? B1 : B0, C, flag, M, N0, N1, K, lda, ldb, N0 + N1, ks, (size_t)M * (N0 + N1)};
+// The q (| kv_a) projection of a short prompt in 64 x 64 tiles: from fp32 x when x is given (16-byte
+// aligned; *clear is then cleared, which k_split does otherwise), else from the planes; ks > 1: the
+// partials of its k ranges into C, else Q and kv_a (ldc = N1) as kEpiQ. Without the k_split launch,
+// 37 tokens FIG_DIRECT.
+static hipError_t gemm_q_small(hipStream_t st, const float *x, int *clear, const uint16_t *Ah, const uint16_t *Al,
+                               const int *flag, const uint16_t *B0, int N0, const uint16_t *B1, int N1, float *C, int M,
+                               int K, int ks, const GemmEpi &e) {
+    GemmArgs a{Ah, Al, B0, B1 ? B1 : B0, C, flag, M, N0, N1, K, K, K, ks > 1 ? N0 + N1 : N1, ks,
+               (size_t)M * (N0 + N1), x, x ? clear : nullptr};
     if (K % (64 * ks)) return hipErrorInvalidValue;
     const int tiles = (M + 63) / 64 * ((N0 + 63) / 64 + (N1 + 63) / 64);
-    return gemm_launch<GemmCfg<64, 64, 64, 4, 2, true>, kEpiPart, false>(st, a, GemmEpi{}, tiles * ks);
+    using P = GemmCfg<64, 64, 64, 4, 2, true>;
+    using F = GemmCfg<64, 64, 64, 4, 2, true, true>;
+    if (ks > 1)
+        return x ? gemm_launch<F, kEpiPart, false>(st, a, e, tiles * ks) : gemm_launch<P, kEpiPart, false>(st, a, e, tiles * ks);
+    return x ? gemm_launch<F, kEpiQ, false>(st, a, e, tiles) : gemm_launch<P, kEpiQ, false>(st, a, e, tiles);
 }
 
 static int gemm_pick(int epi, int M, int N0, int N1, int *tiles) {
@@ -477,7 +511,7 @@ template <int EPI, bool F16 = false>
 static hipError_t gemm(hipStream_t st, const uint16_t *Ah, const uint16_t *Al, const int *flag,
                        int lda, const uint16_t *B0, int N0, const uint16_t *B1, int N1, int ldb,
                        float *C, int ldc, int M, int K, const GemmEpi &e) {
-    GemmArgs a{Ah, Al, B0, B1 ? B1 : B0, C, flag, M, N0, N1, K, lda, ldb, ldc, 1, 0};
+    GemmArgs a{Ah, Al, B0, B1 ? B1 : B0, C, flag, M, N0, N1, K, lda, ldb, ldc, 1, 0, nullptr, nullptr};
     if (K % 64) return hipErrorInvalidValue;
     constexpr bool LO = !F16;  // the fp16 product has no lo operand
     if (!LO && Al) return hipErrorInvalidValue;
@@ -1300,21 +1334,29 @@ hipError_t launch_prefill_all(hipStream_t st, const Dims &d, int S, float eps, c
         // the q GEMM has read it, so no launch clears it first. A value left raised (a call
         // that failed in between, or the buffer reused by another call) only costs the GEMM's lo
         // pass over an exact plane: the flag is never clear while a lo word is non-zero.
-        const int split_blocks = std::min(2048, S);
-        hipLaunchKernelGGL(k_split, dim3(split_blocks), dim3(256), 0, st, x, d.H, xh, xl, d.H, S, d.H, flags + 0);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+        // A short prompt's projections take x as it is (gemm_q_small, launch_kva_tok_f32) and need no planes.
+        int qtiles = 0;
+        const bool small = ks > 1 || gemm_pick(kEpiQ, S, d.QO, qn1, &qtiles) == kTile64x64;
+        const bool direct = small && (uintptr_t)x % 16 == 0 && (!exact || d.H == 2048);
+        if (!direct) {
+            const int split_blocks = std::min(2048, S);
+            hipLaunchKernelGGL(k_split, dim3(split_blocks), dim3(256), 0, st, x, d.H, xh, xl, d.H, S, d.H, flags + 0);
+            if ((e = hipGetLastError()) != hipSuccess) return e;
+        }
         // q (-> Q hi/lo, rotated) | kv_a (-> ykva). When the caller fills a state from this
         // kv_a, it is computed with the decode's k-split arithmetic (launch_kva_tok) so those
         // rows equal the rows a decode appends; otherwise it rides along in the q GEMM.
         // A short prompt splits k (gemm_part_ks) and k_kva_pack adds the partials.
-        if (ks > 1) e = gemm_part(st, xh, xl, flags + 0, d.H, wq, d.QO, exact ? nullptr : wkva, qn1, d.H, ypart, S, d.H, ks);
+        if (small)
+            e = gemm_q_small(st, direct ? x : nullptr, flags + 1, xh, xl, flags + 0, wq, d.QO, exact ? nullptr : wkva, qn1,
+                             ks > 1 ? ypart : ykva, S, d.H, ks, ep);
         else if (exact) e = gemm<kEpiQ>(st, xh, xl, flags + 0, d.H, wq, d.QO, nullptr, 0, d.H, nullptr, 0, S, d.H, ep);
         else e = gemm<kEpiQ>(st, xh, xl, flags + 0, d.H, wq, d.QO, wkva, d.KVO, d.H, ykva, d.KVO, S, d.H, ep);
         if (e != hipSuccess) return e;
         if (exact) {
-            if ((e = launch_kva_tok(st, ykva, (size_t)S * d.KVO, d.KVO, xh, xl, S, wkva, d.KVO, d.H)) !=
-                hipSuccess)
-                return e;
+            e = direct ? launch_kva_tok_f32(st, ykva, (size_t)S * d.KVO, d.KVO, x, S, wkva, d.KVO, d.H)
+                       : launch_kva_tok(st, ykva, (size_t)S * d.KVO, d.KVO, xh, xl, S, wkva, d.KVO, d.H);
+            if (e != hipSuccess) return e;
             if (kva) *kva = PrefillKva{ykva, d.KVO, np, (size_t)S * d.KVO};
         }
         const int vpad = Sp > S ? (d.NH * d.DV + 63) / 64 : 0, ldq = d.QO + qn1;

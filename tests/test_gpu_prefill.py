@@ -233,3 +233,25 @@ def test_prefill_sizes_agree_with_a_longer_prompt(S, bf16_x):
     print(f"[prefill] S={S} against 4096: {e:.3e}", flush=True)
     assert e <= 1e-3, e
     assert np.all(a[S] == 7.0)
+
+
+@pytest.mark.parametrize("S", [5, 37, 64, 100, 128, 129, 250])
+def test_short_prefill_from_an_unaligned_buffer(S):
+    """A short prompt's projections read fp32 x as it is when it is 16-byte aligned and through its bf16
+    planes otherwise: the same words in the same order, so both give the same bits."""
+    cfg = inputs.config(**inputs.KIMI)
+    layer = inputs.make_layer(cfg, 0xCB)
+    w = layer.struct()
+    x = inputs.hidden(cfg, 0xCB, S)
+    dx, do = L.kvl_mla_device_alloc(x.nbytes + 16), L.kvl_mla_device_alloc(x.nbytes)
+    got = []
+    for off in (0, 4):
+        lib.check(L.kvl_mla_copy_to_device(dx + off, x.ctypes.data, x.nbytes), "h2d")
+        lib.check(L.kvl_mla_prefill_device(do, dx + off, S, C.byref(cfg), C.byref(w)), "prefill")
+        a = np.zeros_like(x)
+        lib.check(L.kvl_mla_copy_to_host(a.ctypes.data, do, x.nbytes), "d2h")
+        got.append(a)
+    assert np.all(np.isfinite(got[0])) and np.any(got[0])
+    np.testing.assert_array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    L.kvl_mla_device_free(dx)
+    L.kvl_mla_device_free(do)
