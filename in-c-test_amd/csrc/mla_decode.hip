@@ -2124,7 +2124,8 @@ __device__ __forceinline__ void fq_wait_all(const FqArgs &f, const unsigned *fla
 // threads l, l + 64, l + 128, l + 192, their tree, then the lanes), and every lane scales its own
 // columns, so the operand equals that kernel's output bit for bit. Every workgroup reads all of x (64
 // KB, from its XCD's L2) beside its 64 KB of weights. Decode stack (27 layers, 8 x 32K rows): the
-// launch grows by 2 us and the norm's launch goes, 1539 -> 1513 us. inv: 8 floats of LDS.
+// launch grows by 2 us and the norm's launch goes, 1539 -> 1513 us. Only in the kCombXcd form: the
+// branch alone cost the lone decode 0.2 us of 29.3. inv: 8 floats of LDS.
 __device__ __forceinline__ void fq_norm_x(const FqArgs &f, int B, int kq, v4f (&xa)[2], v4f (&xb)[2], float *inv) {
     const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, n = l & 15, g = l >> 4;
     const float *xr = f.x + (size_t)min(w, B - 1) * f.ldx;
@@ -2172,6 +2173,7 @@ __device__ __forceinline__ void fq_norm_x(const FqArgs &f, int B, int kq, v4f (&
 // Called by both roles before any history request: its loads are then first in the CU's queue
 // and its waits cover nothing else. (Measured on the headline step: with the task on the score
 // waves only and the mix waves' history requests issued beside it, 1.404 ms against 1.378 ms.)
+template <bool NORM>
 __device__ __forceinline__ void fq_gemv(const FqArgs &f, int B, uint8_t *lds) {
     const int i = blockIdx.x;
     const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, n = l & 15, g = l >> 4;
@@ -2196,7 +2198,7 @@ __device__ __forceinline__ void fq_gemv(const FqArgs &f, int B, uint8_t *lds) {
         xa[j] = *(const v4f *)(xr + kbase);
         xb[j] = *(const v4f *)(xr + kbase + 4);
     }
-    if (f.xnorm) fq_norm_x(f, B, kq, xa, xb, (float *)lds);
+    if (NORM && f.xnorm) fq_norm_x(f, B, kq, xa, xb, (float *)lds);
     v4f acc[2][4];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -2521,7 +2523,7 @@ __device__ __forceinline__ void q8_score_role(const AttnArgs &a, const AttnHot &
         // query copy after Q), its producer task, then (one poller, barrier Q) the 16 query heads
         // of its sequence and, where the split holds the new row (whose scale the loads below
         // read and whose chunk the mix waves request after Q), that row
-        fq_gemv(a.fq, h.nseq, smem + 3 * kQ8CodeB);
+        fq_gemv<COMB == kCombXcd>(a.fq, h.nseq, smem + 3 * kQ8CodeB);
         fq_produce(a, h, smem + kQ8WqOff);
         if (w == 0) {
             fq_wait(a.fq, fq_qflag(a.fq, b), 16u);
@@ -2804,7 +2806,7 @@ __device__ __forceinline__ void q8_mix_role(const AttnArgs &a, const AttnHot &h,
         };
         const bool prod = (int)blockIdx.x < 17 * h.nseq;
         // a projection task goes before the history requests (fq_gemv)
-        fq_gemv(a.fq, h.nseq, smem + 3 * kQ8CodeB);
+        fq_gemv<COMB == kCombXcd>(a.fq, h.nseq, smem + 3 * kQ8CodeB);
         if (!prod) issue_ahead();
         fq_produce(a, h, smem + kQ8WqOff);
         if (prod) issue_ahead();
@@ -3131,7 +3133,7 @@ __global__ __launch_bounds__(512) void k_attn_q8_mfma(KVL_ATTN_HOT_PARAMS, AttnA
     // comes in the members argument (-splits; a fused launch is never a block launch), which is
     // preloaded: the argument block's copy would cost every workgroup a memory round trip first.
     if (FUSE && (int)blockIdx.x >= -h.members) {
-        fq_gemv(a.fq, h.nseq, smem);
+        fq_gemv<COMB == kCombXcd>(a.fq, h.nseq, smem);
         return;
     }
     int b, split, pidx;

@@ -190,8 +190,8 @@ struct FqArgs {
     // (16-byte aligned rows, ldx) and the weights wq [out0, in], wkva [out1, in]; needs B <= 8
     // and in = 2048 (gemv_fuse_ok), and runs max(splits, kGemvTasks) workgroups. Flags words
     // kFqFlagStride * (3 kMaxBatch + i), i < kFqGemvFlags: per-head and kv_a task counts.
-    // xnorm (may be null): the projection's input is RMSNorm(x) with these bf16 weights (k_rmsnorm's
-    // arithmetic, eps as below).
+    // xnorm (may be null; comb = 1 only): the projection's input is RMSNorm(x) with these bf16 weights
+    // (k_rmsnorm's arithmetic, eps as below).
     int gemv;
     const float *x;
     const uint16_t *xnorm;

@@ -166,6 +166,7 @@ struct Ctx {
     DevBuf work, part, scores, prefill, fill, fillx, layer, sink;
     DevBuf rflag;  // int: raised by a stream-ordered prefill outside the MFMA route's range
     PinBuf pin_in, pin_out;
+    hipEvent_t stage_ev[2] = {nullptr, nullptr};  // host-buffer prefills: marks in their copies out
     // fused Q8 decode (the attention launch prepares the queries and appends the rows, and where
     // the shapes allow also computes the q_proj | kv_a projection and combines the splits): its
     // readiness flags and counters (device, kFqFlagLines lines; cleared by the o_proj launch
@@ -1027,7 +1028,8 @@ int decode_group(int fmt, const Dims &d, float eps, float theta, const DevWeight
     const bool fuse = fuse_base && (B >= 2 || (pfuse_ok && comb_mode != 0));
     const bool pfuse = fuse && pfuse_ok;
     const int comb = fuse ? comb_mode : 0;
-    if (in_norm && !pfuse) {  // else the projection tasks normalise x themselves (FqArgs::xnorm)
+    const bool norm_inside = in_norm && pfuse && comb == 1;  // the projection tasks normalise x (FqArgs::xnorm)
+    if (in_norm && !norm_inside) {
         HIP_TRY(launch_rmsnorm(st, in_norm->buf, d_x, in_norm->w, d.H, B, eps));
         d_x = in_norm->buf;
     }
@@ -1102,7 +1104,7 @@ int decode_group(int fmt, const Dims &d, float eps, float theta, const DevWeight
             if (pfuse) {
                 fq.gemv = 1;
                 fq.x = d_x;
-                fq.xnorm = in_norm ? in_norm->w : nullptr;
+                fq.xnorm = norm_inside ? in_norm->w : nullptr;
                 fq.wq = dw.q;
                 fq.wkva = dw.kva;
                 fq.ldx = d.H;
@@ -1734,6 +1736,73 @@ int prefill_state_device(float *d_out, const float *d_x, int seq_len, const KvlM
     return 0;
 }
 
+// Host-buffer prefills up to this many bytes of x go through the library's pinned buffers: the copies
+// to and from them are asynchronous, so the host copies one part while the device works on another,
+// and one wait ends the call (a pageable copy waits by itself, and so did the flag and the rows).
+// 250 tokens with FP32 state fill 337 -> 295 us. Longer prompts keep the pageable copies.
+constexpr size_t kPinStage = (size_t)8 << 20;
+
+// x [bytes] to dx on the stream, in two parts through pin_in when staged.
+int stage_in(float *dx, const float *x, size_t bytes, bool staged) {
+    Ctx &c = ctx();
+    if (!staged) {
+        HIP_TRY(hipMemcpyAsync(dx, x, bytes, hipMemcpyHostToDevice, c.stream));
+        return 0;
+    }
+    if (pin_reserve(c.pin_in, bytes) != 0) return -1;
+    const size_t half = (bytes / 2 + 4095) & ~(size_t)4095;
+    for (size_t o = 0; o < bytes; o += half) {
+        const size_t n = std::min(half, bytes - o);
+        memcpy((char *)c.pin_in.p + o, (const char *)x + o, n);
+        HIP_TRY(hipMemcpyAsync((char *)dx + o, (const char *)c.pin_in.p + o, n, hipMemcpyHostToDevice, c.stream));
+    }
+    return 0;
+}
+
+// The end of a staged host-buffer prefill (see kPinStage): rows (rows_bytes of c.fill, 0: none), the
+// call's range flag and the output come through pin_out; put_rows writes the rows to the host arrays
+// while the output is on its way. The output is computed again when the flag is up.
+template <class F>
+int stage_out(float *out, float *dout, const float *dx, size_t bytes, size_t rows_bytes, int seq_len,
+              const KvlMlaConfig *cfg, const KvlMlaBF16 *w, F put_rows) {
+    Ctx &c = ctx();
+    Dims d;
+    const bool flagged = dims_of(cfg, d) && prefill_mfma_shape(d);
+    for (hipEvent_t &e : c.stage_ev)
+        if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    const size_t ro = (bytes + 255) & ~(size_t)255, fo = ro + ((rows_bytes + 255) & ~(size_t)255);
+    if (pin_reserve(c.pin_out, fo + 256) != 0) return -1;
+    char *pin = (char *)c.pin_out.p;
+    int *flag = (int *)(pin + fo);
+    *flag = 0;
+    if (rows_bytes) {
+        HIP_TRY(hipMemcpyAsync(pin + ro, c.fill.p, rows_bytes, hipMemcpyDeviceToHost, c.stream));
+        HIP_TRY(hipEventRecord(c.stage_ev[0], c.stream));
+    }
+    if (flagged)
+        HIP_TRY(hipMemcpyAsync(flag, prefill_range_flag(c.scores.p), sizeof(int), hipMemcpyDeviceToHost, c.stream));
+    const size_t half = (bytes / 2 + 4095) & ~(size_t)4095, first = std::min(half, bytes);
+    HIP_TRY(hipMemcpyAsync(pin, dout, first, hipMemcpyDeviceToHost, c.stream));
+    HIP_TRY(hipEventRecord(c.stage_ev[1], c.stream));
+    if (first < bytes)
+        HIP_TRY(hipMemcpyAsync(pin + first, (char *)dout + first, bytes - first, hipMemcpyDeviceToHost, c.stream));
+    if (rows_bytes) {
+        HIP_TRY(hipEventSynchronize(c.stage_ev[0]));
+        put_rows((const uint8_t *)pin + ro);
+    }
+    HIP_TRY(hipEventSynchronize(c.stage_ev[1]));
+    if (!*flag) memcpy(out, pin, first);
+    HIP_TRY(hipStreamSynchronize(c.stream));
+    if (!*flag) {
+        memcpy((char *)out + first, pin + first, bytes - first);
+        return 0;
+    }
+    if (prefill_device(dout, dx, seq_len, cfg, w, nullptr, true, true) != 0) return -1;
+    HIP_TRY(hipMemcpyAsync(out, dout, bytes, hipMemcpyDeviceToHost, c.stream));
+    HIP_TRY(hipStreamSynchronize(c.stream));
+    return 0;
+}
+
 template <class S>
 int prefill_state(float *out, const float *x, int seq_len, const KvlMlaConfig *cfg, const KvlMlaBF16 *w,
                   S *s) {
@@ -1748,8 +1817,23 @@ int prefill_state(float *out, const float *x, int seq_len, const KvlMlaConfig *c
     if (dev_reserve(c.prefill, 2 * io_al) != 0) return -1;
     float *dx = (float *)c.prefill.p;
     float *dout = (float *)((char *)c.prefill.p + io_al);
-    HIP_TRY(hipMemcpyAsync(dx, x, io, hipMemcpyHostToDevice, c.stream));
-    if (prefill_state_device(dout, dx, seq_len, cfg, w, s, true, true) != 0) return -1;
+    // one fill_rows call leaves all rows in c.fill (it takes at most 4096 tokens at a time)
+    const bool staged = io <= kPinStage && seq_len <= 4096 && !c.capturing;
+    if (stage_in(dx, x, io, staged) != 0) return -1;
+    if (prefill_state_device(dout, dx, seq_len, cfg, w, s, !staged, true) != 0) return -1;
+    if (staged) {
+        const int fmt = fmt_of<S>();
+        const size_t rb = row_bytes_of(fmt, cfg->kv_lora_rank, cfg->qk_rope_dim, 0);
+        const HostView v = view_of(s);
+        const int rc = stage_out(out, dout, dx, io, (size_t)seq_len * rb, seq_len, cfg, w, [&](const uint8_t *rows) {
+            for (int i = 0; i < seq_len; ++i) write_back_rows(fmt, v, i, rows + (size_t)i * rb);
+        });
+        if (rc != 0) {  // the host rows may be incomplete
+            s->len = 0;
+            mirror_lower(s, 0);
+        }
+        return rc;
+    }
     HIP_TRY(hipStreamSynchronize(c.stream));
     // the state rows do not depend on the attention; only the output is computed again
     if (prefill_range_fallback(dout, dx, seq_len, cfg, w) != 0) return -1;
@@ -1853,8 +1937,10 @@ int kvl_mla_prefill_bf16(float *out, const float *x, int seq_len, const KvlMlaCo
     if (dev_reserve(c.prefill, 2 * io + 512) != 0) return -1;
     float *dx = (float *)c.prefill.p;
     float *dout = (float *)((char *)c.prefill.p + ((io + 255) & ~(size_t)255));
-    HIP_TRY(hipMemcpyAsync(dx, x, io, hipMemcpyHostToDevice, c.stream));
+    const bool staged = io <= kPinStage && !c.capturing;
+    if (stage_in(dx, x, io, staged) != 0) return -1;
     if (prefill_device(dout, dx, seq_len, cfg, w, nullptr, true) != 0) return -1;
+    if (staged) return stage_out(out, dout, dx, io, 0, seq_len, cfg, w, [](const uint8_t *) {});
     HIP_TRY(hipStreamSynchronize(c.stream));
     if (prefill_range_fallback(dout, dx, seq_len, cfg, w) != 0) return -1;
     HIP_TRY(hipMemcpyAsync(out, dout, io, hipMemcpyDeviceToHost, c.stream));
