@@ -758,8 +758,8 @@ __global__ __launch_bounds__(256) void k_kva_pack(KvaPackArgs a) {
 
 // ================================================================ flash attention ======
 
-// Causal attention for one head and 128 queries: 8 waves, wave w taking queries 32 (w % 4) .. + 31
-// (two 16-query tiles u = 0, 1) and half w / 4 of every 64-key tile. QD = 192, DV = 128. Operands
+// Causal attention for one head and 64 U queries: 8 waves, wave w taking queries 16 U (w % 4) ..
+// (U 16-query tiles) and half w / 4 of every 64-key tile. QD = 192, DV = 128. Operands
 // are fp16 (11 significant bits, ample range for these values): Q and K as hi + lo pairs, V and P
 // rounded once.
 //
@@ -798,10 +798,11 @@ __global__ __launch_bounds__(256) void k_kva_pack(KvaPackArgs a) {
 //   11.0 / 36.5 / 139 / 1700  one loop for both, K fragments read two groups ahead (two copies of
 //                             the loop left the compiler too few registers for that)
 //   10.3 / 36.0 / 139 / 1687  V fragments read before the weights, one copy of the merge
-constexpr int kFQ = 128, kFK = 64;
+constexpr int kFK = 64;
 constexpr int kFKB = kFK * 192 * 2;  // K tile (hi or lo): 64 rows x 384 B
 constexpr int kFVB = 128 * kFK * 2;  // V^T tile: 128 rows x 128 B
 constexpr int kFSmem = 2 * 2 * kFKB + 3 * kFVB;
+constexpr int kFlashSmall = 256;     // blocks of 128 queries up to which blocks of 64 are taken
 constexpr float kFLazy = 8.0f;       // log2 headroom of the lazy max
 constexpr float kFNone = -1e30f;     // running max of a key half that has seen no key yet (finite:
                                      // differences of it and of itself stay numbers)
@@ -842,6 +843,7 @@ __device__ __forceinline__ float xrow_sum(float v) {
     return __uint_as_float(q[0]) + __uint_as_float(q[1]);
 }
 
+template <int U>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_flash_prefill(FlashArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t smem[kFSmem];
@@ -851,7 +853,8 @@ void k_flash_prefill(FlashArgs a) {
     // kernel arguments as locals (the lambdas below must not capture the argument block)
     const int S = a.S, Sp = a.Sp, NH = a.NH, ldo = a.ldo;
     const float sl2 = a.sl2;
-    const int nqt = Sp / kFQ;
+    constexpr int FQ = 64 * U;  // queries of a block
+    const int nqt = (S + FQ - 1) / FQ;
     // Longest tiles first; with NH % 8 == 0, block b runs on XCD b % 8 and each XCD keeps
     // the same NH / 8 heads, so the blocks streaming one head's K/V share an L2.
     int qt, h;
@@ -863,8 +866,8 @@ void k_flash_prefill(FlashArgs a) {
         qt = nqt - 1 - (int)blockIdx.x / NH;
         h = (int)blockIdx.x % NH;
     }
-    const int nt = 2 * qt + 2;  // key tiles 0 .. nt-1 (the last two straddle the diagonal)
-    const int qw = qt * kFQ + 32 * (w & 3);
+    const int nt = U * (qt + 1);  // key tiles 0 .. nt-1 (the last U straddle the diagonal)
+    const int qw = qt * FQ + 16 * U * (w & 3);
     const size_t hq = (size_t)h * Sp;
 
     // DMA sources. K tile: wave w fills LDS slots (3w + i) * 64 + l (16 B each) of the
@@ -901,13 +904,15 @@ void k_flash_prefill(FlashArgs a) {
 
     // Query tile u of a wave of the second half is tile 1 - u of the first: the merge below is then
     // the same code for both (the kernel's first pass through its code is instruction fetch).
-    const int qu[2] = {qw + 16 * half + n, qw + 16 * (1 - half) + n};  // this lane's query of tile u
+    int qu[U];  // this lane's query of tile u
+#pragma unroll
+    for (int u = 0; u < U; ++u) qu[u] = qw + 16 * (U == 2 ? u ^ half : 0) + n;
     // Q^T B operands: query qu[u], dims 32kb + 8g .. +7: hi as fp16 (main pass), lo as
     // its bf8(lo x 2^11) bytes (the correction operand below, written so by the q GEMM)
-    v8h qa[2][6];
-    uint2 qb[2][6];
+    v8h qa[U][6];
+    uint2 qb[U][6];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < U; ++u) {
         const _Float16 *ph = a.qh + (hq + qu[u]) * 192 + 8 * g;
         const uint8_t *pl = a.ql8 + (hq + qu[u]) * 192 + 8 * g;
 #pragma unroll
@@ -929,9 +934,9 @@ void k_flash_prefill(FlashArgs a) {
     // correction operands: per u, 96 bytes = bf8(Ql 2^11) then bf8(Qh), each in (k-block,
     // element) order, so that byte p meets byte p of the lane group's K8 bytes (hi, then lo);
     // MFMA m takes bytes 32m .. 32m+31
-    v8i q8[2][3];
+    v8i q8[U][3];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < U; ++u) {
         uint32_t wd[24];
 #pragma unroll
         for (int kb = 0; kb < 6; ++kb)
@@ -951,20 +956,25 @@ void k_flash_prefill(FlashArgs a) {
     // a use of every operand here, so that the compiler's wait for their loads stands before the
     // loop: inside it, it would wait for the tile in flight as well, in every step
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < U; ++u) {
 #pragma unroll
         for (int kb = 0; kb < 6; ++kb) asm volatile("" : "+v"(qa[u][kb]));
 #pragma unroll
         for (int m = 0; m < 3; ++m) asm volatile("" : "+v"(q8[u][m]));
     }
 
-    float m_run[2] = {kFNone, kFNone}, l_run[2] = {0.f, 0.f};
-    v4f acc[8][2];
+    float m_run[U], l_run[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        m_run[u] = kFNone;
+        l_run[u] = 0.f;
+    }
+    v4f acc[8][U];
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
-        for (int u = 0; u < 2; ++u) acc[dt][u] = v4f{0.f, 0.f, 0.f, 0.f};
-    v4f sc[2][2];
+        for (int u = 0; u < U; ++u) acc[dt][u] = v4f{0.f, 0.f, 0.f, 0.f};
+    v4f sc[2][U];
 
     // Scores of tile j (K slot j & 1): each accumulator receives its products in the order Kh Qh
     // for kb = 0 .. 5, then the corrections m = 0 .. 2. Six groups of four independent MFMAs and six
@@ -985,7 +995,7 @@ void k_flash_prefill(FlashArgs a) {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int u = 0; u < 2; ++u) sc[t][u] = v4f{0.f, 0.f, 0.f, 0.f};
+            for (int u = 0; u < U; ++u) sc[t][u] = v4f{0.f, 0.f, 0.f, 0.f};
         load_kh(0);
         load_kh(1);
 #pragma unroll
@@ -994,7 +1004,7 @@ void k_flash_prefill(FlashArgs a) {
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int u = 0; u < 2; ++u) sc[t][u] = mfma_f16(kf[kb & 1][t], qa[u][kb], sc[t][u]);
+                for (int u = 0; u < U; ++u) sc[t][u] = mfma_f16(kf[kb & 1][t], qa[u][kb], sc[t][u]);
             if (kb + 2 < 6) load_kh(kb + 2);
             else load_k8(kb - 4);
         }
@@ -1002,7 +1012,7 @@ void k_flash_prefill(FlashArgs a) {
         for (int c = 0; c < 6; ++c) {
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int u = 0; u < 2; ++u) sc[c & 1][u] = mfma_bf8_s11(k8[c & 1], q8[u][c >> 1], sc[c & 1][u]);
+            for (int u = 0; u < U; ++u) sc[c & 1][u] = mfma_bf8_s11(k8[c & 1], q8[u][c >> 1], sc[c & 1][u]);
             if (c + 2 < 6) load_k8(c + 2);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -1015,21 +1025,24 @@ void k_flash_prefill(FlashArgs a) {
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int u = 0; u < 2; ++u)
+                for (int u = 0; u < U; ++u)
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
                         if (k0 + 16 * t + 4 * g + i > qu[u]) sc[t][u][i] = -INFINITY;
         }
         // The running max moves only when a score of the tile exceeds it by more than kFLazy, which
         // each lane can tell from its own scores; the max over a query's four lanes is taken then.
-        float mx[2];
+        float mx[U];
+        bool over = false;
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < U; ++u)
             mx[u] = max3(max3(max3(sc[0][u][0], sc[0][u][1], sc[0][u][2]), sc[0][u][3], sc[1][u][0]),
                          max3(sc[1][u][1], sc[1][u][2], sc[1][u][3]), sc[1][u][3]) * sl2;
-        if (__any((mx[0] > m_run[0] + kFLazy) | (mx[1] > m_run[1] + kFLazy))) {
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
+        for (int u = 0; u < U; ++u) over |= mx[u] > m_run[u] + kFLazy;
+        if (__any(over)) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
                 const float m = xrow_max(mx[u]);
                 const float mnew = m > m_run[u] + kFLazy ? m : m_run[u];
                 const float alpha = __builtin_amdgcn_exp2f(m_run[u] - mnew);
@@ -1043,9 +1056,9 @@ void k_flash_prefill(FlashArgs a) {
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt) vv0[dt] = *(const v8h *)(vt + dt * 16 * 128);
         __builtin_amdgcn_sched_barrier(0);
-        v8h pb[2];
+        v8h pb[U];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int u = 0; u < U; ++u) {
             float ps = 0.f;
 #pragma unroll
             for (int t = 0; t < 2; ++t)
@@ -1060,13 +1073,13 @@ void k_flash_prefill(FlashArgs a) {
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) {
 #pragma unroll
-            for (int u = 0; u < 2; ++u) acc[dt][u] = mfma_f16(vv0[dt & 3], pb[u], acc[dt][u]);
+            for (int u = 0; u < U; ++u) acc[dt][u] = mfma_f16(vv0[dt & 3], pb[u], acc[dt][u]);
             if (dt < 4) vv0[dt] = *(const v8h *)(vt + (dt + 4) * 16 * 128);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
     // a tile whose first key of this half comes after this wave's last query adds nothing
-    auto live = [&](int j) __attribute__((always_inline)) { return j * kFK + 32 * half <= qw + 31; };
+    auto live = [&](int j) __attribute__((always_inline)) { return j * kFK + 32 * half <= qw + 16 * U - 1; };
 
     // Both halves run one loop, QK(j) then softmax and PV of tile j; the second passes the barrier of
     // step j + 1 between the two, the first before QK(j). Passing the barrier of step j: tile j is in
@@ -1091,15 +1104,18 @@ void k_flash_prefill(FlashArgs a) {
         vs = v1;
     }
 
-    // Merge of the two key halves: wave w gives its query tile 1 to wave w ^ 4, whose tile 0 that is,
-    // and finishes its own tile 0.
+    // Merge of the two key halves. U = 2: wave w gives its query tile 1 to wave w ^ 4, whose tile 0
+    // that is, and finishes its own tile 0. U = 1: the second half gives, the first finishes.
     lds_barrier();  // the ring is free
     float *xw = (float *)(smem + w * 9216), *xr = (float *)(smem + (w ^ 4) * 9216);
+    if (U == 2 || half) {
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) *(v4f *)(xw + 256 * dt + 4 * l) = acc[dt][1];
-    xw[2048 + l] = m_run[1];
-    xw[2112 + l] = l_run[1];
+        for (int dt = 0; dt < 8; ++dt) *(v4f *)(xw + 256 * dt + 4 * l) = acc[dt][U - 1];
+        xw[2048 + l] = m_run[U - 1];
+        xw[2112 + l] = l_run[U - 1];
+    }
     lds_barrier();
+    if (U == 1 && half) return;
     // range check of each query row: the reference max (log2 units, within kFLazy of the row's
     // true max) and every output value (NaN or Inf from operands beyond the fp16 range: an
     // exponent field of ones, which the addition carries into the sign bit)
@@ -1375,7 +1391,13 @@ hipError_t launch_prefill_all(hipStream_t st, const Dims &d, int S, float eps, c
             return e;
         FlashArgs fa{qh, kh, ql8, k8, vt, heads, flags + 1, range ? range->sticky : nullptr, S, Sp, d.NH, d.HO,
                      smscale * 1.4426950408889634f};
-        hipLaunchKernelGGL(k_flash_prefill, dim3(Sp / kFQ * d.NH), dim3(512), 0, st, fa);
+        // 64 queries per block while 128 would leave CUs without one: a launch then lasts as long as
+        // its last query tile's key tiles, which U = 1 takes in less time each. 64 / 128 queries, alone
+        // (us): 6.2 / 10.2 at 37 tokens, 9.2 / 14.0 at 250, 24.2 / 34.8 at 1181, 47.6 / 53.2 at 2048,
+        // 81.2 / 64.0 at 2500 (320 blocks of 128).
+        const int nq2 = (S + 127) / 128 * d.NH;
+        if (nq2 <= kFlashSmall) hipLaunchKernelGGL(k_flash_prefill<1>, dim3((S + 63) / 64 * d.NH), dim3(512), 0, st, fa);
+        else hipLaunchKernelGGL(k_flash_prefill<2>, dim3(nq2), dim3(512), 0, st, fa);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         // out = heads . o_proj^T in fp16 (heads rounded once, o_proj converted exactly), the
         // two scales undone (or NaN when the range flag of this call is up)
