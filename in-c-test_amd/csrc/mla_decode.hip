@@ -352,7 +352,6 @@ struct KvaTokArgs {
     const uint16_t *W;         // [out, in]
     size_t pstride;
     int ldy, S, out, in;
-    const float *X;            // k_kva_gemm<., true>: fp32 [S, in] in place of the planes
 };
 
 template <int KPW>
@@ -443,15 +442,14 @@ __global__ __launch_bounds__(256) void k_kva_tok(KvaTokArgs a) {
 // and one for the lo half, added to the running sums in k order (the sums of k_gemv_ksplit's
 // waves 0..15). Tiles are numbered row block fastest, then quarter, then token block, and XCD
 // b % 8 takes a contiguous eighth of them, so the row blocks sharing a token block's
-// activations run under one L2. F32X: x comes as fp32 (128-byte rows, slot s at s ^ (r & 7)) and each
-// wave splits its fragments itself (split8_cvt: k_split's words for finite values).
+// activations run under one L2.
 template <int TU_, int TT_, int WT_, int WR_, int NS_>
 struct KvgShape {
     static constexpr int TU = TU_, TT = TT_, WT = WT_, WR = WR_, NS = NS_;  // NS: ring stages
     static constexpr int BT = 16 * TU * WT, BR = 16 * TT * WR, NT = 64 * WT * WR;
 };
 
-template <class Sh, bool F32X = false>
+template <class Sh>
 __global__ __launch_bounds__(Sh::NT) void k_kva_gemm(KvaTokArgs a) {
     constexpr int TU = Sh::TU, TT = Sh::TT, NS = Sh::NS;
     constexpr int NWV = Sh::WT * Sh::WR, NT = Sh::NT, BT = Sh::BT, BR = Sh::BR;
@@ -477,11 +475,6 @@ __global__ __launch_bounds__(Sh::NT) void k_kva_gemm(KvaTokArgs a) {
         const int xrow = (p % (BT * 4)) / 4, wrow = (p - 2 * BT * 4) / 4;
         const uint16_t *rp;
         int s;
-        if (F32X && p < 2 * BT * 4) {
-            const int r = p / 8;
-            src[i] = (const uint8_t *)(a.X + (size_t)min(tok0 + r, a.S - 1) * a.in + kq * 512 + 4 * ((p & 7) ^ (r & 7)));
-            continue;
-        }
         if (p < 2 * BT * 4) {
             rp = (p < BT * 4 ? a.XH : a.XL) + (size_t)min(tok0 + xrow, a.S - 1) * a.in;
             s = (p & 3) ^ swz(xrow);
@@ -495,14 +488,13 @@ __global__ __launch_bounds__(Sh::NT) void k_kva_gemm(KvaTokArgs a) {
         const uint32_t dst = sbase + (j % NS) * STAGE + (uint32_t)w * 1024;
 #pragma unroll
         for (int i = 0; i < NI; ++i)
-            if (i < NMIN || (i * NWV + w) * 64 < SLOTS)
-                dma_b128(src[i] + (size_t)j * (F32X && (i * NWV + w) * 64 < 2 * BT * 4 ? 128 : 64), dst + i * (NWV * 1024));
+            if (i < NMIN || (i * NWV + w) * 64 < SLOTS) dma_b128(src[i] + (size_t)j * 64, dst + i * (NWV * 1024));
     };
     int fx[TU], fw[TT];  // fragment offsets: row 16 u + n of the wave's tile, logical slot g
 #pragma unroll
     for (int u = 0; u < TU; ++u) {
         const int row = 16 * (TU * wt + u) + n;
-        fx[u] = F32X ? row * 128 : row * ROWB + 16 * (g ^ swz(row));
+        fx[u] = row * ROWB + 16 * (g ^ swz(row));
     }
 #pragma unroll
     for (int t = 0; t < TT; ++t) {
@@ -523,14 +515,8 @@ __global__ __launch_bounds__(Sh::NT) void k_kva_gemm(KvaTokArgs a) {
         v8bf xh[TU], xl[TU], wv[TT];
 #pragma unroll
         for (int u = 0; u < TU; ++u) {
-            if constexpr (F32X) {
-                const v4f x0 = *(const v4f *)(st + fx[u] + 16 * ((2 * g) ^ (n & 7)));
-                const v4f x1 = *(const v4f *)(st + fx[u] + 16 * ((2 * g + 1) ^ (n & 7)));
-                split8_cvt(x0, x1, xh[u], xl[u]);
-            } else {
-                xh[u] = *(const v8bf *)(st + fx[u]);
-                xl[u] = *(const v8bf *)(st + XPL + fx[u]);
-            }
+            xh[u] = *(const v8bf *)(st + fx[u]);
+            xl[u] = *(const v8bf *)(st + XPL + fx[u]);
         }
 #pragma unroll
         for (int t = 0; t < TT; ++t) wv[t] = *(const v8bf *)(st + fw[t]);
@@ -570,11 +556,11 @@ __global__ __launch_bounds__(Sh::NT) void k_kva_gemm(KvaTokArgs a) {
     }
 }
 
-template <class Sh, bool F32X = false>
+template <class Sh>
 static hipError_t kva_gemm_launch(hipStream_t st, const KvaTokArgs &a) {
     const size_t tiles = (size_t)((a.out + Sh::BR - 1) / Sh::BR) * kGemvKs * ((a.S + Sh::BT - 1) / Sh::BT);
     if (tiles > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_kva_gemm<Sh, F32X>), dim3((unsigned)tiles), dim3(Sh::NT), 0, st, a);
+    hipLaunchKernelGGL((k_kva_gemm<Sh>), dim3((unsigned)tiles), dim3(Sh::NT), 0, st, a);
     return hipGetLastError();
 }
 
@@ -584,30 +570,27 @@ hipError_t launch_kva_tok(hipStream_t st, float *Y, size_t pstride, int ldy, con
         ((uintptr_t)XH % 16) != 0 || ((uintptr_t)XL % 16) != 0 || ((uintptr_t)W % 16) != 0 ||
         ((uintptr_t)Y % 16) != 0 || pstride % 4 != 0)
         return hipErrorInvalidValue;
-    KvaTokArgs a{Y, XH, XL, W, pstride, ldy, S, out, in, nullptr};
+    KvaTokArgs a{Y, XH, XL, W, pstride, ldy, S, out, in};
     if (in == 2048) {
-        // Small tiles while they do not outnumber the places for them (two blocks per CU), so that a
-        // short prompt spreads over the CUs; large ones take in fewer bytes per product. 64 x 64, 64 x
-        // 96, 128 x 192 (us): 9.5 / 11.8 / 17.1 at 37 tokens, 10.1 / 12.2 / 19.4 at 250, 12.5 / 13.4 /
-        // 19.8 at 512, 21.5 / 18.2 / 21.4 at 1181, 31.0 / 26.0 / 22.4 at 2048, - / 171 / 127 at 16000.
-        const long places = 512, tb = (S + 63) / 64 * (long)kGemvKs;
-        if (tb * ((out + 63) / 64) <= places) return kva_gemm_launch<KvgShape<2, 2, 2, 2, 6>>(st, a);
-        if (tb * ((out + 95) / 96) <= places) return kva_gemm_launch<KvgShape<2, 3, 2, 2, 4>>(st, a);
+        // Small tiles while they do not outnumber the places for them, so that a short prompt spreads
+        // over the CUs: first with a ring that holds all 16 k steps (one block per CU; a block then waits
+        // for memory about once), then two blocks per CU; large tiles take in fewer bytes per product.
+        // us, 32 x 32 and 32 x 64 (16 stages), 32 x 64 (8), 64 x 64, 64 x 96, 128 x 192 (tokens x rows):
+        //   37 tokens 5.4 / 6.5 / 6.9 / 9.6 / 11.8 / 17.2   200: 10.3 / 7.2 / 7.4 / 9.9 / - / 19.1
+        //   384: 18.5 / 12.5 / 9.2 / 10.3 / - / 19.2        896: 35.7 / 23.9 / 16.5 / 14.3 / - / 20.5
+        //   1181: - / - / - / 21.5 / 18.2 / 21.4            16000: - / - / - / - / 171 / 127
+        auto tiles = [&](int bt, int br) { return (long)((S + bt - 1) / bt) * kGemvKs * ((out + br - 1) / br); };
+        if (tiles(32, 32) <= 256) return kva_gemm_launch<KvgShape<1, 1, 2, 2, 16>>(st, a);
+        if (tiles(32, 64) <= 256) return kva_gemm_launch<KvgShape<1, 2, 2, 2, 16>>(st, a);
+        if (tiles(32, 64) <= 512) return kva_gemm_launch<KvgShape<1, 2, 2, 2, 8>>(st, a);
+        if (tiles(64, 64) <= 512) return kva_gemm_launch<KvgShape<2, 2, 2, 2, 6>>(st, a);
+        if (tiles(64, 96) <= 512) return kva_gemm_launch<KvgShape<2, 3, 2, 2, 4>>(st, a);
         return kva_gemm_launch<KvgShape<4, 4, 2, 3, 3>>(st, a);
     } else {
         const dim3 grid((out + 63) / 64, kGemvKs, (S + 127) / 128);
         hipLaunchKernelGGL((k_kva_tok<2>), grid, dim3(256), 0, st, a);
     }
     return hipGetLastError();
-}
-
-hipError_t launch_kva_tok_f32(hipStream_t st, float *Y, size_t pstride, int ldy, const float *X, int S,
-                              const uint16_t *W, int out, int in) {
-    if (in != 2048 || S < 1 || out <= 0 || ldy < out || ((uintptr_t)X % 16) != 0 || ((uintptr_t)W % 16) != 0 ||
-        ((uintptr_t)Y % 16) != 0 || pstride % 4 != 0)
-        return hipErrorInvalidValue;
-    const KvaTokArgs a{Y, nullptr, nullptr, W, pstride, ldy, S, out, in, X};
-    return kva_gemm_launch<KvgShape<2, 2, 2, 2, 6>, true>(st, a);
 }
 
 bool gemv_xs_ok(int in) { return in == 2048 || in == 4096; }

@@ -98,10 +98,6 @@ hipError_t launch_gemv_ksplit(hipStream_t st, float *Y, size_t pstride, int ldy,
 // prefill's kv_a projection and the state prefill. Shapes as launch_gemv_ksplit.
 hipError_t launch_kva_tok(hipStream_t st, float *Y, size_t pstride, int ldy, const uint16_t *XH,
                           const uint16_t *XL, int S, const uint16_t *W, int out, int in);
-// The same from fp32 x [S, in] (16-byte aligned), in = 2048: for short prompts, which then need no
-// k_split launch.
-hipError_t launch_kva_tok_f32(hipStream_t st, float *Y, size_t pstride, int ldy, const float *X, int S,
-                              const uint16_t *W, int out, int in);
 // Y[b, o] (+)= sum_k W[o, k] x[b, k] with x given as bf16 planes XS[2][B][in] (hi, lo), as
 // launch_combine writes them (DecodeWork::hos). Shapes when gemv_xs_ok (in = 2048 or 4096),
 // any B.

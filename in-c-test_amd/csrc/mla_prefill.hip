@@ -1350,10 +1350,11 @@ hipError_t launch_prefill_all(hipStream_t st, const Dims &d, int S, float eps, c
         // the q GEMM has read it, so no launch clears it first. A value left raised (a call
         // that failed in between, or the buffer reused by another call) only costs the GEMM's lo
         // pass over an exact plane: the flag is never clear while a lo word is non-zero.
-        // A short prompt's projections take x as it is (gemm_q_small, launch_kva_tok_f32) and need no planes.
+        // A short prompt's projection takes x as it is (gemm_q_small) and needs no planes (with a state
+        // fill, launch_kva_tok needs them all the same: reading fp32 x there cost more than the launch).
         int qtiles = 0;
         const bool small = ks > 1 || gemm_pick(kEpiQ, S, d.QO, qn1, &qtiles) == kTile64x64;
-        const bool direct = small && (uintptr_t)x % 16 == 0 && (!exact || d.H == 2048);
+        const bool direct = small && !exact && (uintptr_t)x % 16 == 0;
         if (!direct) {
             const int split_blocks = std::min(2048, S);
             hipLaunchKernelGGL(k_split, dim3(split_blocks), dim3(256), 0, st, x, d.H, xh, xl, d.H, S, d.H, flags + 0);
@@ -1370,9 +1371,9 @@ hipError_t launch_prefill_all(hipStream_t st, const Dims &d, int S, float eps, c
         else e = gemm<kEpiQ>(st, xh, xl, flags + 0, d.H, wq, d.QO, wkva, d.KVO, d.H, ykva, d.KVO, S, d.H, ep);
         if (e != hipSuccess) return e;
         if (exact) {
-            e = direct ? launch_kva_tok_f32(st, ykva, (size_t)S * d.KVO, d.KVO, x, S, wkva, d.KVO, d.H)
-                       : launch_kva_tok(st, ykva, (size_t)S * d.KVO, d.KVO, xh, xl, S, wkva, d.KVO, d.H);
-            if (e != hipSuccess) return e;
+            if ((e = launch_kva_tok(st, ykva, (size_t)S * d.KVO, d.KVO, xh, xl, S, wkva, d.KVO, d.H)) !=
+                hipSuccess)
+                return e;
             if (kva) *kva = PrefillKva{ykva, d.KVO, np, (size_t)S * d.KVO};
         }
         const int vpad = Sp > S ? (d.NH * d.DV + 63) / 64 : 0, ldq = d.QO + qn1;
