@@ -278,6 +278,10 @@ bool prefill_mfma_shape(const Dims &d);
 // even). cols % 8 == 0, 16-byte aligned rows.
 hipError_t launch_split(hipStream_t st, const float *src, int ld_src, uint16_t *hi, uint16_t *lo,
                         int ld_dst, int rows, int cols);
+// *out = max(*out, ...) over the largest |bf16 word| of src [n], or over the L2 norms (fp32 words) of
+// kv_b's V rows; NaN left out.
+hipError_t launch_bf16_absmax(hipStream_t st, const uint16_t *src, size_t n, unsigned *out);
+hipError_t launch_vrow_l2max(hipStream_t st, const uint16_t *kvb, const Dims &d, unsigned *out);
 // dst[i] = (fp16)(bf16 src[i] * scale), scale a power of two: exact while the scaled value is a
 // normal fp16 (bf16 has 8 significant bits).
 hipError_t launch_bf16_to_f16(hipStream_t st, _Float16 *dst, const uint16_t *src, size_t n, float scale);

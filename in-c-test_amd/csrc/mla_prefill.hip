@@ -1245,6 +1245,59 @@ __global__ __launch_bounds__(256) void k_bf16_to_f16(_Float16 *dst, const uint16
         dst[i] = (_Float16)(bf16_to_f32(src[i]) * scale);
 }
 
+// *out = max(*out, largest |src[i]| as its bf16 word), NaN words left out (n % 8 == 0 or not; src
+// 16-byte aligned). The operand ranges of a prefill's weights, once per weight upload: the host took
+// 2.6 ms a layer for them (8 MB of o_proj, 2 MB of kv_b), which was most of a first prefill's 2.9 ms.
+__global__ __launch_bounds__(256) void k_bf16_absmax(const uint16_t *src, size_t n, unsigned *out) {
+    unsigned m = 0;
+    auto take = [&](unsigned v) __attribute__((always_inline)) {
+        v &= 0x7fffu;
+        m = max(m, v <= 0x7f80u ? v : 0u);
+    };
+    const size_t n8 = n / 8;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n8; i += (size_t)gridDim.x * 256) {
+        const v4i x = *(const v4i *)(src + 8 * i);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            take((unsigned)x[k]);
+            take((unsigned)x[k] >> 16);
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x < (n & 7)) take(src[8 * n8 + threadIdx.x]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o));
+    if ((threadIdx.x & 63) == 0) atomicMax(out, m);
+}
+
+// *out = max(*out, largest L2 norm of kv_b's V rows as an fp32 word), NaN left out: one wave per row,
+// double sums.
+__global__ __launch_bounds__(256) void k_vrow_l2max(const uint16_t *kvb, int NH, int DN, int DV, int R, unsigned *out) {
+    const int r = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+    if (r >= NH * DV) return;
+    const uint16_t *row = kvb + ((size_t)(r / DV) * (DN + DV) + DN + r % DV) * R;
+    double ss = 0.0;
+    for (int k = l; k < R; k += 64) {
+        const double v = (double)bf16_to_f32(row[k]);
+        ss += v * v;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+    const float f = (float)sqrt(ss);
+    if (l == 0 && f == f) atomicMax(out, __float_as_uint(f));
+}
+
+hipError_t launch_bf16_absmax(hipStream_t st, const uint16_t *src, size_t n, unsigned *out) {
+    if (((uintptr_t)src % 16) != 0 || n == 0) return hipErrorInvalidValue;
+    const int blocks = (int)std::min<size_t>(1024, (n + 2047) / 2048);
+    hipLaunchKernelGGL(k_bf16_absmax, dim3(blocks), dim3(256), 0, st, src, n, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_vrow_l2max(hipStream_t st, const uint16_t *kvb, const Dims &d, unsigned *out) {
+    hipLaunchKernelGGL(k_vrow_l2max, dim3((d.NH * d.DV + 3) / 4), dim3(256), 0, st, kvb, d.NH, d.DN, d.DV, d.R, out);
+    return hipGetLastError();
+}
+
 hipError_t launch_split(hipStream_t st, const float *src, int ld_src, uint16_t *hi, uint16_t *lo,
                         int ld_dst, int rows, int cols) {
     if (rows < 1 || cols < 8 || cols % 8 || ld_src % 4 || ld_dst % 8 || ld_src < cols || ld_dst < cols ||

@@ -164,6 +164,7 @@ struct Ctx {
     std::unordered_map<const void *, Mirror> mirrors;
     std::unordered_map<uint64_t, RopeTable> ropes;  // key: theta bits << 16 | DR
     DevBuf work, part, scores, prefill, fill, fillx, layer, sink;
+    DevBuf wmax;   // unsigned: result of a weight range reduction
     DevBuf rflag;  // int: raised by a stream-ordered prefill outside the MFMA route's range
     PinBuf pin_in, pin_out;
     hipEvent_t stage_ev[2] = {nullptr, nullptr};  // host-buffer prefills: marks in their copies out
@@ -415,6 +416,18 @@ float bf16_abs(uint16_t b) {
     return f;
 }
 
+// A range reduction over weights on the device (launch_bf16_absmax, launch_vrow_l2max) and its result.
+template <class F>
+int weight_max(F launch, unsigned *res) {
+    Ctx &c = ctx();
+    if (dev_reserve(c.wmax, 256) != 0) return -1;
+    HIP_TRY(hipMemsetAsync(c.wmax.p, 0, sizeof(unsigned), c.stream));
+    HIP_TRY(launch((unsigned *)c.wmax.p));
+    HIP_TRY(hipMemcpyAsync(res, c.wmax.p, sizeof(unsigned), hipMemcpyDeviceToHost, c.stream));
+    HIP_TRY(hipStreamSynchronize(c.stream));
+    return 0;
+}
+
 // fp16 copy of a weight array times 2^shift (converted on the device from its bf16 copy,
 // stream-ordered). shift puts the largest |w| in [2^13, 2^14): far from the fp16 maximum
 // (65504) and with the array's small values above the fp16 subnormals as far as the bf16
@@ -430,8 +443,9 @@ int dev_weight_f16(const uint16_t *host, size_t elems, const _Float16 **out, int
             set_err("fp16 weight conversion during graph capture");
             return -1;
         }
-        float mx = 0.f;
-        for (size_t i = 0; i < elems; ++i) mx = std::max(mx, bf16_abs(host[i]));
+        unsigned mxw = 0;
+        if (weight_max([&](unsigned *r) { return launch_bf16_absmax(c.stream, d16, elems, r); }, &mxw) != 0) return -1;
+        const float mx = bf16_abs((uint16_t)mxw);
         int ex = 0;
         e.f16_shift = 0;
         if (mx > 0.f && std::isfinite(mx)) {
@@ -456,7 +470,11 @@ float prefill_vscale(const KvlMlaBF16 *w, const Dims &d) {
     auto it = c.weights.find(w->kv_b_proj);
     if (it == c.weights.end()) return 1.0f;
     WeightEntry &e = it->second;
-    if (e.row_l2max < 0.f) {
+    unsigned l2w = 0;
+    if (e.row_l2max < 0.f && !c.capturing &&
+        weight_max([&](unsigned *r) { return launch_vrow_l2max(c.stream, (const uint16_t *)e.dev, d, r); }, &l2w) == 0)
+        memcpy(&e.row_l2max, &l2w, sizeof l2w);
+    if (e.row_l2max < 0.f) {  // during a graph capture (nothing can be read back), from the host array
         double mx = 0.0;
         for (int h = 0; h < d.NH; ++h)
             for (int r = 0; r < d.DV; ++r) {

@@ -255,3 +255,23 @@ def test_short_prefill_from_an_unaligned_buffer(S):
     np.testing.assert_array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
     L.kvl_mla_device_free(dx)
     L.kvl_mla_device_free(do)
+
+
+def test_prefill_scale_leaves_out_nan_weights():
+    """The range reductions over o_proj and kv_b leave NaN words out (a NaN weight makes its own output
+    column NaN, not the scale of the others): the other columns equal the clean run's bit for bit."""
+    cfg = inputs.config(**inputs.KIMI)
+    layer = inputs.make_layer(cfg, 0xCD)
+    x = inputs.hidden(cfg, 0xCD, 40)
+    out = []
+    for bad in (False, True):
+        if bad:
+            layer.o_proj = layer.o_proj.copy()
+            layer.o_proj[7, 3] = 0x7FC1
+        w = layer.struct()
+        a = np.zeros_like(x)
+        lib.check(L.kvl_mla_prefill_bf16(f32(a), f32(x), 40, C.byref(cfg), C.byref(w)), "prefill")
+        out.append(a)
+    keep = np.arange(cfg.hidden_size) != 7
+    assert np.all(np.isfinite(out[0])) and np.all(np.isnan(out[1][:, 7]))
+    np.testing.assert_array_equal(out[0][:, keep].view(np.uint32), out[1][:, keep].view(np.uint32))
