@@ -2107,8 +2107,8 @@ __device__ __forceinline__ void fq_wait_all(const FqArgs &f, const unsigned *fla
 // threads l, l + 64, l + 128, l + 192, their tree, then the lanes), and every lane scales its own
 // columns, so the operand equals that kernel's output bit for bit. Every workgroup reads all of x (64
 // KB, from its XCD's L2) beside its 64 KB of weights. Decode stack (27 layers, 8 x 32K rows): the
-// launch grows by 2 us and the norm's launch goes, 1539 -> 1513 us. Only in the kCombXcd form: the
-// branch alone cost the lone decode 0.2 us of 29.3. inv: 8 floats of LDS.
+// launch grows by 2 us and the norm's launch goes, 1539 -> 1513 us. An instance of its own of the
+// kCombXcd form: a branch in the others cost the lone decode 0.2 us of 29.3. inv: 8 floats of LDS.
 __device__ __forceinline__ void fq_norm_x(const FqArgs &f, int B, int kq, v4f (&xa)[2], v4f (&xb)[2], float *inv) {
     const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, n = l & 15, g = l >> 4;
     const float *xr = f.x + (size_t)min(w, B - 1) * f.ldx;
@@ -2181,7 +2181,7 @@ __device__ __forceinline__ void fq_gemv(const FqArgs &f, int B, uint8_t *lds) {
         xa[j] = *(const v4f *)(xr + kbase);
         xb[j] = *(const v4f *)(xr + kbase + 4);
     }
-    if (NORM && f.xnorm) fq_norm_x(f, B, kq, xa, xb, (float *)lds);
+    if (NORM) fq_norm_x(f, B, kq, xa, xb, (float *)lds);
     v4f acc[2][4];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -2478,7 +2478,7 @@ __device__ __forceinline__ void put_q8_weights(int8_t *wqc, const float *pv, flo
 // one XCD, partials read from its L2); across XCDs (partials stored with device-scope stores,
 // read from memory).
 enum { kCombNone = 0, kCombXcd = 1, kCombCross = 2 };
-template <bool FUSE, int COMB>  // FUSE: the launch also prepares the queries and appends the rows (fq_produce)
+template <bool FUSE, int COMB, bool NORM>  // FUSE: the launch also prepares the queries and appends the rows (fq_produce)
 __device__ __forceinline__ void q8_score_role(const AttnArgs &a, const AttnHot &h, const SeqDesc &sd, uint8_t *smem, int w, int b,
                                               int r0, int r1, int nch, int sid, int cpos) {
     int8_t *wq = (int8_t *)(smem + kQ8WqOff);
@@ -2506,7 +2506,7 @@ __device__ __forceinline__ void q8_score_role(const AttnArgs &a, const AttnHot &
         // query copy after Q), its producer task, then (one poller, barrier Q) the 16 query heads
         // of its sequence and, where the split holds the new row (whose scale the loads below
         // read and whose chunk the mix waves request after Q), that row
-        fq_gemv<COMB == kCombXcd>(a.fq, h.nseq, smem + 3 * kQ8CodeB);
+        fq_gemv<NORM>(a.fq, h.nseq, smem + 3 * kQ8CodeB);
         fq_produce(a, h, smem + kQ8WqOff);
         if (w == 0) {
             fq_wait(a.fq, fq_qflag(a.fq, b), 16u);
@@ -2682,7 +2682,7 @@ __device__ __forceinline__ void q8_score_role(const AttnArgs &a, const AttnHot &
     }
 }
 
-template <bool ONCE, bool FUSE, int COMB>
+template <bool ONCE, bool FUSE, int COMB, bool NORM>
 __device__ __forceinline__ void q8_mix_role(const AttnArgs &a, const AttnHot &h, const SeqDesc &sd, uint8_t *smem, int mw, int b,
                                             int r0, int r1, int nch, int sid, int cpos) {
     const int8_t *wq = (const int8_t *)(smem + kQ8WqOff);
@@ -2789,7 +2789,7 @@ __device__ __forceinline__ void q8_mix_role(const AttnArgs &a, const AttnHot &h,
         };
         const bool prod = (int)blockIdx.x < 17 * h.nseq;
         // a projection task goes before the history requests (fq_gemv)
-        fq_gemv<COMB == kCombXcd>(a.fq, h.nseq, smem + 3 * kQ8CodeB);
+        fq_gemv<NORM>(a.fq, h.nseq, smem + 3 * kQ8CodeB);
         if (!prod) issue_ahead();
         fq_produce(a, h, smem + kQ8WqOff);
         if (prod) issue_ahead();
@@ -3105,7 +3105,7 @@ __device__ __forceinline__ void q8_comb_tail(const AttnArgs &a, const SeqDesc &s
 
 // ONCE: each history row is read by one workgroup (non-temporal loads). FUSE: the launch
 // prepares the queries and appends the rows itself (fq_produce; no block launches).
-template <bool ONCE, bool FUSE = false, int COMB = kCombNone>
+template <bool ONCE, bool FUSE = false, int COMB = kCombNone, bool NORM = false>
 __global__ __launch_bounds__(512) void k_attn_q8_mfma(KVL_ATTN_HOT_PARAMS, AttnArgs a) {
     static_assert(COMB == kCombNone || FUSE, "the combine tail is a form of the fused launch");
     KVL_ATTN_HOT_INIT;
@@ -3116,7 +3116,7 @@ __global__ __launch_bounds__(512) void k_attn_q8_mfma(KVL_ATTN_HOT_PARAMS, AttnA
     // comes in the members argument (-splits; a fused launch is never a block launch), which is
     // preloaded: the argument block's copy would cost every workgroup a memory round trip first.
     if (FUSE && (int)blockIdx.x >= -h.members) {
-        fq_gemv<COMB == kCombXcd>(a.fq, h.nseq, smem);
+        fq_gemv<NORM>(a.fq, h.nseq, smem);
         return;
     }
     int b, split, pidx;
@@ -3127,8 +3127,8 @@ __global__ __launch_bounds__(512) void k_attn_q8_mfma(KVL_ATTN_HOT_PARAMS, AttnA
     const int nch = (r1 - r0 + kQ8Ch - 1) / kQ8Ch;
     // chunk of this split holding the row appended in this launch, or -1
     const int cpos = FUSE && split == s.nsplit - 1 ? (s.pos - r0) / kQ8Ch : -1;
-    if (w >= 4) q8_mix_role<ONCE, FUSE, COMB>(a, h, s, smem, w - 4, b, r0, r1, nch, pidx, cpos);
-    else q8_score_role<FUSE, COMB>(a, h, s, smem, w, b, r0, r1, nch, pidx, cpos);
+    if (w >= 4) q8_mix_role<ONCE, FUSE, COMB, NORM>(a, h, s, smem, w - 4, b, r0, r1, nch, pidx, cpos);
+    else q8_score_role<FUSE, COMB, NORM>(a, h, s, smem, w, b, r0, r1, nch, pidx, cpos);
     if constexpr (COMB != kCombNone) q8_comb_tail<COMB>(a, s, b, split, smem);
 }
 
@@ -3165,6 +3165,7 @@ hipError_t launch_attention(hipStream_t st, int kind, int fmt, const SeqTable &t
                (fq->comb == kCombXcd && !comb_ok(t, d, total_splits)) ||
                (fq->comb == kCombCross && !comb_cross_ok(t, d)) || fq->comb < 0 || fq->comb > kCombCross ||
                (fq->comb && (!fq->kvb || !fq->ho || !fq->hos)) || fq->splits != total_splits ||
+               (fq->xnorm && (fq->comb != kCombXcd || !fq->gemv)) ||
                (fq->gemv && (!gemv_fuse_ok(d, t.n) || !fq->x || !fq->wq || !fq->wkva ||
                              fq->in != d.H || fq->out0 != d.QO || fq->out1 != d.KVO || (uintptr_t)fq->x % 16 != 0 ||
                              fq->ldx % 4 != 0))))
@@ -3193,6 +3194,7 @@ hipError_t launch_attention(hipStream_t st, int kind, int fmt, const SeqTable &t
     }
     if (kind == kAttnQ8Mfma) {
         if (a.members > 0) hipLaunchKernelGGL(k_attn_q8_mfma<false>, dim3(grid), dim3(512), 0, st, a.members, a.nseq, a.qhi, a.qlo, a.qrhi, a.qrlo, a.qs, a.qf, a.part, a);
+        else if (fq && fq->comb == kCombXcd && fq->gemv && fq->xnorm) hipLaunchKernelGGL((k_attn_q8_mfma<true, true, kCombXcd, true>), dim3(grid), dim3(512), 0, st, -total_splits, a.nseq, a.qhi, a.qlo, a.qrhi, a.qrlo, a.qs, a.qf, a.part, a);
         else if (fq && fq->comb == kCombXcd) hipLaunchKernelGGL((k_attn_q8_mfma<true, true, kCombXcd>), dim3(grid), dim3(512), 0, st, -total_splits, a.nseq, a.qhi, a.qlo, a.qrhi, a.qrlo, a.qs, a.qf, a.part, a);
         else if (fq && fq->comb == kCombCross) hipLaunchKernelGGL((k_attn_q8_mfma<true, true, kCombCross>), dim3(grid), dim3(512), 0, st, -total_splits, a.nseq, a.qhi, a.qlo, a.qrhi, a.qrlo, a.qs, a.qf, a.part, a);
         else if (fq) hipLaunchKernelGGL((k_attn_q8_mfma<true, true>), dim3(grid), dim3(512), 0, st, -total_splits, a.nseq, a.qhi, a.qlo, a.qrhi, a.qrlo, a.qs, a.qf, a.part, a);
