@@ -2,13 +2,15 @@
 // reference: non-absorbed attention, K/V expanded through kv_b for every token).
 //
 // MFMA route (H, R and NH * DV multiples of 64, QD = 192, DV = 128, DN multiple of 8):
-//   split     x (fp32) -> bf16 hi + lo operands; a flag records whether any lo is non-zero
-//   gemm      [q | kv_a] = x . W^T           (bf16 MFMA, fp32 accumulate, lo pass skipped
+//   split     x (fp32) -> bf16 hi + lo operands; a flag records whether any lo is non-zero (a short
+//             prompt without a state fill skips this: its projection splits fp32 x itself)
+//   gemm      [q | kv_a] = x . W^T           (bf16 MFMA, fp32 accumulate, the lo part skipped
 //                                             when the operand is exactly bf16); epilogue:
-//                                             Q = [q_nope | RoPE(q_rope)] as hi/lo fp16
+//                                             Q = [q_nope | RoPE(q_rope)] as fp16 hi and bf8 lo.
+//             A short prompt splits k over blocks and leaves the sums to kva_pack.
 //   kva_pack  RMSNorm -> latent (hi/lo bf16), RoPE(k_rope) -> rope part of K (fp16 hi + K8)
 //   gemm      kv = latent . kv_b^T           epilogue: k_nope -> K (fp16 hi + K8), V^T (fp16)
-//   flash     causal attention per (128-query tile, head), online softmax; scores Kh Qh in
+//   flash     causal attention per (64- or 128-query tile, head), online softmax; scores Kh Qh in
 //             fp16 plus the Kh Ql + Kl Qh correction from bf8 operands (K8: bf8 of the hi
 //             parts and of the lo parts x 2^11)
 //   gemm      out = heads . o_proj^T          (fp16 heads and fp16 copy of o_proj, one pass)
@@ -1330,6 +1332,18 @@ static int gen_query_tile(const Dims &d, int S) {
     return (int)std::max<size_t>(1, std::min<size_t>((size_t)S, cap / per_query));
 }
 
+// Largest partials of a split q (| kv_a) projection, whatever the call: the workspace of S tokens then
+// never exceeds that of more tokens, so a graph capture fits what a longer call has grown.
+static size_t gemm_part_bytes(const Dims &d) {
+    size_t most = 0;
+    for (int mt = 1; mt <= 128; ++mt) {  // 64-token tile rows; more never split
+        const int k0 = gemm_part_ks(64 * mt, d.QO, 0, d.H), k1 = gemm_part_ks(64 * mt, d.QO, d.KVO, d.H);
+        const size_t n = std::max(k0 > 1 ? k0 * d.QO : 0, k1 > 1 ? k1 * (d.QO + d.KVO) : 0);
+        most = std::max(most, 4 * (size_t)(64 * mt) * n);
+    }
+    return most;
+}
+
 size_t prefill_bytes(const Dims &d, int S, bool generic) {
     const size_t Sp = (size_t)(S + 127) / 128 * 128;
     size_t b = 0;
@@ -1339,9 +1353,7 @@ size_t prefill_bytes(const Dims &d, int S, bool generic) {
         add(2 * (size_t)S * d.H);                // x hi
         add(2 * (size_t)S * d.H);                // x lo
         add(4 * (size_t)S * d.KVO * (prefill_kva_exact(d) ? kGemvKs : 1));  // kv_a projection
-        // partials of a split q | kv_a projection (of q alone where a state fill asks for its own kv_a)
-        const int k0 = gemm_part_ks(S, d.QO, 0, d.H), k1 = gemm_part_ks(S, d.QO, d.KVO, d.H);
-        add(4 * (size_t)S * std::max(k0 > 1 ? k0 * d.QO : 0, k1 > 1 ? k1 * (d.QO + d.KVO) : 0));
+        add(gemm_part_bytes(d));                 // partials of a split q | kv_a projection
         add(2 * (size_t)S * d.R);                // latent hi
         add(2 * (size_t)S * d.R);                // latent lo
         add(2 * (size_t)d.NH * Sp * d.QD);       // q hi (fp16)
@@ -1388,7 +1400,7 @@ hipError_t launch_prefill_all(hipStream_t st, const Dims &d, int S, float eps, c
         const int np = exact ? kGemvKs : 1;
         const int qn1 = exact ? 0 : d.KVO, ks = gemm_part_ks(S, d.QO, qn1, d.H);
         float *ykva = (float *)take(4 * (size_t)S * d.KVO * np);
-        float *ypart = ks > 1 ? (float *)take(4 * (size_t)S * ks * (d.QO + qn1)) : nullptr;
+        float *ypart = (float *)take(gemm_part_bytes(d));
         uint16_t *lath = (uint16_t *)take(2 * (size_t)S * d.R);
         uint16_t *latl = (uint16_t *)take(2 * (size_t)S * d.R);
         _Float16 *qh = (_Float16 *)take(2 * (size_t)d.NH * Sp * d.QD);
@@ -1434,7 +1446,7 @@ hipError_t launch_prefill_all(hipStream_t st, const Dims &d, int S, float eps, c
         KvaPackArgs ka{kpart ? ypart + d.QO : ykva, wnorm, cs, lath, latl, qh, ql8, kh, k8, vt,
                        kpart ? (size_t)S * ldq : (size_t)S * d.KVO, kpart ? ks : np,
                        S, Sp, d.NH, kpart ? ldq : d.KVO, d.R, d.DN, d.DR, d.DV, eps, flags + 0,
-                       ypart, (size_t)S * ldq, ks, ldq, vpad, ep};
+                       ks > 1 ? ypart : nullptr, (size_t)S * ldq, ks, ldq, vpad, ep};
         const int qblocks = ks > 1 ? (int)(((size_t)S * (d.QO / 4) + 255) / 256) : 0;
         hipLaunchKernelGGL(k_kva_pack, dim3((S + 3) / 4 + vpad + qblocks), dim3(256), 0, st, ka);
         if ((e = hipGetLastError()) != hipSuccess) return e;
