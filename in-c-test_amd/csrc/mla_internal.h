@@ -116,10 +116,11 @@ hipError_t launch_clear_flags(hipStream_t st, unsigned *flags, int nlines);
 // nrows > 0: rows mode, nrows rows of the single sequence t.s[0] starting at t.s[0].pos,
 // input row i at y + i*ldy, staged row i at w.rows + i*row_bytes.
 // y holds ynp (1 or kGemvKs) partials ypstride floats apart; their in-order sum is the input.
+// stage = false: the copy at w.rows (which stays a valid buffer) may be left out in rows mode.
 hipError_t launch_append(hipStream_t st, int fmt, const SeqTable &t, const Dims &d,
                          const float *y, int ldy, int koff, int ynp, size_t ypstride,
                          const uint16_t *kv_a_norm, float eps, const float2 *rope_cs,
-                         const DecodeWork &w, bool normed, int nrows);
+                         const DecodeWork &w, bool normed, int nrows, bool stage = true);
 
 // y[i] = RMSNorm(x[i]) * w for `rows` rows of length n (src/ops.c:76-83).
 hipError_t launch_rmsnorm(hipStream_t st, float *y, const float *x, const uint16_t *w, int n,

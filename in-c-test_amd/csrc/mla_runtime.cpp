@@ -1565,10 +1565,11 @@ int fill_begin(int seq_len, const KvlMlaConfig *cfg, const KvlMlaBF16 *w, S *s, 
 // Rows [t0, t0 + n) of the state from the kv_a projection of those tokens on the device (np
 // partials pstride floats apart, token i at y + i * ldy): the append kernel in rows mode
 // (RMSNorm, RoPE, the state's row format) writes the device mirror and stages the rows in
-// c.fill; with host_rows they are also copied into the host arrays (synchronous).
+// c.fill (unless !stage: nobody reads them there); with host_rows they are also copied into the host
+// arrays (synchronous).
 template <class S>
 int fill_rows(S *s, const FillCtx &f, const float *y, int ldy, int np, size_t pstride, int t0, int n,
-              bool host_rows) {
+              bool host_rows, bool stage = true) {
     Ctx &c = ctx();
     const size_t rb = row_bytes_of(f.fmt, f.d.R, f.d.DR, 0);
     if (dev_reserve(c.fill, (size_t)n * rb) != 0) return -1;
@@ -1582,7 +1583,8 @@ int fill_rows(S *s, const FillCtx &f, const float *y, int ldy, int np, size_t ps
     t.s[0].pos = t0;
     DecodeWork wk{};
     wk.rows = drows;
-    HIP_TRY(launch_append(c.stream, f.fmt, t, f.d, y, ldy, 0, np, pstride, f.norm, f.eps, f.cs, wk, false, n));
+    HIP_TRY(launch_append(c.stream, f.fmt, t, f.d, y, ldy, 0, np, pstride, f.norm, f.eps, f.cs, wk, false, n,
+                          host_rows || stage));
     if (!host_rows) return 0;
     if (pin_reserve(c.pin_out, (size_t)n * rb) != 0) return -1;
     HIP_TRY(hipMemcpyAsync(c.pin_out.p, drows, (size_t)n * rb, hipMemcpyDeviceToHost, c.stream));
@@ -1739,7 +1741,7 @@ int prefill_state_device(float *d_out, const float *d_x, int seq_len, const KvlM
     PrefillKva kv{};
     if (prefill_device(d_out, d_x, seq_len, cfg, w, &kv, host_call) != 0) return -1;
     if (kv.y) {
-        if (fill_rows(s, f, kv.y, kv.ldy, kv.np, kv.pstride, 0, seq_len, host_rows) != 0) return -1;
+        if (fill_rows(s, f, kv.y, kv.ldy, kv.np, kv.pstride, 0, seq_len, host_rows, host_call) != 0) return -1;
     } else {
         Ctx &c = ctx();
         const int chunk = 4096;

@@ -216,3 +216,29 @@ def test_rows_do_not_depend_on_the_prompt_length(S):
         _long_rows[2000] = f32_rows(2000)
     for got, full in zip(f32_rows(S), _long_rows[2000]):
         np.testing.assert_array_equal(got, full[:S])
+
+
+@pytest.mark.parametrize("kind", ["f32", "q8"])
+def test_prefilled_special_rows_equal_decoded_rows(kind):
+    """The rows kernel of a state prefill against the append of a decode, on tokens whose rows meet the
+    quantiser's special cases: all zero, overflowing, NaN, subnormal products (NaN compares equal)."""
+    cfg = inputs.config(**inputs.KIMI)
+    layer = inputs.make_layer(cfg, 0xD9)
+    w = layer.struct()
+    x = np.ascontiguousarray(inputs.hidden(cfg, 0xD9, 7))
+    x[1] = 0.0
+    x[2] *= np.float32(1e38)
+    x[3, 100] = np.nan
+    x[4] *= np.float32(1e-30)
+    x[5, 0] = np.inf
+    _, dec = decode_seq(G, kind, cfg, w, x)
+    st = new_state(G, kind, cfg, 7)
+    lib.check(getattr(G, STATE[kind][1] + "_prefill_bf16")(f32(x), 7, C.byref(cfg), C.byref(w), C.byref(st)),
+              "state prefill")
+    pre = snapshot(kind, st, cfg)
+    free_state(G, kind, st)
+    for name in dec:
+        a, b = pre[name], dec[name]
+        if name == "rope" and kind == "q8":
+            a, b = (inputs.bf16_bits_to_f32(v) for v in (a, b))
+        np.testing.assert_array_equal(a, b, err_msg=f"{kind} {name}")
