@@ -825,11 +825,11 @@ struct FlashArgs {
 // row-max logits up to ~150 give 3e-4, ~500 give 6e-4, ~1450 give 1.7e-3, ~4400 give 2.3e-3.
 constexpr float kFLogitMax = 512.0f;
 
-// v_max3_f32 as one instruction (fmaxf makes the compiler quiet each operand first).
+// v_maximum3_f32: two operations that the compiler knows, so that it puts the wait states an MFMA
+// result needs in front of them. A NaN score makes the maximum NaN, which raises nothing; its weight
+// makes the query's sum and outputs NaN, which the range check finds.
 __device__ __forceinline__ float max3(float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
+    return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
 }
 // Max / sum over the four lanes n, n + 16, n + 32, n + 48 (one per 16-lane row).
 __device__ __forceinline__ float xrow_max(float v) {
