@@ -7,7 +7,6 @@
 //   gemm      [q | kv_a] = x . W^T           (bf16 MFMA, fp32 accumulate, the lo part skipped
 //                                             when the operand is exactly bf16); epilogue:
 //                                             Q = [q_nope | RoPE(q_rope)] as fp16 hi and bf8 lo.
-//             A short prompt splits k over blocks and leaves the sums to kva_pack.
 //   kva_pack  RMSNorm -> latent (hi/lo bf16), RoPE(k_rope) -> rope part of K (fp16 hi + K8)
 //   gemm      kv = latent . kv_b^T           epilogue: k_nope -> K (fp16 hi + K8), V^T (fp16)
 //   flash     causal attention per (64- or 128-query tile, head), online softmax; scores Kh Qh in
@@ -109,7 +108,7 @@ struct GemmCfg {
     static constexpr int Threads = 64 * (MW + kGemmDma);
     static_assert(LO || !AF32, "fp32 A is split into hi and lo");
     static_assert(Stages >= 2 && TM >= 1 && WM * WN == MW && WM * TM * 16 == BM, "tile shape");
-    static_assert(Smem >= MW * 16 * 68 * 4, "the epilogue's staging fits the ring");
+    static_assert(Smem >= MW * 16 * (16 * TN + 4) * 4, "the epilogue's staging fits the ring");
     __device__ static int swz(int row) { return BK == 64 ? row & 7 : (row >> 1) & 3; }
 };
 
@@ -118,8 +117,6 @@ struct GemmArgs {
     float *C;
     const int *lo_flag;
     int M, N0, N1, K, lda, ldb, ldc;
-    int ks;          // kEpiPart: k ranges, range s written to C + s * pstride
-    size_t pstride;
     const float *Af;  // fp32 A [M, lda] (GemmCfg::AF32)
     int *clear;       // a word the launch clears (may be null)
 };
@@ -130,8 +127,7 @@ struct GemmArgs {
 // (kv_b projection): k_nope -> K hi [NH, Sp, QD] fp16 and K8 [NH, Sp, 384 bytes] (bf8 of the
 // hi parts and of the lo parts x 2^11, k8_hi_byte order), values -> V^T [NH, DV, Sp] fp16 with
 // the keys of each 32-key group in vt_perm order.
-// kEpiPart: the fp32 sums of one of a.ks ranges of k (k_kva_pack adds them in order).
-enum { kEpiPlain = 0, kEpiQ = 1, kEpiKV = 2, kEpiPart = 3 };
+enum { kEpiPlain = 0, kEpiQ = 1, kEpiKV = 2 };
 struct GemmEpi {
     _Float16 *qh, *kh;
     uint8_t *ql8;  // bf8(Q lo x 2^11), the flash kernel's correction operand (kEpiQ)
@@ -207,12 +203,11 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
     const int wm = w / Sh::WN, wn = w % Sh::WN;
     const int M = a.M, N0 = a.N0, N1 = a.N1, K = a.K, lda = a.lda, ldb = a.ldb;
     const int tn0 = (N0 + BN - 1) / BN, tn = tn0 + (N1 + BN - 1) / BN;
-    const int tm = (M + BM - 1) / BM, ks = EPI == kEpiPart ? a.ks : 1, ntiles = tm * tn * ks;
+    const int tm = (M + BM - 1) / BM, ntiles = tm * tn;
     // Tiles in row-major order, XCD b % 8 taking a contiguous eighth of them (blocks of one XCD
     // share A rows in its L2).
     const int xcd = blockIdx.x & 7, per = ntiles >> 3, rem = ntiles & 7;
-    const int task = xcd * per + min(xcd, rem) + (blockIdx.x >> 3);
-    const int tile = EPI == kEpiPart ? task / ks : task, kr = EPI == kEpiPart ? task % ks : 0;
+    const int tile = xcd * per + min(xcd, rem) + (blockIdx.x >> 3);
     const int mt = tile / tn, nt = tile % tn;
     const bool seg1 = nt >= tn0;
     const uint16_t *B = seg1 ? a.B1 : a.B0;
@@ -223,7 +218,7 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
     const bool use_lo = Sh::LO && (Sh::AF32 || (a.Al && (!a.lo_flag || *a.lo_flag)));
     if (a.clear && blockIdx.x == 0 && tid == 0) __hip_atomic_store(a.clear, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 
-    const int nkt = K / BK / ks, kt0 = kr * nkt;  // this block's k steps (ks divides K / BK)
+    const int nkt = K / BK;
     constexpr int NS = Sh::Stages;
     if (w >= Sh::MW) {
         // DMA wave dw: instruction i fills slot (4i + dw) * 64 + l of a tile: row p / Spr,
@@ -257,7 +252,7 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
             constexpr bool kLo = decltype(lo_tag)::value;
             auto issue = [&](int kt, int stage) __attribute__((always_inline)) {
                 const uint32_t dst = sbase + stage * Sh::Stage + (uint32_t)dw * 1024;
-                const size_t ko = (size_t)(kt0 + kt) * RowB;
+                const size_t ko = (size_t)kt * RowB;
 #pragma unroll
                 for (int i = 0; i < (Sh::AF32 ? 2 : 1) * NA; ++i)
                     dma_b128_s(gah + (Sh::AF32 ? 2 * ko : ko), aoff[i], dst + i * (kGemmDma * 1024));
@@ -344,14 +339,13 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
     if (Sh::AF32 || use_lo) compute(std::integral_constant<bool, Sh::LO>{});
     else compute(std::false_type{});
     // Epilogue. D layout: lane (g, n) of tile (i, j) holds rows 4g + r, column n. Row-major
-    // outputs go through a per-wave LDS buffer (16 rows x 64 columns per tile row i): lane l
-    // then takes columns 4 (l % 16) .. + 3 of rows l / 16 + 4 q, q = 0..3, so the 16 lanes of a
-    // row write its 64 columns as one contiguous run (scattered 16-byte pieces per lane cost
+    // outputs go through a per-wave LDS buffer (16 rows x CW = 16 TN columns per tile row i): lane
+    // l then takes columns 4 (l % LR) .. + 3 of rows l / LR + RP q, so the LR lanes of a row
+    // write its CW columns as one contiguous run (scattered 16-byte pieces per lane cost
     // ~10 us more per launch at these sizes), and the rope pairs (2p, 2p+1) sit in one lane.
     // The V^T part of kEpiKV wants 4 consecutive tokens per lane, which the D layout gives.
-    if constexpr (TN < 4) {
-        // narrow tiles (kEpiPlain): stored from the D layout, 64-byte runs
-        static_assert(TN == 4 || EPI == kEpiPlain, "the staged epilogue assumes 64 columns per wave");
+    static_assert(TN == 4 || EPI != kEpiKV, "a wave's columns of kEpiKV are all keys or all values");
+    if constexpr (TN < 4 && EPI == kEpiPlain) {  // stored from the D layout, 64-byte runs
         lds_barrier();  // the DMA waves' last barrier
         float al = e.alpha;
         if (e.nan_flag && __hip_atomic_load(e.nan_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
@@ -372,10 +366,11 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
     } else {
     const int QD = e.DN + e.DR, KH = e.DN + e.DV;
     lds_barrier();  // every wave is done with the ring
-    float *ep = (float *)smem + w * (16 * 68);
-    const int cw = wn * 64;                      // wave's first column within the tile
+    constexpr int CW = 16 * TN, LR = CW / 4, RP = 64 / LR, EpS = CW + 4;
+    float *ep = (float *)smem + w * (16 * EpS);
+    const int cw = wn * CW;                      // wave's first column within the tile
     const bool vt_wave = EPI == kEpiKV && ((nb0 + cw) % KH) >= e.DN;
-    const int rr = l >> 4, cc = (l & 15) * 4;    // staged row (+ 4 q) / first column of this lane
+    const int rr = l / LR, cc = (l % LR) * 4;    // staged row (+ RP q) / first column of this lane
     const int nl0 = nb0 + cw + cc;               // segment column of v[0]
     float alpha = e.alpha;
     if (EPI == kEpiPlain && e.nan_flag && __hip_atomic_load(e.nan_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
@@ -406,19 +401,17 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) ep[(4 * g + r) * 68 + 16 * j + n] = acc[i][j][r];
-        v4f vq[4];
+            for (int r = 0; r < 4; ++r) ep[(4 * g + r) * EpS + 16 * j + n] = acc[i][j][r];
+        v4f vq[16 / RP];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) vq[q] = *(const v4f *)(ep + (rr + 4 * q) * 68 + cc);
+        for (int q = 0; q < 16 / RP; ++q) vq[q] = *(const v4f *)(ep + (rr + RP * q) * EpS + cc);
         if (nl0 >= Nseg) continue;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int t = rbase + rr + 4 * q;
+        for (int q = 0; q < 16 / RP; ++q) {
+            const int t = rbase + rr + RP * q;
             if (t >= M) continue;
-            if (EPI == kEpiPlain || EPI == kEpiPart || (EPI == kEpiQ && seg1)) {
-                float *dst = EPI == kEpiPlain  ? a.C + (size_t)t * a.ldc + c0 + cw + cc
-                             : EPI == kEpiPart ? a.C + kr * a.pstride + (size_t)t * a.ldc + c0 + cw + cc
-                                               : a.C + (size_t)t * a.ldc + nl0;
+            if (EPI == kEpiPlain || (EPI == kEpiQ && seg1)) {
+                float *dst = EPI == kEpiPlain ? a.C + (size_t)t * a.ldc + c0 + cw + cc : a.C + (size_t)t * a.ldc + nl0;
                 *(v4f *)dst = EPI == kEpiPlain ? vq[q] * alpha : vq[q];
             } else if (EPI == kEpiQ) {
                 store_q4(e, t, nl0, vq[q]);
@@ -458,32 +451,35 @@ static hipError_t gemm_launch(hipStream_t st, const GemmArgs &a, const GemmEpi &
 
 enum { kTile64x64 = 0, kTile128x64, kTile128x128, kTile192x128, kTile256x128, kTile256x256, kGemmTiles };
 
-// K ranges of the q | kv_a projection of M tokens: 64 x 64 tiles with the whole of k take in 768 KB
-// each, at the 70 GB/s a CU takes in, so while their number leaves CUs idle k is split over 2 or 4
-// blocks, whose sums go through memory to k_kva_pack. Alone, whole k / 2 / 4 ranges (us): 10.3 / 6.8 / 5.0 at
-// 37 tokens (57 tiles), 11.6 / 8.1 / 8.4 at 100 (114), 12.8 / 12.3 / 12.0 at 192 (171).
-static int gemm_part_ks(int M, int N0, int N1, int K) {
-    const int tiles = (M + 63) / 64 * ((N0 + 63) / 64 + (N1 + 63) / 64);
-    const int ks = tiles <= 64 ? 4 : tiles <= 128 ? 2 : 1;
-    return K % (64 * ks) == 0 && N0 % 4 == 0 && N1 % 4 == 0 ? ks : 1;
+// The q (| kv_a) projection of a short prompt, from fp32 x when x is given (16-byte aligned; *clear is
+// then cleared, which k_split does otherwise), else from the planes. Every tile sums the whole of k in
+// one order, as the tiles of longer prompts do, so a token's Q and kv_a do not depend on how many tokens
+// follow it (k split over 4 blocks, its sums added by k_kva_pack, gave 30.2 us for 37 tokens in all where
+// this gives 35.3, and lost that). A block's time is the serial chain of its 64 k-subs (LDS reads, splits,
+// MFMAs; stages of 128 or 256 k change nothing), so the smallest tile that still gives every tile a CU
+// runs. us with weights in
+// the caches / from memory, 32 x 32, 32 x 64, 64 x 64 (tokens x columns, two blocks a CU):
+//   fp32 x, q | kv_a   37: 11.3 / 15.0  13.5 / 17.8  14.5 / 21.7   128: 19.7 / 23.2  14.3 / 20.4  15.5 / 23.9
+//   planes, q alone    37:  7.7 / 14.5   9.8 / 17.5  11.0 / 22.2   160: 13.7 / 20.9  13.1 / 19.8  13.9 / 23.8
+//   fp32 x, q | kv_a  160: 27.7 / 31.2  24.3 / 28.5  15.8 / 24.1
+// The planes are 3 us quicker to multiply than fp32 x at 37 tokens, the k_split launch costs 2.3.
+template <class P, class F>
+static hipError_t gemm_q_launch(hipStream_t st, const GemmArgs &a, const GemmEpi &e) {
+    const int tiles = (a.M + P::BM - 1) / P::BM * ((a.N0 + P::BN - 1) / P::BN + (a.N1 + P::BN - 1) / P::BN);
+    return a.Af ? gemm_launch<F, kEpiQ, false>(st, a, e, tiles) : gemm_launch<P, kEpiQ, false>(st, a, e, tiles);
 }
 
-// The q (| kv_a) projection of a short prompt in 64 x 64 tiles: from fp32 x when x is given (16-byte
-// aligned; *clear is then cleared, which k_split does otherwise), else from the planes; ks > 1: the
-// partials of its k ranges into C, else Q and kv_a (ldc = N1) as kEpiQ. Without the k_split launch,
-// 37 tokens take 34.2 us in all instead of 36.5.
 static hipError_t gemm_q_small(hipStream_t st, const float *x, int *clear, const uint16_t *Ah, const uint16_t *Al,
                                const int *flag, const uint16_t *B0, int N0, const uint16_t *B1, int N1, float *C, int M,
-                               int K, int ks, const GemmEpi &e) {
-    GemmArgs a{Ah, Al, B0, B1 ? B1 : B0, C, flag, M, N0, N1, K, K, K, ks > 1 ? N0 + N1 : N1, ks,
-               (size_t)M * (N0 + N1), x, x ? clear : nullptr};
-    if (K % (64 * ks)) return hipErrorInvalidValue;
-    const int tiles = (M + 63) / 64 * ((N0 + 63) / 64 + (N1 + 63) / 64);
-    using P = GemmCfg<64, 64, 64, 4, 2, true>;
-    using F = GemmCfg<64, 64, 64, 4, 2, true, true>;
-    if (ks > 1)
-        return x ? gemm_launch<F, kEpiPart, false>(st, a, e, tiles * ks) : gemm_launch<P, kEpiPart, false>(st, a, e, tiles * ks);
-    return x ? gemm_launch<F, kEpiQ, false>(st, a, e, tiles) : gemm_launch<P, kEpiQ, false>(st, a, e, tiles);
+                               int K, const GemmEpi &e) {
+    const GemmArgs a{Ah, Al, B0, B1 ? B1 : B0, C, flag, M, N0, N1, K, K, K, N1, x, x ? clear : nullptr};
+    if (K % 64) return hipErrorInvalidValue;
+    auto tiles = [&](int bm, int bn) { return (M + bm - 1) / bm * ((N0 + bn - 1) / bn + (N1 + bn - 1) / bn); };
+    if (tiles(32, 32) <= 256)
+        return gemm_q_launch<GemmCfg<32, 32, 64, 2, 2, true>, GemmCfg<32, 32, 64, 2, 2, true, true>>(st, a, e);
+    if (tiles(32, 64) <= 256)
+        return gemm_q_launch<GemmCfg<32, 64, 64, 2, 2, true>, GemmCfg<32, 64, 64, 2, 2, true, true>>(st, a, e);
+    return gemm_q_launch<GemmCfg<64, 64, 64, 4, 2, true>, GemmCfg<64, 64, 64, 4, 2, true, true>>(st, a, e);
 }
 
 static int gemm_pick(int epi, int M, int N0, int N1, int *tiles) {
@@ -513,7 +509,7 @@ template <int EPI, bool F16 = false>
 static hipError_t gemm(hipStream_t st, const uint16_t *Ah, const uint16_t *Al, const int *flag,
                        int lda, const uint16_t *B0, int N0, const uint16_t *B1, int N1, int ldb,
                        float *C, int ldc, int M, int K, const GemmEpi &e) {
-    GemmArgs a{Ah, Al, B0, B1 ? B1 : B0, C, flag, M, N0, N1, K, lda, ldb, ldc, 1, 0, nullptr, nullptr};
+    GemmArgs a{Ah, Al, B0, B1 ? B1 : B0, C, flag, M, N0, N1, K, lda, ldb, ldc, nullptr, nullptr};
     if (K % 64) return hipErrorInvalidValue;
     constexpr bool LO = !F16;  // the fp16 product has no lo operand
     if (!LO && Al) return hipErrorInvalidValue;
@@ -603,8 +599,6 @@ struct KvaPackArgs {
     const uint16_t *norm;
     const float2 *cs;
     uint16_t *lath, *latl;
-    _Float16 *qh;
-    uint8_t *ql8;
     _Float16 *kh;
     uint8_t *k8;
     _Float16 *vt;
@@ -612,12 +606,6 @@ struct KvaPackArgs {
     int np, S, Sp, NH, ldy, R, DN, DR, DV;
     float eps;
     int *x_flag;     // the x lo flag, cleared for the next prefill (its one reader has run)
-    // q (may be null): nq partials of the q projection [S, ldq], qpstride floats apart; blocks past
-    // the tokens and the padding add them in order and write Q (store_q4)
-    const float *q;
-    size_t qpstride;
-    int nq, ldq, pad_blocks;
-    GemmEpi qe;
 };
 
 __global__ __launch_bounds__(256) void k_kva_pack(KvaPackArgs a) {
@@ -625,16 +613,6 @@ __global__ __launch_bounds__(256) void k_kva_pack(KvaPackArgs a) {
     if (blockIdx.x == 0 && threadIdx.x == 0 && a.x_flag) *a.x_flag = 0;
     const int QD = a.DN + a.DR, half = a.DR / 2, R = a.R;
     const int tblocks = (a.S + 3) / 4;
-    if ((int)blockIdx.x >= tblocks + a.pad_blocks) {
-        const int i = ((int)blockIdx.x - tblocks - a.pad_blocks) * 256 + threadIdx.x, per = a.NH * QD / 4;
-        if (i >= a.S * per) return;
-        const int tq = i / per, c = 4 * (i % per);
-        const float *q = a.q + (size_t)tq * a.ldq + c;
-        v4f v = *(const v4f *)q;
-        for (int p = 1; p < a.nq; ++p) v += *(const v4f *)(q + p * a.qpstride);
-        store_q4(a.qe, tq, c, v);
-        return;
-    }
     if ((int)blockIdx.x >= tblocks) {  // padding keys of V^T: 16 rows (h, d) per wave, one key per lane
         const int r0 = 16 * (t - 4 * tblocks);
         for (int r = r0; r < min(r0 + 16, a.NH * a.DV); ++r)
@@ -1345,18 +1323,6 @@ static int gen_query_tile(const Dims &d, int S) {
     return (int)std::max<size_t>(1, std::min<size_t>((size_t)S, cap / per_query));
 }
 
-// Largest partials of a split q (| kv_a) projection, whatever the call: the workspace of S tokens then
-// never exceeds that of more tokens, so a graph capture fits what a longer call has grown.
-static size_t gemm_part_bytes(const Dims &d) {
-    size_t most = 0;
-    for (int mt = 1; mt <= 128; ++mt) {  // 64-token tile rows; more never split
-        const int k0 = gemm_part_ks(64 * mt, d.QO, 0, d.H), k1 = gemm_part_ks(64 * mt, d.QO, d.KVO, d.H);
-        const size_t n = std::max(k0 > 1 ? k0 * d.QO : 0, k1 > 1 ? k1 * (d.QO + d.KVO) : 0);
-        most = std::max(most, 4 * (size_t)(64 * mt) * n);
-    }
-    return most;
-}
-
 size_t prefill_bytes(const Dims &d, int S, bool generic) {
     const size_t Sp = (size_t)(S + 127) / 128 * 128;
     size_t b = 0;
@@ -1366,7 +1332,6 @@ size_t prefill_bytes(const Dims &d, int S, bool generic) {
         add(2 * (size_t)S * d.H);                // x hi
         add(2 * (size_t)S * d.H);                // x lo
         add(4 * (size_t)S * d.KVO * (prefill_kva_exact(d) ? kGemvKs : 1));  // kv_a projection
-        add(gemm_part_bytes(d));                 // partials of a split q | kv_a projection
         add(2 * (size_t)S * d.R);                // latent hi
         add(2 * (size_t)S * d.R);                // latent lo
         add(2 * (size_t)d.NH * Sp * d.QD);       // q hi (fp16)
@@ -1411,9 +1376,8 @@ hipError_t launch_prefill_all(hipStream_t st, const Dims &d, int S, float eps, c
         uint16_t *xl = (uint16_t *)take(2 * (size_t)S * d.H);
         const bool exact = kva && prefill_kva_exact(d);
         const int np = exact ? kGemvKs : 1;
-        const int qn1 = exact ? 0 : d.KVO, ks = gemm_part_ks(S, d.QO, qn1, d.H);
+        const int qn1 = exact ? 0 : d.KVO;
         float *ykva = (float *)take(4 * (size_t)S * d.KVO * np);
-        float *ypart = (float *)take(gemm_part_bytes(d));
         uint16_t *lath = (uint16_t *)take(2 * (size_t)S * d.R);
         uint16_t *latl = (uint16_t *)take(2 * (size_t)S * d.R);
         _Float16 *qh = (_Float16 *)take(2 * (size_t)d.NH * Sp * d.QD);
@@ -1431,7 +1395,7 @@ hipError_t launch_prefill_all(hipStream_t st, const Dims &d, int S, float eps, c
         // A short prompt's projection takes x as it is (gemm_q_small) and needs no planes (with a state
         // fill, launch_kva_tok needs them all the same: reading fp32 x there cost more than the launch).
         int qtiles = 0;
-        const bool small = ks > 1 || gemm_pick(kEpiQ, S, d.QO, qn1, &qtiles) == kTile64x64;
+        const bool small = gemm_pick(kEpiQ, S, d.QO, qn1, &qtiles) == kTile64x64;
         const bool direct = small && !exact && (uintptr_t)x % 16 == 0;
         if (!direct) {
             const int split_blocks = std::min(2048, S);
@@ -1441,10 +1405,9 @@ hipError_t launch_prefill_all(hipStream_t st, const Dims &d, int S, float eps, c
         // q (-> Q hi/lo, rotated) | kv_a (-> ykva). When the caller fills a state from this
         // kv_a, it is computed with the decode's k-split arithmetic (launch_kva_tok) so those
         // rows equal the rows a decode appends; otherwise it rides along in the q GEMM.
-        // A short prompt splits k (gemm_part_ks) and k_kva_pack adds the partials.
         if (small)
             e = gemm_q_small(st, direct ? x : nullptr, flags + 1, xh, xl, flags + 0, wq, d.QO, exact ? nullptr : wkva, qn1,
-                             ks > 1 ? ypart : ykva, S, d.H, ks, ep);
+                             ykva, S, d.H, ep);
         else if (exact) e = gemm<kEpiQ>(st, xh, xl, flags + 0, d.H, wq, d.QO, nullptr, 0, d.H, nullptr, 0, S, d.H, ep);
         else e = gemm<kEpiQ>(st, xh, xl, flags + 0, d.H, wq, d.QO, wkva, d.KVO, d.H, ykva, d.KVO, S, d.H, ep);
         if (e != hipSuccess) return e;
@@ -1454,14 +1417,10 @@ hipError_t launch_prefill_all(hipStream_t st, const Dims &d, int S, float eps, c
                 return e;
             if (kva) *kva = PrefillKva{ykva, d.KVO, np, (size_t)S * d.KVO};
         }
-        const int vpad = Sp > S ? (d.NH * d.DV + 63) / 64 : 0, ldq = d.QO + qn1;
-        const bool kpart = ks > 1 && !exact;  // kv_a is part of the split projection
-        KvaPackArgs ka{kpart ? ypart + d.QO : ykva, wnorm, cs, lath, latl, qh, ql8, kh, k8, vt,
-                       kpart ? (size_t)S * ldq : (size_t)S * d.KVO, kpart ? ks : np,
-                       S, Sp, d.NH, kpart ? ldq : d.KVO, d.R, d.DN, d.DR, d.DV, eps, flags + 0,
-                       ks > 1 ? ypart : nullptr, (size_t)S * ldq, ks, ldq, vpad, ep};
-        const int qblocks = ks > 1 ? (int)(((size_t)S * (d.QO / 4) + 255) / 256) : 0;
-        hipLaunchKernelGGL(k_kva_pack, dim3((S + 3) / 4 + vpad + qblocks), dim3(256), 0, st, ka);
+        const int vpad = Sp > S ? (d.NH * d.DV + 63) / 64 : 0;
+        KvaPackArgs ka{ykva, wnorm, cs, lath, latl, kh, k8, vt, (size_t)S * d.KVO, np,
+                       S, Sp, d.NH, d.KVO, d.R, d.DN, d.DR, d.DV, eps, flags + 0};
+        hipLaunchKernelGGL(k_kva_pack, dim3((S + 3) / 4 + vpad), dim3(256), 0, st, ka);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         // kv_b (-> K nope part as fp16 hi + K8, V^T scaled by vscale)
         ep.vscale = vscale;

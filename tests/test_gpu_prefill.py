@@ -235,6 +235,22 @@ def test_prefill_sizes_agree_with_a_longer_prompt(S, bf16_x):
     assert np.all(a[S] == 7.0)
 
 
+@pytest.mark.parametrize("S,bf16_x", [(1, False), (16, True), (31, False), (37, False), (37, True), (64, False),
+                                      (65, False), (96, True), (100, False), (128, False), (129, True), (160, False),
+                                      (161, False), (250, False), (700, False), (2048, False), (2049, True)])
+def test_prefill_is_a_prefix_of_a_longer_prompt(S, bf16_x):
+    """Every stage sums a token in one order whatever the prompt's length, so the outputs of S tokens
+    are the first S outputs of 4096 tokens bit for bit: at the edges of the projection's tile shapes (64
+    and 128 tokens from fp32 x, 64 and 160 from the planes), of attention with 64 and 128 queries a block
+    (2048), and in between."""
+    full, x, layer = long_prefill(bf16_x)
+    cfg = inputs.config(**inputs.KIMI)
+    w = layer.struct()
+    a = np.zeros((S, cfg.hidden_size), np.float32)
+    lib.check(L.kvl_mla_prefill_bf16(f32(a), f32(np.ascontiguousarray(x[:S])), S, C.byref(cfg), C.byref(w)), "prefill")
+    np.testing.assert_array_equal(a, full[:S])
+
+
 @pytest.mark.parametrize("S", [5, 37, 64, 100, 128, 129, 250])
 def test_short_prefill_from_an_unaligned_buffer(S):
     """A short prompt's projections read fp32 x as it is when it is 16-byte aligned and through its bf16
