@@ -457,8 +457,7 @@ enum { kTile64x64 = 0, kTile128x64, kTile128x128, kTile192x128, kTile256x128, kT
 // follow it (k split over 4 blocks, its sums added by k_kva_pack, gave 30.2 us for 37 tokens in all where
 // this gives 35.3, and lost that). A block's time is the serial chain of its 64 k-subs (LDS reads, splits,
 // MFMAs; stages of 128 or 256 k change nothing), so the smallest tile that still gives every tile a CU
-// runs. us with weights in
-// the caches / from memory, 32 x 32, 32 x 64, 64 x 64 (tokens x columns, two blocks a CU):
+// runs. us with weights in the caches / from memory, 32 x 32, 32 x 64, 64 x 64 (tokens x columns):
 //   fp32 x, q | kv_a   37: 11.3 / 15.0  13.5 / 17.8  14.5 / 21.7   128: 19.7 / 23.2  14.3 / 20.4  15.5 / 23.9
 //   planes, q alone    37:  7.7 / 14.5   9.8 / 17.5  11.0 / 22.2   160: 13.7 / 20.9  13.1 / 19.8  13.9 / 23.8
 //   fp32 x, q | kv_a  160: 27.7 / 31.2  24.3 / 28.5  15.8 / 24.1

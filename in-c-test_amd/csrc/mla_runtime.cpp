@@ -973,7 +973,7 @@ int prepare_groups(int fmt, const Dims &d, float theta, S *const *states, int B,
 }
 
 // Norm of the inputs of a decode group: x is n = RMSNorm(d_x, w) instead of d_x. buf: a group's
-// rows [<= kMaxBatch, H], used where the projection does not normalise its operand itself.
+// rows [<= kMaxBatch, H], 16-byte aligned, used where the projection does not normalise its operand itself.
 struct InNorm {
     const uint16_t *w;
     float *buf;
@@ -1030,10 +1030,12 @@ int decode_group(int fmt, const Dims &d, float eps, float theta, const DevWeight
     const bool fuse_base = c.fq_on && fmt == kFmtQ8 && kind == kAttnQ8Mfma && !solo && part_cap == 0 &&
                            kimi_attn(d) && d.DN == 128 && d.QD == 192 && gemv_ksplit_ok(d.H, d.H) && ukt_shape(d) &&
                            dw.ukt && 17 * B <= total_splits && total_splits <= c.ncu && c.fq_flags && c.fq_err;
-    // ... and the q_proj | kv_a projection inside it too (fq_gemv): at most eight sequences, x
-    // 16-byte aligned, a launch of max(splits, kGemvTasks) <= CU count workgroups.
+    // ... and the q_proj | kv_a projection inside it too (fq_gemv): at most eight sequences, a launch
+    // of max(splits, kGemvTasks) <= CU count workgroups, an input with 16-byte aligned rows (a norm's
+    // launch gives one whatever the caller's buffer).
+    const bool x16 = ((uintptr_t)d_x % 16) == 0;
     const bool pfuse_ok = fuse_base && c.gemv_on && gemv_fuse_ok(d, B) && gemv_ksplit_ok(d.H, d.H) &&
-                          ((uintptr_t)d_x % 16) == 0 && std::max(total_splits, kGemvTasks) <= c.ncu;
+                          (x16 || in_norm) && std::max(total_splits, kGemvTasks) <= c.ncu;
     // ... and the combine inside it (q8_comb_tail): eight sequences (or a multiple) with equal
     // split counts, each sequence's splits on one XCD (kCombXcd); or sequences of 16 or more
     // splits each, their partials exchanged past the L2s (kCombCross). Measured (headline
@@ -1046,7 +1048,7 @@ int decode_group(int fmt, const Dims &d, float eps, float theta, const DevWeight
     const bool fuse = fuse_base && (B >= 2 || (pfuse_ok && comb_mode != 0));
     const bool pfuse = fuse && pfuse_ok;
     const int comb = fuse ? comb_mode : 0;
-    const bool norm_inside = in_norm && pfuse && comb == 1;  // the projection tasks normalise x (FqArgs::xnorm)
+    const bool norm_inside = in_norm && x16 && pfuse && comb == 1;  // the projection tasks normalise x (FqArgs::xnorm)
     if (in_norm && !norm_inside) {
         HIP_TRY(launch_rmsnorm(st, in_norm->buf, d_x, in_norm->w, d.H, B, eps));
         d_x = in_norm->buf;

@@ -175,3 +175,52 @@ def test_layer_norm_inside_the_projection_equals_its_launch(lens):
     for s in states:
         L.kvl_mla_compressed_q8_state_free(C.byref(s))
     lib.check(L.kvl_mla_release_weights(C.byref(w)), "release")
+
+
+@pytest.mark.parametrize("lens", [[8300], [6000] * 8, [7000, 5100, 9000]], ids=["1", "8", "3"])
+def test_layer_from_an_unaligned_buffer_keeps_the_fused_launch(lens):
+    """The projection inside the attention launch reads 16-byte vectors. Hidden states at a 4-byte
+    boundary go through the norm's launch into the library's aligned buffer and keep that form: no launch
+    of the projection (stage 0) is timed, and h and n2 equal those of an aligned buffer bit for bit."""
+    cfg = inputs.config(**KIMI)
+    H, B = cfg.hidden_size, len(lens)
+    layer = inputs.make_layer(cfg, 0xAB)
+    w = layer.struct()
+    lib.check(L.kvl_mla_bind_weights(C.byref(cfg), C.byref(w)), "bind")
+    norms = [inputs.normal_bf16(0xAB, n, (H,), mean=1.0, std=0.1) for n in ("n1", "n2")]
+    h0 = np.ascontiguousarray(inputs.hidden(cfg, 0xAC, B))
+    states = []
+    for i, n in enumerate(lens):
+        st = abi.KvlMlaCompressedQ8State()
+        lib.check(L.kvl_mla_compressed_q8_state_init(C.byref(st), C.byref(cfg), n + 1), "init")
+        lib.check(L.kvl_mla_compressed_q8_state_fill_synthetic(C.byref(st), 0, n, 0xAC0 + i), "fill")
+        states.append(st)
+    arr = (C.POINTER(abi.KvlMlaCompressedQ8State) * B)(*[C.pointer(s) for s in states])
+    nb = h0.nbytes
+    base, d_n2 = L.kvl_mla_device_alloc(nb + 16), L.kvl_mla_device_alloc(nb)
+    got = []
+    for off in (0, 4):
+        d_h = base + off
+        lib.check(L.kvl_mla_copy_to_device(d_h, h0.ctypes.data, nb), "h2d")
+        ms, count = (C.c_double * 6)(), (C.c_int * 6)()
+        lib.check(L.kvl_mla_timing_enable(1), "timing on")
+        try:
+            lib.check(L.kvl_mla_attention_layer_q8_device(d_h, d_n2, B, C.byref(cfg), C.byref(w), u16(norms[0]),
+                                                          u16(norms[1]), arr, lib.NO_ADVANCE), "layer")
+            lib.check(L.kvl_mla_timing_read(ms, count), "timing read")
+        finally:
+            lib.check(L.kvl_mla_timing_enable(0), "timing off")
+        h, n2 = np.zeros_like(h0), np.zeros_like(h0)
+        lib.check(L.kvl_mla_copy_to_host(h.ctypes.data, d_h, nb), "d2h")
+        lib.check(L.kvl_mla_copy_to_host(n2.ctypes.data, d_n2, nb), "d2h")
+        got.append((h, n2))
+        print(f"[layer] offset {off}: launches per stage {list(count)}", flush=True)
+        assert count[0] == 0 and count[3] == 1, (off, list(count))
+    for a, b in zip(*got):
+        assert np.all(np.isfinite(a)) and np.any(a)
+        np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
+    L.kvl_mla_device_free(base)
+    L.kvl_mla_device_free(d_n2)
+    for s in states:
+        L.kvl_mla_compressed_q8_state_free(C.byref(s))
+    lib.check(L.kvl_mla_release_weights(C.byref(w)), "release")
