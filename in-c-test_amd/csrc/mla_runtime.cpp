@@ -165,6 +165,7 @@ struct Ctx {
     std::unordered_map<uint64_t, RopeTable> ropes;  // key: theta bits << 16 | DR
     DevBuf work, part, scores, prefill, fill, fillx, layer, sink;
     DevBuf wmax;   // unsigned: result of a weight range reduction
+    hipStream_t side = nullptr;  // weight range reductions: their result is waited for, other work is not
     DevBuf rflag;  // int: raised by a stream-ordered prefill outside the MFMA route's range
     PinBuf pin_in, pin_out;
     hipEvent_t stage_ev[2] = {nullptr, nullptr};  // host-buffer prefills: marks in their copies out
@@ -416,15 +417,18 @@ float bf16_abs(uint16_t b) {
     return f;
 }
 
-// A range reduction over weights on the device (launch_bf16_absmax, launch_vrow_l2max) and its result.
+// A range reduction over uploaded weights on the device (launch_bf16_absmax, launch_vrow_l2max) and its
+// result. On a stream of its own: the uploads have ended (blocking copies), and a stream-ordered call
+// must not wait for the work queued before it on the library stream.
 template <class F>
 int weight_max(F launch, unsigned *res) {
     Ctx &c = ctx();
+    if (!c.side) HIP_TRY(hipStreamCreateWithFlags(&c.side, hipStreamNonBlocking));
     if (dev_reserve(c.wmax, 256) != 0) return -1;
-    HIP_TRY(hipMemsetAsync(c.wmax.p, 0, sizeof(unsigned), c.stream));
-    HIP_TRY(launch((unsigned *)c.wmax.p));
-    HIP_TRY(hipMemcpyAsync(res, c.wmax.p, sizeof(unsigned), hipMemcpyDeviceToHost, c.stream));
-    HIP_TRY(hipStreamSynchronize(c.stream));
+    HIP_TRY(hipMemsetAsync(c.wmax.p, 0, sizeof(unsigned), c.side));
+    HIP_TRY(launch(c.side, (unsigned *)c.wmax.p));
+    HIP_TRY(hipMemcpyAsync(res, c.wmax.p, sizeof(unsigned), hipMemcpyDeviceToHost, c.side));
+    HIP_TRY(hipStreamSynchronize(c.side));
     return 0;
 }
 
@@ -444,7 +448,7 @@ int dev_weight_f16(const uint16_t *host, size_t elems, const _Float16 **out, int
             return -1;
         }
         unsigned mxw = 0;
-        if (weight_max([&](unsigned *r) { return launch_bf16_absmax(c.stream, d16, elems, r); }, &mxw) != 0) return -1;
+        if (weight_max([&](hipStream_t st, unsigned *r) { return launch_bf16_absmax(st, d16, elems, r); }, &mxw) != 0) return -1;
         const float mx = bf16_abs((uint16_t)mxw);
         int ex = 0;
         e.f16_shift = 0;
@@ -465,16 +469,19 @@ int dev_weight_f16(const uint16_t *host, size_t elems, const _Float16 **out, int
 // |v| = |kv_b_row . latent| <= ||kv_b_row||_2 ||latent||_2 with ||latent||_2 <= sqrt(R)
 // max|kv_a_norm| (an RMSNorm output has ||x / rms(x)||_2 <= sqrt(R)), the scale puts the
 // bound below 2^14 (the fp16 maximum is 65504).
-float prefill_vscale(const KvlMlaBF16 *w, const Dims &d) {
+int prefill_vscale(const KvlMlaBF16 *w, const Dims &d, float *scale) {
     Ctx &c = ctx();
+    *scale = 1.0f;
     auto it = c.weights.find(w->kv_b_proj);
-    if (it == c.weights.end()) return 1.0f;
+    if (it == c.weights.end()) return 0;
     WeightEntry &e = it->second;
-    unsigned l2w = 0;
-    if (e.row_l2max < 0.f && !c.capturing &&
-        weight_max([&](unsigned *r) { return launch_vrow_l2max(c.stream, (const uint16_t *)e.dev, d, r); }, &l2w) == 0)
+    if (e.row_l2max < 0.f && !c.capturing) {
+        unsigned l2w = 0;
+        if (weight_max([&](hipStream_t st, unsigned *r) { return launch_vrow_l2max(st, (const uint16_t *)e.dev, d, r); },
+                       &l2w) != 0)
+            return -1;
         memcpy(&e.row_l2max, &l2w, sizeof l2w);
-    if (e.row_l2max < 0.f) {  // during a graph capture (nothing can be read back), from the host array
+    } else if (e.row_l2max < 0.f) {  // during a graph capture (nothing can be read back), from the host array
         double mx = 0.0;
         for (int h = 0; h < d.NH; ++h)
             for (int r = 0; r < d.DV; ++r) {
@@ -491,10 +498,11 @@ float prefill_vscale(const KvlMlaBF16 *w, const Dims &d) {
     float nmax = 0.f;
     for (int k = 0; k < d.R; ++k) nmax = std::max(nmax, bf16_abs(w->kv_a_norm[k]));
     const double bound = 1.001 * sqrt((double)d.R) * (double)nmax * (double)e.row_l2max;
-    if (!(bound > 0.0) || !std::isfinite(bound)) return 1.0f;
+    if (!(bound > 0.0) || !std::isfinite(bound)) return 0;
     int ex = 0;
     (void)frexp(bound, &ex);  // bound < 2^ex
-    return ldexpf(1.0f, std::min(100, std::max(-100, 14 - ex)));
+    *scale = ldexpf(1.0f, std::min(100, std::max(-100, 14 - ex)));
+    return 0;
 }
 
 // W_UK^T of a kv_b array in MFMA fragment order (transposed on the device from its bf16 copy,
@@ -1688,7 +1696,7 @@ int prefill_device(float *d_out, const float *d_x, int S, const KvlMlaConfig *cf
         int shift = 0;
         if (dev_weight_f16(w->o_proj, (size_t)d.H * d.HO, &wo16, &shift) != 0) return -1;
         range.oscale = ldexpf(1.0f, shift);
-        range.vscale = prefill_vscale(w, d);
+        if (prefill_vscale(w, d, &range.vscale) != 0) return -1;
         if (!host_call) {
             if (!c.rflag.p) {
                 if (c.capturing) {

@@ -1,6 +1,7 @@
 """Parity of the causal prefill (C ABI kvl_mla_prefill_bf16) with the oracle's restatement of
 src/mla_prefill_streaming.c:78-206. Bar: max|got - ref| / max|ref| <= 2e-3."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -291,3 +292,42 @@ def test_prefill_scale_leaves_out_nan_weights():
     keep = np.arange(cfg.hidden_size) != 7
     assert np.all(np.isfinite(out[0])) and np.all(np.isnan(out[1][:, 7]))
     np.testing.assert_array_equal(out[0][:, keep].view(np.uint32), out[1][:, keep].view(np.uint32))
+
+
+def test_first_prefill_of_bound_weights_does_not_wait_for_queued_work():
+    """A stream-ordered prefill returns after enqueueing, also the first one with a layer's weights, whose
+    operand ranges are reduced on the device and read back. Behind about 50 ms of queued prefills of
+    another layer it returns while most of them are still to run; the output is that of a later call."""
+    cfg = inputs.config(**inputs.KIMI)
+    busy, fresh = inputs.make_layer(cfg, 0xCE), inputs.make_layer(cfg, 0xCF)
+    wb, wf = busy.struct(), fresh.struct()
+    S, n = 8192, 60
+    x = inputs.hidden(cfg, 0xCE, S)
+    dx, do, d2 = (L.kvl_mla_device_alloc(x.nbytes) for _ in range(3))
+    lib.check(L.kvl_mla_copy_to_device(dx, x.ctypes.data, x.nbytes), "h2d")
+    for w in (wb, wf):
+        lib.check(L.kvl_mla_bind_weights(C.byref(cfg), C.byref(w)), "bind")
+    lib.check(L.kvl_mla_prefill_device(do, dx, S, C.byref(cfg), C.byref(wb)), "warm")
+    lib.check(L.kvl_mla_synchronize(), "sync")
+    for _ in range(n):
+        lib.check(L.kvl_mla_prefill_device(do, dx, S, C.byref(cfg), C.byref(wb)), "queue")
+    t0 = time.perf_counter()
+    lib.check(L.kvl_mla_prefill_device(d2, dx, 64, C.byref(cfg), C.byref(wf)), "first")
+    t1 = time.perf_counter()
+    lib.check(L.kvl_mla_synchronize(), "sync")
+    t2 = time.perf_counter()
+    print(f"[prefill] first call {1e3 * (t1 - t0):.2f} ms, the queue behind it {1e3 * (t2 - t1):.2f} ms", flush=True)
+    assert t1 - t0 < t2 - t1
+    got = []
+    for again in (False, True):
+        if again:
+            lib.check(L.kvl_mla_prefill_device(d2, dx, 64, C.byref(cfg), C.byref(wf)), "later")
+        a = np.zeros((64, cfg.hidden_size), np.float32)
+        lib.check(L.kvl_mla_copy_to_host(a.ctypes.data, d2, a.nbytes), "d2h")
+        got.append(a)
+    assert np.all(np.isfinite(got[0])) and np.any(got[0])
+    np.testing.assert_array_equal(got[0], got[1])
+    for w in (wb, wf):
+        lib.check(L.kvl_mla_release_weights(C.byref(w)), "release")
+    for p in (dx, do, d2):
+        L.kvl_mla_device_free(p)
