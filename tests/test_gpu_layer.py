@@ -132,11 +132,14 @@ def test_attention_layer_rejects_bad_arguments():
     L.kvl_mla_compressed_q8_state_free(C.byref(st))
 
 
-@pytest.mark.parametrize("lens", [[8300], [6000] * 8, [7000, 5100, 9000]], ids=["1", "8", "3"])
+@pytest.mark.parametrize("lens", [[6000] * 8, [5950, 6000, 6010, 6050, 6090, 6120, 6130, 6150], [8300], [7000, 5100, 9000]],
+                         ids=["8", "8-lengths", "1", "3"])
 def test_layer_norm_inside_the_projection_equals_its_launch(lens):
-    """Q8 decodes whose projection runs inside the attention launch normalise their input there; with
-    the projection in its own launch the norm is a launch too. Same sums in the same order: h and n2
-    are equal bit for bit, from hidden states of very different scale per sequence."""
+    """Eight sequences with equal split counts (24 of 256 rows here, also for the eight different lengths)
+    have their projection and their combine inside the attention launch, which then normalises its input
+    too; with the projection in its own launch the norm is a launch. Same sums in the same order: h and n2
+    are equal bit for bit, from hidden states of very different scale per sequence. One and three sequences
+    keep the norm's launch in both forms."""
     cfg = inputs.config(**KIMI)
     H, B = cfg.hidden_size, len(lens)
     layer = inputs.make_layer(cfg, 0xA7)

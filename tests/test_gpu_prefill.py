@@ -220,10 +220,11 @@ def long_prefill(bf16_x):
                                       (257, False), (385, False), (513, False), (700, True), (897, False), (1025, False),
                                       (1181, False), (1537, True), (2049, False), (3000, False)])
 def test_prefill_sizes_agree_with_a_longer_prompt(S, bf16_x):
-    """Every tile shape of the three GEMMs at its edges: attention is causal, so the first S outputs
-    of the 4096-token prefill (whose tiles are checked against the oracle above) are those of the
-    S-token one, up to fp32 summation order and its fp16 roundings. Each side is within 3.5e-4 of
-    the oracle where it was measured, so the two are within 1e-3 of each other."""
+    """Sizes on both sides of the limits between the GEMMs' tile shapes, up to 3000 tokens, and one output
+    row past the last that stays untouched. Attention is causal, so the first S outputs of the 4096-token
+    prefill (checked against the oracle above) are those of the S-token one. Each side is within 3.5e-4
+    of the oracle where it was measured, so the two are within 1e-3 of each other; the test below asks
+    for equal bits."""
     full, x, layer = long_prefill(bf16_x)
     cfg = inputs.config(**inputs.KIMI)
     w = layer.struct()
@@ -238,18 +239,74 @@ def test_prefill_sizes_agree_with_a_longer_prompt(S, bf16_x):
 
 @pytest.mark.parametrize("S,bf16_x", [(1, False), (16, True), (31, False), (37, False), (37, True), (64, False),
                                       (65, False), (96, True), (100, False), (128, False), (129, True), (160, False),
-                                      (161, False), (250, False), (700, False), (2048, False), (2049, True)])
+                                      (161, False), (250, False), (300, False), (520, False), (700, False),
+                                      (1181, False), (1600, False), (2048, False), (2049, True), (2500, False),
+                                      (3500, False)])
 def test_prefill_is_a_prefix_of_a_longer_prompt(S, bf16_x):
     """Every stage sums a token in one order whatever the prompt's length, so the outputs of S tokens
-    are the first S outputs of 4096 tokens bit for bit: at the edges of the projection's tile shapes (64
-    and 128 tokens from fp32 x, 64 and 160 from the planes), of attention with 64 and 128 queries a block
-    (2048), and in between."""
+    are the first S outputs of 4096 tokens bit for bit: at the edges of the short projection's tile
+    shapes (64 and 128 tokens), of attention with 64 and 128 queries a block (2048), and, for every
+    larger tile shape of the three GEMMs that a prompt below 4096 tokens takes, at a size that leaves its
+    last row of tiles ragged."""
     full, x, layer = long_prefill(bf16_x)
     cfg = inputs.config(**inputs.KIMI)
     w = layer.struct()
     a = np.zeros((S, cfg.hidden_size), np.float32)
     lib.check(L.kvl_mla_prefill_bf16(f32(a), f32(np.ascontiguousarray(x[:S])), S, C.byref(cfg), C.byref(w)), "prefill")
     np.testing.assert_array_equal(a, full[:S])
+
+
+@pytest.mark.parametrize("S", [4500, 6200])
+def test_prefill_longer_than_4096(S):
+    """Ragged prompts of the tile shapes that start above 4096 tokens: 192 x 128 in all three GEMMs (4500),
+    o_proj in 256 x 256 tiles with two 64-deep stages (from 6145 tokens). The first 4096 outputs equal the
+    4096-token prompt's bit for bit; the others are checked against the oracle on rows at the edges of the
+    last tiles."""
+    full, x, layer = long_prefill(False)
+    cfg = inputs.config(**inputs.KIMI)
+    w = layer.struct()
+    xs = np.concatenate([x, inputs.hidden(cfg, 0xD0, S - 4096)])
+    a = np.zeros_like(xs)
+    lib.check(L.kvl_mla_prefill_bf16(f32(a), f32(xs), S, C.byref(cfg), C.byref(w)), "prefill")
+    np.testing.assert_array_equal(a[:4096], full)
+    rows = [4096, 4223, 4351, 4352, S // 256 * 256 - 1, S // 256 * 256, S // 192 * 192, S - 2, S - 1]
+    idx = np.ascontiguousarray(sorted(set(rows)), dtype=np.int32)
+    ref = np.zeros((len(idx), cfg.hidden_size), np.float32)
+    assert ORC.orc_mla_prefill_streaming_rows(f32(ref), f32(xs), S, idx.ctypes.data_as(C.POINTER(C.c_int)),
+                                              len(idx), C.byref(cfg), C.byref(w)) == 0
+    e = rel_err(a[idx], ref)
+    print(f"[prefill] S={S}, {len(idx)} rows vs oracle {e:.3e}", flush=True)
+    assert np.all(np.isfinite(a)) and e <= TOL, e
+
+
+@pytest.mark.parametrize("S", [1, 37, 64, 65, 100, 129, 250])
+def test_prefill_after_a_call_that_left_nan_in_the_workspace(S):
+    """Padding rows of Q, K and K8 are not cleared: the causal mask sets their scores whatever they hold.
+    A 512-token prompt of NaN leaves NaN in every operand of the workspace; the next call gives the same
+    bits as before it."""
+    cfg = inputs.config(**inputs.KIMI)
+    layer = inputs.make_layer(cfg, 0xD1)
+    w = layer.struct()
+    x = inputs.hidden(cfg, 0xD1, S)
+    bad = np.full((512, cfg.hidden_size), np.nan, np.float32)
+    dx, do, db = (L.kvl_mla_device_alloc(bad.nbytes) for _ in range(3))
+    lib.check(L.kvl_mla_copy_to_device(dx, x.ctypes.data, x.nbytes), "h2d")
+    lib.check(L.kvl_mla_copy_to_device(db, bad.ctypes.data, bad.nbytes), "h2d")
+    assert L.kvl_mla_prefill_range_status() == 0
+    got = []
+    for spoil in (False, True):
+        if spoil:
+            lib.check(L.kvl_mla_prefill_device(do, db, 512, C.byref(cfg), C.byref(w)), "NaN prefill")
+            assert L.kvl_mla_prefill_range_status() == 1
+        lib.check(L.kvl_mla_prefill_device(do, dx, S, C.byref(cfg), C.byref(w)), "prefill")
+        a = np.zeros_like(x)
+        lib.check(L.kvl_mla_copy_to_host(a.ctypes.data, do, a.nbytes), "d2h")
+        got.append(a)
+    assert L.kvl_mla_prefill_range_status() == 0
+    assert np.all(np.isfinite(got[0])) and np.any(got[0])
+    np.testing.assert_array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    for p in (dx, do, db):
+        L.kvl_mla_device_free(p)
 
 
 @pytest.mark.parametrize("S", [5, 37, 64, 100, 128, 129, 250])

@@ -27,8 +27,10 @@ STREAM = dict(hidden_size=16, num_heads=2, qk_nope_dim=4, qk_rope_dim=4, v_head_
 KIMI = dict(inputs.KIMI)
 
 STATE = {"f32": (abi.KvlMlaCompressedState, "mla_compressed_state"),
+         "bf16": (abi.KvlMlaCompressedBF16State, "mla_compressed_bf16_state"),
          "q8": (abi.KvlMlaCompressedQ8State, "mla_compressed_q8_state")}
-FUSED = {"f32": "mla_prefill_compressed_state", "q8": "mla_prefill_compressed_q8_state"}
+FUSED = {"f32": "mla_prefill_compressed_state", "bf16": "mla_prefill_compressed_bf16_state",
+         "q8": "mla_prefill_compressed_q8_state"}
 
 
 def new_state(api, kind, cfg, cap):
@@ -242,3 +244,136 @@ def test_prefilled_special_rows_equal_decoded_rows(kind):
         if name == "rope" and kind == "q8":
             a, b = (inputs.bf16_bits_to_f32(v) for v in (a, b))
         np.testing.assert_array_equal(a, b, err_msg=f"{kind} {name}")
+
+
+def rows_of(kind, st, cfg):
+    """The host rows [0, len), bit patterns."""
+    n = st.len
+    if kind != "bf16":
+        return snapshot(kind, st, cfg)
+    return {"latent": np.ctypeslib.as_array(st.latent, (n, cfg.kv_lora_rank)).copy(),
+            "rope": np.ctypeslib.as_array(st.rope, (n, cfg.qk_rope_dim)).copy()}
+
+
+def fused_device(kind, cfg, w, x):
+    """Output and pulled rows of the device call."""
+    S, nbytes = x.shape[0], x.nbytes
+    st = new_state(G, kind, cfg, S)
+    dx, do = L.kvl_mla_device_alloc(nbytes), L.kvl_mla_device_alloc(nbytes)
+    lib.check(L.kvl_mla_copy_to_device(dx, x.ctypes.data, nbytes), "h2d")
+    lib.check(getattr(G, FUSED[kind] + "_device")(do, dx, S, C.byref(cfg), C.byref(w), C.byref(st)), "fused device")
+    out = np.zeros_like(x)
+    lib.check(L.kvl_mla_copy_to_host(out.ctypes.data, do, nbytes), "d2h")
+    lib.check(getattr(G, STATE[kind][1] + "_pull")(C.byref(st), 0, S), "pull")
+    rows = rows_of(kind, st, cfg)
+    free_state(G, kind, st)
+    L.kvl_mla_device_free(dx)
+    L.kvl_mla_device_free(do)
+    return out, rows
+
+
+def state_rows(kind, cfg, w, x):
+    """Rows of the state prefill alone."""
+    st = new_state(G, kind, cfg, x.shape[0])
+    lib.check(getattr(G, STATE[kind][1] + "_prefill_bf16")(f32(x), x.shape[0], C.byref(cfg), C.byref(w), C.byref(st)),
+              "state prefill")
+    rows = rows_of(kind, st, cfg)
+    free_state(G, kind, st)
+    return rows
+
+
+_long_fill = {}
+
+
+def long_fill():
+    """Layer, input, output and FP32 rows of a 4500-token prefill with state fill, computed once: its output
+    against the plain prefill's (see test_fused_equals_prefill_then_state_prefill), its rows against the
+    state prefill's."""
+    if not _long_fill:
+        cfg = inputs.config(**KIMI)
+        layer = inputs.make_layer(cfg, 0xDB)
+        w = layer.struct()
+        x = inputs.hidden(cfg, 0xDB, 4500)
+        out, rows = fused_device("f32", cfg, w, x)
+        plain = np.zeros_like(x)
+        lib.check(L.kvl_mla_prefill_bf16(f32(plain), f32(x), 4500, C.byref(cfg), C.byref(w)), "prefill")
+        assert np.all(np.isfinite(out)) and rel_err(out, plain) <= 5e-4, rel_err(out, plain)
+        assert_snap_equal(rows, state_rows("f32", cfg, w, x))
+        _long_fill.update(layer=layer, x=x, out=out, rows=rows)
+    return _long_fill
+
+
+@pytest.mark.parametrize("S", [1, 37, 64, 65, 128, 160, 161, 321, 650, 705, 1000, 1025, 1281, 1921, 2600, 4097])
+def test_fill_is_a_prefix_of_a_longer_one(S):
+    """The projection without kv_a, whose tile shapes change at other sizes than the plain prefill's (64, 160,
+    320, 640, 704, 1280, 1920, 2560 and 4096 tokens): outputs and rows of S tokens are the first S of 4500
+    bit for bit, through the device call and through the host call, which is staged through pinned memory
+    up to 1024 tokens."""
+    ref = long_fill()
+    cfg = inputs.config(**KIMI)
+    w = ref["layer"].struct()
+    x = np.ascontiguousarray(ref["x"][:S])
+    out, rows = fused_device("f32", cfg, w, x)
+    host, st = fused("f32", cfg, w, x, S)
+    for o, r in ((out, rows), (host, snapshot("f32", st, cfg))):
+        np.testing.assert_array_equal(o, ref["out"][:S])
+        for k in r:
+            np.testing.assert_array_equal(r[k], ref["rows"][k][:S], err_msg=k)
+    free_state(G, "f32", st)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "q8"])
+@pytest.mark.parametrize("S", [1000, 1100])
+def test_fused_host_call_on_both_sides_of_the_staging_limit(kind, S):
+    """1000 tokens go through pinned memory, 1100 do not: outputs and rows equal the device call's."""
+    ref = long_fill()
+    cfg = inputs.config(**KIMI)
+    w = ref["layer"].struct()
+    x = np.ascontiguousarray(ref["x"][:S])
+    host, st = fused(kind, cfg, w, x, S)
+    out, rows = fused_device(kind, cfg, w, x)
+    np.testing.assert_array_equal(host, out)
+    assert_snap_equal(rows_of(kind, st, cfg), rows)
+    free_state(G, kind, st)
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16", "q8"])
+def test_long_fill_rows(kind):
+    """8197 rows: four to a block, so more than the 2048 blocks that the rows kernel launches."""
+    cfg = inputs.config(**KIMI)
+    layer = inputs.make_layer(cfg, 0xDC)
+    w = layer.struct()
+    x = inputs.hidden(cfg, 0xDC, 8197)
+    out, rows = fused_device(kind, cfg, w, x)
+    assert np.all(np.isfinite(out))
+    assert_snap_equal(rows, state_rows(kind, cfg, w, x))
+
+
+@pytest.mark.parametrize("S", [256, 1100])
+def test_fused_host_call_beyond_the_operand_range(S):
+    """kv_b x 3000 raises the range flag (row-max logits of about 4400): the host call, staged through pinned
+    memory (256) or not (1100), computes the output again on the fp32 route and keeps the rows, which do
+    not depend on the attention."""
+    cfg = inputs.config(**KIMI)
+    layer = inputs.make_layer(cfg, 0xDD)
+    layer.kv_b_proj[...] = inputs.f32_to_bf16_bits(inputs.bf16_bits_to_f32(layer.kv_b_proj) * np.float32(3000.0))
+    w = layer.struct()
+    x = inputs.hidden(cfg, 0xDD, S, bf16_exact=True)
+    out, st = fused("q8", cfg, w, x, S)
+    idx = np.ascontiguousarray(sorted({0, 1, S // 2, S - 2, S - 1}), dtype=np.int32)
+    ref = np.zeros((len(idx), cfg.hidden_size), np.float32)
+    assert ORC.orc_mla_prefill_streaming_rows(f32(ref), f32(x), S, idx.ctypes.data_as(C.POINTER(C.c_int)), len(idx),
+                                              C.byref(cfg), C.byref(w)) == 0
+    e = rel_err(out[idx], ref)
+    print(f"[fused] range S={S}: {e:.3e}", flush=True)
+    assert np.all(np.isfinite(out)) and e <= TOL, e
+    assert L.kvl_mla_prefill_range_status() == 0
+    assert st.len == S
+    assert_snap_equal(rows_of("q8", st, cfg), state_rows("q8", cfg, w, x))
+    dx, do = L.kvl_mla_device_alloc(x.nbytes), L.kvl_mla_device_alloc(x.nbytes)
+    lib.check(L.kvl_mla_copy_to_device(dx, x.ctypes.data, x.nbytes), "h2d")
+    lib.check(L.kvl_mla_prefill_device(do, dx, S, C.byref(cfg), C.byref(w)), "device prefill")
+    assert L.kvl_mla_prefill_range_status() == 1  # the flag was up
+    L.kvl_mla_device_free(dx)
+    L.kvl_mla_device_free(do)
+    free_state(G, "q8", st)
