@@ -611,7 +611,8 @@ hipError_t launch_gemv_xs(hipStream_t st, float *Y, int ldy, const uint16_t *XS,
         (B + 15) / 16 > 65535)
         return hipErrorInvalidValue;
     // 16-token groups of a block: one up to 32 tokens, two in turn beyond (a block's weights serve
-    // both): two / one 12.0 / 10.3 us at 17 tokens, 14.2 / 10.5 at 32, 14.5 / 15.9 at 48 (cold weights)
+    // both). Decodes of 12 layers in turn, kernel trace, two / one group a block (us): 9.7 / 8.0 at 17
+    // sequences, 10.1 / 7.7 at 20, 10.8 / 8.0 at 24, 12.2 / 7.7 at 32; at 48, alone, 14.5 / 15.9
     const dim3 grid((out + 15) / 16, 1, B <= 32 ? (B + 15) / 16 : (B + 31) / 32);
     const bool two = B > 8;
     if (in == 2048) {

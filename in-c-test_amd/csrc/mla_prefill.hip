@@ -437,12 +437,16 @@ __global__ __launch_bounds__(Sh::Threads, (Sh::MW + kGemmDma) / 4 * Sh::BPC) voi
 // its blocks, so the shape with the smallest rounds x time per round runs. Below a few hundred
 // tokens a large tile leaves most CUs idle and a block's time is the latency of its k loop, which
 // small tiles hide with deeper rings; above a few thousand the bytes a CU takes in per MFMA decide
-// for the large ones. Measured time per round in us (stand-alone launches, K = 2048 for q | kv_a
-// and o_proj, 512 for kv_b); tokens -> us of the chosen shape, in brackets that of the 256-row
+// for the large ones. The times per round (gemm_pick) are of q | kv_a and kv_b launches with the lo
+// part: whether x has one is known on the device only. Stand-alone launches back to back (K = 2048 for
+// q | kv_a and o_proj, 512 for kv_b), tokens -> us of the chosen shape, in brackets that of the 256-row
 // tiles with two passes over k that every size took before:
-//   q | kv_a  37: 11.4 (46)  250: 15.5 (50)  1181: 45 (55)  4096: 106 (134)  16000: 405
-//   kv_b      37: 5.6 (17)   250: 6.1 (21)   1181: 19 (24)  4096: 43 (50)    16000: 166 (171)
-//   o_proj    37: 8.2 (24)   250: 8.8 (24)   1181: 19 (27)  4096: 33 (38)    16000: 109 (118)
+//   q | kv_a  250: 15.3 (50)  1181: 44 (55)  4096: 108 (134)  16000: 415, without a lo part 13.3, 35, 67, 257
+//   kv_b      250: 5.6 (21)   1181: 18 (24)  4096: 41 (50)    16000: 151 (171)
+//   o_proj    250: 8.1 (24)   1181: 18 (27)  4096: 34 (38)    16000: 117 (118)
+// Without a lo part the choice is within a tenth of the best shape but for q alone at 2561 to 4096 tokens
+// (128 x 128: 97 us with, 70 without a lo part at 4096; 256 x 256: 101 and 61). Within a call, operands
+// from memory and the clock under load, a launch takes up to a quarter longer (q | kv_a at 4096: 134).
 template <class Sh, int EPI, bool F16>
 static hipError_t gemm_launch(hipStream_t st, const GemmArgs &a, const GemmEpi &e, int tiles) {
     hipLaunchKernelGGL((k_gemm16<Sh, EPI, F16>), dim3(tiles), dim3(Sh::Threads), 0, st, a, e);
@@ -520,7 +524,9 @@ static hipError_t gemm(hipStream_t st, const uint16_t *Ah, const uint16_t *Al, c
         if (N1 == 0 && tiles <= 256) return gemm_launch<GemmCfg<64, 32, 64, 4, 2, LO>, EPI, F16>(st, a, e, tiles);
     }
     switch (gemm_pick(EPI, M, N0, N1, &tiles)) {
-    case kTile64x64: return gemm_launch<GemmCfg<64, 64, 64, 4, 2, LO>, EPI, F16>(st, a, e, tiles);
+    case kTile64x64:
+        if constexpr (EPI == kEpiQ) return hipErrorInvalidValue;  // gemm_q_small's
+        else return gemm_launch<GemmCfg<64, 64, 64, 4, 2, LO>, EPI, F16>(st, a, e, tiles);
     case kTile128x64: return gemm_launch<GemmCfg<128, 64, 64, 4, 1, LO>, EPI, F16>(st, a, e, tiles);
     case kTile128x128: return gemm_launch<GemmCfg<128, 128, 64, 8, 1, LO>, EPI, F16>(st, a, e, tiles);
     case kTile192x128: return gemm_launch<GemmCfg<192, 128, 64, 8, 1, LO>, EPI, F16>(st, a, e, tiles);
@@ -777,6 +783,7 @@ __global__ __launch_bounds__(256) void k_kva_pack(KvaPackArgs a) {
 //   11.0 / 36.5 / 139 / 1700  one loop for both, K fragments read two groups ahead (two copies of
 //                             the loop left the compiler too few registers for that)
 //   10.3 / 36.0 / 139 / 1687  V fragments read before the weights, one copy of the merge
+//    6.2 / 24.2 / 139 / 1687  U = 1 up to kFlashSmall blocks of 128 queries
 constexpr int kFK = 64;
 constexpr int kFKB = kFK * 192 * 2;  // K tile (hi or lo): 64 rows x 384 B
 constexpr int kFVB = 128 * kFK * 2;  // V^T tile: 128 rows x 128 B
